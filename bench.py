@@ -25,7 +25,7 @@ PEAK = {"fp64_mfma_tflops": 78.6, "fp32_mfma_tflops": 157.3, "hbm_gbs": 8000.0}
 
 # kernel-timing family -> kernel symbol (as rocprofv3 names it), {T} = double/float
 FAMILY_KERNEL = {
-    "qp3s": "spq::k_qp3<{T}>",
+    "qp3s": "spq::k_qp3<{T}>", "rrqr_init": "spq::k_rrqr_init<{T}>", "rrqr_upd": "spq::k_rrqr_update<{T}>",
     "panel": "spq::k_panel_r<{T}>", "gemm": "spq::k_gemm<{T}>", "larft": "spq::k_larft<{T}>",
     "trsm": "spq::k_trsm_block<{T}>", "copy": "spq::k_copy", "init": "spq::k_init_blocks",
     "apply": "solve program (hipGraph of k_refl/k_bwd/k_move)",
@@ -41,10 +41,13 @@ MATRIX_DESC = {
 
 def family_kernel(fam):
     """Kernel symbol (as rocprofv3 prints it) of a timing family; the register
-    RRQR families are qp3r<threads>_<rows per lane>."""
+    RRQR families are qp3r<threads>_<rows per lane>, the blocked form's panels
+    rrqrp<waves>_<rows per lane>."""
     if fam.startswith("qp3r") and "_" in fam:
         nt, rc = fam[4:].split("_")
         return "spq::k_qp3r<{T}, " + nt + ", " + rc + ">"
+    if fam.startswith("rrqrp"):
+        return "spq::k_rrqr_panel<{T}, " + fam[5:].replace("_", ", ") + ">"
     if fam.startswith("gemm"):
         return FAMILY_KERNEL["gemm"]
     return FAMILY_KERNEL.get(fam, fam)

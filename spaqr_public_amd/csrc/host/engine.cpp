@@ -752,12 +752,19 @@ class Engine final : public EngineBase {
     T* Ct;
     int k, N;
     int rank = 0, nwg = 1;
-    T* V = nullptr;
+    T* V = nullptr;  // reflectors: k x rank by columns (ld ldv), or by rows
+    int ldv = 0;
+    bool byrows = false;
     T* tau = nullptr;
   };
   // rc_force > 0: rows per lane of the register form (the autotuner's trial
   // runs); else the tuned or closed-form choice
   void rrqr_batch(std::vector<RrqrJob>& jobs, int rc_force = 0);
+  void rrqr_blocked(std::vector<RrqrJob>& jobs);
+  // the first `rank` reflectors of a job as columns (ld k)
+  static CopyDesc rrqr_v_copy(const RrqrJob& j, T* V, int rank) {
+    return j.byrows ? CopyDesc{j.V, V, j.ldv, j.k, rank, j.k, 1, 0} : CopyDesc{j.V, V, j.ldv, j.k, j.k, rank, 0, 0};
+  }
   bool trial_ = false;  // inside an autotuner trial: no ledger, no logging
   void sparsify_extra_level(const std::vector<int>& cs);
   void build_solve_program();
@@ -1454,6 +1461,88 @@ void Engine<T>::scale_level(const std::vector<int>& cs) {
   for (auto& f : run) f();
 }
 
+// The blocked form of rrqr_batch: rounds of a panel and an update launch over
+// the whole batch until every problem is done.  The rounds a batch needs are
+// not known: what its largest problem typically takes is queued, then two at a
+// time until the done flags, read back with the ranks, say so (a queued round
+// of finished problems costs about 10 us, a read-back 20; a round finds at
+// least one pivot, so min(k, N) rounds always suffice).
+template <typename T>
+void Engine<T>::rrqr_blocked(std::vector<RrqrJob>& jobs) {
+  const size_t nj = jobs.size();
+  int kmax = 0;
+  for (auto& j : jobs) kmax = std::max(kmax, j.k);
+  const int form = rrqr_form(kmax, (int)nj), utile = rrqr_update_cols();
+  RrqrState* st = (RrqrState*)scratch_.alloc(sizeof(RrqrState) * nj);
+  std::vector<RrqrDesc<T>> qd(nj);
+  std::vector<int> icnt(nj), ucnt(nj), ist, ust;
+  double by = 0;
+  for (size_t q = 0; q < nj; ++q) {
+    RrqrJob& jb = jobs[q];
+    const size_t N = std::max(jb.N, 1), k = jb.k;
+    jb.nwg = 1;
+    // a round writes its 32 columns whole: V is by rows, padded
+    jb.ldv = iceil(jb.k + kRrqrPivots - 1, 16) * 16;
+    jb.byrows = true;
+    jb.V = alloc_scr((k + 15) * jb.ldv);
+    jb.tau = alloc_scr(k);
+    RrqrDesc<T>& d = qd[q];
+    d.Ct = jb.Ct; d.V = jb.V; d.tau = jb.tau;
+    d.Tm = (double*)scratch_.alloc(sizeof(double) * kRrqrPivots * kRrqrPivots);
+    d.vn = (double*)scratch_.alloc(sizeof(double) * N);
+    d.ipos = (int*)scratch_.alloc(sizeof(int) * N);
+    d.perm = (int*)scratch_.alloc(sizeof(int) * N);
+    d.st = st + q;
+    d.ldc = (int)N; d.k = jb.k; d.N = jb.N; d.ldv = jb.ldv; d.tol = tol_;
+    icnt[q] = rrqr_init_tiles(jb.N);
+    ucnt[q] = iceil(std::max(jb.N, 1), utile);
+    by += (double)sizeof(T) * jb.k * jb.N;
+    const int kk = std::min(jb.k, jb.N);
+    flops_ += 4.0 * jb.k * jb.N * kk - 2.0 * (jb.k + jb.N) * kk * kk + 4.0 / 3.0 * kk * kk * kk;
+  }
+  const int nit = prefix_tiles(icnt, ist), nut = prefix_tiles(ucnt, ust);
+  const RrqrDesc<T>* dd = stager_.push(qd);
+  const int* dis = stager_.push(ist);
+  const int* dus = stager_.push(ust);
+  const int nd = (int)nj;
+  timed("rrqr_init", 0.0, by, [&] { launch_rrqr_init<T>(stream_, dd, dis, nd, nit); });
+  static const std::vector<std::string> names = [] {
+    std::vector<std::string> v(1);
+    for (int f = 1; rrqr_form_waves(f) > 0; ++f)
+      v.push_back("rrqrp" + std::to_string(rrqr_form_waves(f)) + "_" + std::to_string(rrqr_form_rows(f)));
+    return v;
+  }();
+  // a rank of 0.7 k at 24 pivots a round, and one round more
+  int rounds = 1 + iceil(7 * kmax, 240);
+  // read back into the pinned rank buffer (its last int is the error flag's)
+  std::vector<RrqrState> big;
+  RrqrState* hs = reinterpret_cast<RrqrState*>(rank_host_);
+  if (sizeof(RrqrState) * nj > sizeof(int) * 65534) {
+    big.resize(nj);
+    hs = big.data();
+  }
+  for (int queued = 0;;) {
+    for (int r = 0; r < rounds; ++r) {
+      timed(names[form].c_str(), 0.0, 0.0, [&] { launch_rrqr_panel<T>(stream_, dd, nd, form); });
+      timed("rrqr_upd", 0.0, 2 * by, [&] { launch_rrqr_update<T>(stream_, dd, dus, nd, nut, kmax); });
+    }
+    SPQ_HIP(hipMemcpyAsync(hs, st, sizeof(RrqrState) * nj, hipMemcpyDeviceToHost, stream_));
+    sync();
+    bool all = true;
+    for (size_t q = 0; q < nj && all; ++q) all = hs[q].done != 0;
+    if (all) break;
+    queued += rounds;
+    if (queued > kmax) throw Error(kErrNumeric, "rrqr: a round made no progress");
+    rounds = 2;
+  }
+  for (size_t q = 0; q < nj; ++q) jobs[q].rank = hs[q].next;
+  if (kprof_)
+    for (size_t q = 0; q < nj; ++q) {
+      const double k = jobs[q].k, N = jobs[q].N, r = jobs[q].rank;
+      kev_["rrqr_upd"].flops += 4 * k * N * r - 2 * (k + N) * r * r + 4.0 / 3.0 * r * r * r;
+    }
+}
+
 // Truncated column-pivoted QR (the geqp3 + choose_rank of util.cpp:466-477,
 // 795-816) of a batch of independent problems whose transposed inputs Ct
 // (N x k, ld N) are already gathered.  Per problem: the register form when its
@@ -1464,6 +1553,20 @@ void Engine<T>::scale_level(const std::vector<int>& cs) {
 template <typename T>
 void Engine<T>::rrqr_batch(std::vector<RrqrJob>& jobs, int rc_force) {
   if (jobs.empty()) return;
+  // the blocked form takes every problem whose rows one panel workgroup
+  // holds; the column-by-column forms below keep the larger ones, the
+  // autotuner's trials and the forms asked for by name
+  if (rc_force == 0 && qp3_rc_ == 0 && qp3_reg_ && tol_ < 1.0 && !global_tuner().tuning()) {
+    std::vector<RrqrJob> blk, rest;
+    for (auto& j : jobs) (rrqr_form(j.k, 1) ? blk : rest).push_back(j);
+    if (!blk.empty()) {
+      rrqr_blocked(blk);
+      if (!rest.empty()) rrqr_batch(rest);
+      size_t b = 0, r = 0;
+      for (auto& j : jobs) j = rrqr_form(j.k, 1) ? blk[b++] : rest[r++];
+      return;
+    }
+  }
   int kmax = 0, nmax = 0;
   for (auto& j : jobs) { kmax = std::max(kmax, j.k); nmax = std::max(nmax, j.N); }
   // rows per lane of the register form, one for the whole batch (one launch
@@ -1548,6 +1651,8 @@ void Engine<T>::rrqr_batch(std::vector<RrqrJob>& jobs, int rc_force) {
     if (G == 0) nwg = lds_ok ? std::max(1, std::min(qp3_max_wg_, jb.N / 256)) : 1;
     jb.nwg = nwg;
     jb.V = alloc_scr((size_t)jb.k * jb.k);
+    jb.ldv = jb.k;
+    jb.byrows = false;
     jb.tau = alloc_scr(jb.k);
     Qp3Desc<T> d{};
     d.Ct = jb.Ct; d.V = jb.V; d.tau = jb.tau;
@@ -1777,7 +1882,7 @@ void Engine<T>::sparsify_level(const std::vector<int>& cs) {
       T* W = nullptr;  // order 1.5: top k rows of the in-edge blocks, k x spm (ld k)
       T* Rest = nullptr;  // least squares: rows [k, rows) of the in-edge blocks, rest x spm
       int rest = 0;
-      T *Ct, *V, *tau;
+      T *Ct, *tau;
     };
     std::vector<CopyDesc> gather;
     std::vector<RrqrJob> rj;
@@ -1861,7 +1966,6 @@ void Engine<T>::sparsify_level(const std::vector<int>& cs) {
     std::vector<int> ranks(jobs.size(), 0);
     for (size_t q = 0; q < jobs.size(); ++q) {
       ranks[q] = rj[q].rank;
-      jobs[q].V = rj[q].V;
       jobs[q].tau = rj[q].tau;
     }
     if (verbose_ > 1) {
@@ -1897,7 +2001,7 @@ void Engine<T>::sparsify_level(const std::vector<int>& cs) {
       T* Tb = alloc_perm((size_t)nb_ * iceil(std::max(rank, 1), nb_) * nb_);
       factor_bytes_ += sizeof(T) * ((double)k * rank + (double)nb_ * iceil(std::max(rank, 1), nb_) * nb_);
       if (rank > 0) {
-        scatter.push_back(CopyDesc{jb.V, V, k, k, k, rank, 0, 0});
+        scatter.push_back(rrqr_v_copy(rj[q], V, rank));
         scatter.push_back(CopyDesc{jb.tau, tau, rank, rank, rank, 1, 0, 0});
         lf.push_back(LarftDesc<T>{V, tau, Tb, k, k, rank, 0});
         lcnt.push_back(iceil(rank, nb_));
@@ -2167,7 +2271,7 @@ void Engine<T>::sparsify0_level(const std::vector<int>& cs) {
       factor_bytes_ += sizeof(T) * ((double)k * rank + (double)nb_ * iceil(std::max(rank, 1), nb_) * nb_);
       const Block self = ed_[jb.es].a;  // a copy: add_edge below may move ed_
       if (rank > 0) {
-        vcopy.push_back(CopyDesc{rj[q].V, V, k, k, k, rank, 0, 0});
+        vcopy.push_back(rrqr_v_copy(rj[q], V, rank));
         vcopy.push_back(CopyDesc{rj[q].tau, tau, rank, rank, rank, 1, 0, 0});
         lf.push_back(LarftDesc<T>{V, tau, Tb, k, k, rank, 0});
         lcnt.push_back(iceil(rank, nb_));

@@ -166,6 +166,33 @@ struct Qp3Desc {
   int rc = 0;         // register form: rows per lane (the kernel's RC)
 };
 
+// Blocked form of the truncated pivoted QR (rrqr.hip), same input and output
+// as Qp3Desc.  A problem advances in rounds of one panel launch and one
+// update launch; everything a round hands to the next lives in memory.
+constexpr int kRrqrPivots = 32;  // most pivots of a round
+constexpr int kRrqrCols = 64;    // candidate columns of a round (one per lane)
+struct RrqrState {
+  int i0;    // first pivot step of the last round
+  int b;     // its pivots (0: nothing to update)
+  int next;  // pivot steps done; the rank, once done
+  int done;
+  double r00;
+};
+template <typename T>
+struct RrqrDesc {
+  T* Ct;         // N x k (ld ldc): row r of C is column r
+  T* V;          // reflectors by rows: V[r * ldv + i] is row r >= i of reflector i;
+                 // k + 15 rows, ldv >= k + 31 (a round writes its 32 columns and 16-row tiles whole)
+  T* tau;        // k
+  double* Tm;    // the round's 32 x 32 T factor, by rows
+  double* vn;    // N: squared norms below the finished rows; -1 NaN, -2 pivoted
+  int* ipos;     // N: position of each column (LAPACK's swaps)
+  int* perm;     // N: column at each position
+  RrqrState* st;
+  int ldc, k, N, ldv;
+  double tol;
+};
+
 // Solve-side vector segment (cluster x buffer offset, length).
 struct Seg {
   int64_t off;

@@ -37,30 +37,6 @@ __device__ __forceinline__ T structured(const T* __restrict__ M, int ld, int r, 
 constexpr int TK = 16;
 constexpr int kTileMaxM = 128, kTileMaxN = 128;
 
-
-// Operands: lane l holds A(l % 16, l / 16) of the 16 x 4 A block and
-// B(l / 16, l % 16) of the 4 x 16 B block.  Accumulator c of lane l holds
-// D(row(l / 16, c), l % 16): row = l / 16 + 4 c for FP64, 4 (l / 16) + c for
-// FP32 (the two instructions interleave their result rows differently).
-template <typename T>
-struct Mfma;
-template <>
-struct Mfma<double> {
-  typedef double v4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ v4 mac(double a, double b, v4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int k4, int c) { return k4 + 4 * c; }
-};
-template <>
-struct Mfma<float> {
-  typedef float v4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ v4 mac(float a, float b, v4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ int row(int k4, int c) { return 4 * k4 + c; }
-};
-
 // One TM x TN tile (TM = 32 WM, TN = 32 WN, WM * WN = 4 waves).
 template <typename T, int WM, int WN>
 __device__ __forceinline__ void gemm_tile(const GemmDesc<T>& D, int local, T (*As)[kTileMaxM + 2],

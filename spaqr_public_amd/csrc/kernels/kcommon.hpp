@@ -136,6 +136,76 @@ __device__ __forceinline__ T wave_reduce_scatter32_nolds(T (&a)[32]) {
   return a[0] + lane_xor<1>(a[0]);
 }
 
+// Global-address-space view of a pointer read from a descriptor (global
+// loads instead of flat ones, which would also count against the LDS wait
+// counter).
+template <typename T>
+using gptr = const __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ __forceinline__ gptr<T> to_global(const T* p) {
+  return (gptr<T>)p;
+}
+template <typename T>
+using gmut = __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ __forceinline__ gmut<T> to_global_mut(T* p) {
+  return (gmut<T>)p;
+}
+// base[byte_off / sizeof(T)] for a uniform base and a 32-bit byte offset
+// (one scalar base register pair plus one vector register per load)
+template <typename T>
+__device__ __forceinline__ T load_at(const T* base, unsigned byte_off) {
+  return *(gptr<T>)((const __attribute__((address_space(1))) char*)to_global(base) + byte_off);
+}
+template <typename T>
+__device__ __forceinline__ void store_at(T* base, unsigned byte_off, T v) {
+  *(gmut<T>)((__attribute__((address_space(1))) char*)to_global_mut(base) + byte_off) = v;
+}
+
+// Value of v in lane l (l uniform) for every lane of the wave.
+__device__ __forceinline__ double lane_bcast(double v, int l) {
+  const unsigned long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ float lane_bcast(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// Orders one wavefront's LDS and memory accesses around an exchange among its
+// own lanes (no other wave takes part).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// ---------------------------------------------------------------------------
+// Matrix cores, 16 x 16 x 4.
+// Operands: lane l holds A(l % 16, l / 16) of the 16 x 4 A block and
+// B(l / 16, l % 16) of the 4 x 16 B block.  Accumulator c of lane l holds
+// D(row(l / 16, c), l % 16): row = l / 16 + 4 c for FP64, 4 (l / 16) + c for
+// FP32 (the two instructions interleave their result rows differently).
+template <typename T>
+struct Mfma;
+template <>
+struct Mfma<double> {
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 mac(double a, double b, v4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int k4, int c) { return k4 + 4 * c; }
+};
+template <>
+struct Mfma<float> {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 mac(float a, float b, v4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int k4, int c) { return 4 * k4 + c; }
+};
+
 // Block-wide sum of one value; `red` must hold >= blockDim.x/64 entries.
 template <typename T>
 __device__ __forceinline__ T block_sum_x(T v, T* red) {

@@ -61,6 +61,23 @@ int qp3_capacity(int kmax);
 template <typename T>
 int launch_qp3(hipStream_t s, const Qp3Desc<T>* d, const int* wstart, int nd, int nwg_total, int kmax, int coop);
 
+// rrqr.hip
+// Blocked form of the truncated pivoted QR: the panel form for nd problems of
+// at most k rows (0: k is beyond it), the tiles of the init grid for N columns, the columns per
+// workgroup of the update, and the launches of a round.  kmax: largest k of
+// the launch.
+int rrqr_form(int k, int nd);
+int rrqr_form_waves(int form);
+int rrqr_form_rows(int form);
+int rrqr_init_tiles(int N);
+int rrqr_update_cols();
+template <typename T>
+void launch_rrqr_init(hipStream_t s, const RrqrDesc<T>* d, const int* tstart, int nd, int ntiles);
+template <typename T>
+void launch_rrqr_panel(hipStream_t s, const RrqrDesc<T>* d, int nd, int form);
+template <typename T>
+void launch_rrqr_update(hipStream_t s, const RrqrDesc<T>* d, const int* tstart, int nd, int ntiles, int kmax);
+
 // solve.hip
 // register form of the reflector apply: nrw row waves per workgroup (1, 2
 // or 7), so <= 64 nrw rows per workgroup; reflr_rows() = 448 (nrw = 7) and

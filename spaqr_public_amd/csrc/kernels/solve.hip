@@ -185,21 +185,6 @@ size_t reflr_lds(int nseg_max) {
   return (((size_t)nseg_max + 1) * sizeof(int) + 7) / 8 * 8 + (size_t)std::max(nseg_max, 1) * sizeof(int64_t);
 }
 
-// Global-address-space view of a pointer read from a descriptor (global
-// loads instead of flat ones, which would also count against the LDS wait
-// counter).
-template <typename T>
-using gptr = const __attribute__((address_space(1))) T*;
-template <typename T>
-__device__ __forceinline__ gptr<T> to_global(const T* p) {
-  return (gptr<T>)p;
-}
-template <typename T>
-using gmut = __attribute__((address_space(1))) T*;
-template <typename T>
-__device__ __forceinline__ gmut<T> to_global_mut(T* p) {
-  return (gmut<T>)p;
-}
 // The relaxed-barrier protocol of kcommon.hpp (agent-scope stores and loads
 // of the exchanged values, relaxed counter) on global pointers: flat
 // accesses would make every later LDS wait also wait for vector memory.
@@ -218,32 +203,6 @@ __device__ __forceinline__ void barrier_arrive_wait_g(unsigned int* ctr, unsigne
     }
   }
 }
-// base[byte_off / sizeof(T)] for a uniform base and a 32-bit byte offset
-// (one scalar base register pair plus one vector register per load)
-template <typename T>
-__device__ __forceinline__ T load_at(const T* base, unsigned byte_off) {
-  return *(gptr<T>)((const __attribute__((address_space(1))) char*)to_global(base) + byte_off);
-}
-
-// Value of v in lane l (l uniform) for every lane of the wave.
-__device__ __forceinline__ double lane_bcast(double v, int l) {
-  const unsigned long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-__device__ __forceinline__ float lane_bcast(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
-// Orders one wavefront's LDS and memory accesses around an exchange among its
-// own lanes (no other wave takes part).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // Descriptor owning workgroup `t` (start[] exclusive prefix sums, strictly
 // increasing): every lane of the wave tests 64 entries per load round, so
 // a launch of up to 256 descriptors costs one round of loads.

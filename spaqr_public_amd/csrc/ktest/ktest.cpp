@@ -234,6 +234,58 @@ int ktest_qp3(int k, int N, double* Ct, double* V, double* tau, double tol, int 
   return rank;
 }
 
+// The same by the blocked form (rounds of a panel and an update launch) in T
+// storage.  Returns the rank (rounds in *rounds), or -1.
+}  // extern "C"
+namespace {
+template <typename X>
+int rrqr_one(int k, int N, X* Ct, X* V, X* tau, double tol, int nd, int* perm, int* rounds) {
+  const int form = rrqr_form(k, nd);  // the form a launch of nd problems takes
+  if (!form || k < 1 || N < 0) { g_err = "k beyond the blocked form"; return -1; }
+  const size_t n1 = std::max(N, 1);
+  const int ldv = k + kRrqrPivots - 1, kr = k + 15;  // V by rows, padded
+  X *dC = dup(Ct, n1 * k), *dV = dup<X>(nullptr, (size_t)kr * ldv), *dt = dup<X>(nullptr, k);
+  double* tm = dup<double>(nullptr, kRrqrPivots * kRrqrPivots);
+  double* vn = dup<double>(nullptr, n1);
+  int *ip = dup<int>(nullptr, n1), *pm = dup<int>(nullptr, n1);
+  RrqrState* st = dup<RrqrState>(nullptr, 1);
+  RrqrDesc<X> d{dC, dV, dt, tm, vn, ip, pm, st, (int)n1, k, N, ldv, tol};
+  RrqrDesc<X>* dd = dup(&d, 1);
+  int zero = 0;
+  int* ws = dup(&zero, 1);
+  launch_rrqr_init<X>(0, dd, ws, 1, rrqr_init_tiles(N));
+  RrqrState h{};
+  int r = 0;
+  for (; r <= k; ++r) {
+    launch_rrqr_panel<X>(0, dd, 1, form);
+    launch_rrqr_update<X>(0, dd, ws, 1, ((int)n1 + rrqr_update_cols() - 1) / rrqr_update_cols(), k);
+    KT(hipDeviceSynchronize());
+    back(&h, st, 1);
+    if (h.done) break;
+  }
+  std::vector<X> hv((size_t)kr * ldv);
+  back(Ct, dC, n1 * k);
+  back(hv.data(), dV, hv.size());
+  for (int c = 0; c < k; ++c)
+    for (int i = 0; i < k; ++i) V[i + (size_t)c * k] = hv[(size_t)i * ldv + c];
+  back(tau, dt, k);
+  back(perm, pm, N);
+  *rounds = r + 1;
+  for (void* q : {(void*)dC, (void*)dV, (void*)dt, (void*)tm, (void*)vn, (void*)ip, (void*)pm, (void*)st,
+                  (void*)dd, (void*)ws})
+    (void)hipFree(q);
+  if (!h.done) { g_err = "no progress"; return -1; }
+  return h.next;
+}
+}  // namespace
+extern "C" {
+int ktest_rrqr(int k, int N, double* Ct, double* V, double* tau, double tol, int nd, int* perm, int* rounds) {
+  return rrqr_one<double>(k, N, Ct, V, tau, tol, nd, perm, rounds);
+}
+int ktest_rrqr_f32(int k, int N, float* Ct, float* V, float* tau, double tol, int nd, int* perm, int* rounds) {
+  return rrqr_one<float>(k, N, Ct, V, tau, tol, nd, perm, rounds);
+}
+
 // Timing of one truncated QP3 problem (either form): `reps` launches on a
 // fresh copy of C each, the average kernel time in *ms.  Returns the rank.
 int ktest_qp3_bench(int k, int N, const double* Ct, double tol, int form, int nwg, int reps, double* ms) {
