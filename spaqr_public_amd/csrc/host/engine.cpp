@@ -547,14 +547,13 @@ class Engine final : public EngineBase {
   void blocked_qr_plan(std::vector<QrJobT<U>>& jobs, Run& run) {
     int kmax = 0;
     for (auto& j : jobs) kmax = std::max(kmax, std::min(j.m, j.k));
-    // panel steps run in the register form: rows [jb, m) over nwg
-    // workgroups; barrier counters of all multi-workgroup steps come from one
-    // pool cleared by one launch
-    const int rpw = panel_rows_per_wg();
+    // panel steps: rows [jb, m) in one workgroup, or over nwg of them; the
+    // exchange slots of all multi-workgroup steps come from one pool cleared by
+    // one launch
     size_t words = 0;
     for (int jb = 0; jb < kmax; jb += nb_)
       for (auto& j : jobs)
-        if (jb < std::min(j.m, j.k) && iceil(j.m - jb, rpw) > 1) words += barrier_words(iceil(j.m - jb, rpw));
+        if (jb < std::min(j.m, j.k)) words += sizeof(U) / 4 * panel_slots(panel_wgs<U>(j.m - jb));
     unsigned int* pool = words ? (unsigned int*)scratch_.alloc(sizeof(unsigned int) * words) : nullptr;
     if (words) run.push_back([this, pool, words] { launch_zero(stream_, 4, pool, words); });
     size_t pool_used = 0;
@@ -569,12 +568,11 @@ class Engine final : public EngineBase {
         if (jb >= std::min(j.m, j.k)) continue;
         PanelDesc<U> d{};
         d.P = j.P; d.tau = j.tau; d.Tb = j.Tb; d.ld = j.ld; d.m = j.m; d.k = j.k;
-        d.nwg = iceil(j.m - jb, rpw);
+        d.nwg = panel_wgs<U>(j.m - jb);
         d.err = qp3_err_;
         if (d.nwg > 1) {
-          d.part = (U*)ws_.alloc(sizeof(U) * 2 * (size_t)d.nwg * 2 * nb_);
-          d.sync = pool + pool_used;
-          pool_used += barrier_words(d.nwg);
+          d.part = (U*)(pool + pool_used);
+          pool_used += sizeof(U) / 4 * panel_slots(d.nwg);
           multi.push_back(d);
         } else {
           single.push_back(d);
@@ -607,9 +605,11 @@ class Engine final : public EngineBase {
         const int* dst = stager_.push(st);
         const double f = li == 0 ? pfl : 0.0, by = li == 0 ? pby : 0.0;
         const int nd = (int)L.first.size(), coop = L.second;
-        run.push_back([this, f, by, dpd, dst, nd, nt, jb, coop] {
+        int rows = 0;
+        for (auto& d : L.first) rows = std::max(rows, d.m - jb);
+        run.push_back([this, f, by, dpd, dst, nd, nt, jb, rows, coop] {
           int rc = 0;
-          timed("panel", f, by, [&] { rc = launch_panel_r<U>(stream_, dpd, dst, nd, nt, jb, coop); });
+          timed("panel", f, by, [&] { rc = launch_panel_r<U>(stream_, dpd, dst, nd, nt, jb, rows, coop); });
           if (rc != 0) throw Error(kErrHip, std::string("panel launch failed: ") + hipGetErrorString((hipError_t)rc));
         });
       }

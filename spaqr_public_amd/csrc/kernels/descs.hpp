@@ -103,9 +103,9 @@ void larfb_step_descs(const U* Vb, int ldv, const U* Tb, int ldt, int rows, int 
 
 // Householder panel block: factor columns [jb, jb+w) of P (m x k, ld), writing
 // reflectors below the diagonal, R on/above it, tau[j] and the nb x nb block
-// T factor of this block into Tb + jb*nb (ld nb).  The register form splits
-// rows [jb, m) over nwg workgroups (part: 2 * nwg * 64 partial sums and the
-// published pivot row; sync: barrier_words(nwg) counters, zero on entry).
+// T factor of this block into Tb + jb*nb (ld nb).  Rows [jb, m) beyond one
+// workgroup's are split over nwg = panel_wgs workgroups (part: panel_slots(nwg)
+// exchange slots, zero on entry).
 template <typename T>
 struct PanelDesc {
   T* P;
@@ -114,7 +114,6 @@ struct PanelDesc {
   int ld, m, k;
   int nwg;
   T* part;
-  unsigned int* sync;
   int* err;
 };
 

@@ -181,6 +181,25 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// sqrt and reciprocal of a normal number well inside the range, by Newton
+// steps on the hardware's estimates
+__device__ __forceinline__ double sqrt_nr(double a) {
+  const double y = __builtin_amdgcn_rsq(a);
+  double g = a * y, h = 0.5 * y;
+  double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  r = fma(-h, g, 0.5);
+  h = fma(h, r, h);
+  g = fma(g, r, g);
+  return fma(fma(-g, g, a), h, g);
+}
+__device__ __forceinline__ double rcp_nr(double a) {
+  double y = __builtin_amdgcn_rcp(a);
+  y = fma(fma(-a, y, 1.0), y, y);
+  y = fma(fma(-a, y, 1.0), y, y);
+  return fma(fma(-a, y, 1.0), y, y);
+}
 // ---------------------------------------------------------------------------
 // Matrix cores, 16 x 16 x 4.
 // Operands: lane l holds A(l % 16, l / 16) of the 16 x 4 A block and

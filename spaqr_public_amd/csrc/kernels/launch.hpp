@@ -26,13 +26,18 @@ template <typename T>
 void launch_gemm(hipStream_t s, const GemmDesc<T>* d, const int* tstart, int nd, int ntiles);
 
 // panel.hip
-// Register form of the panel step: rows per workgroup, resident capacity,
-// launch (multi-workgroup problems need coop = 1 or a grid within capacity).
-int panel_rows_per_wg();
+// The panel step: workgroups of a panel of `rows` rows, the exchange slots it
+// needs with more than one, resident workgroups of the form those take, launch
+// (rows: most rows of a panel in the launch; coop = 1 if one has several
+// workgroups).
+template <typename T>
+int panel_wgs(int rows);
+size_t panel_slots(int nwg);
 template <typename T>
 int panel_r_capacity();
 template <typename T>
-int launch_panel_r(hipStream_t s, const PanelDesc<T>* d, const int* wstart, int nd, int nwg_total, int jb, int coop);
+int launch_panel_r(hipStream_t s, const PanelDesc<T>* d, const int* wstart, int nd, int nwg_total, int jb, int rows,
+                   int coop);
 int panel_nb();
 int trsm_rows_per_tile();
 template <typename T>

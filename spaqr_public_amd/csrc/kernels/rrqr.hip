@@ -38,25 +38,6 @@ namespace spq {
 
 constexpr double kDead = -2.0;  // norm slot of a pivoted column
 
-// sqrt and reciprocal of a normal number well inside the range, by Newton
-// steps on the hardware's estimates
-__device__ __forceinline__ double sqrt_nr(double a) {
-  const double y = __builtin_amdgcn_rsq(a);
-  double g = a * y, h = 0.5 * y;
-  double r = fma(-h, g, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  r = fma(-h, g, 0.5);
-  h = fma(h, r, h);
-  g = fma(g, r, g);
-  return fma(fma(-g, g, a), h, g);
-}
-__device__ __forceinline__ double rcp_nr(double a) {
-  double y = __builtin_amdgcn_rcp(a);
-  y = fma(fma(-a, y, 1.0), y, y);
-  y = fma(fma(-a, y, 1.0), y, y);
-  return fma(fma(-a, y, 1.0), y, y);
-}
 __device__ __forceinline__ double wave_max(double v) {
   v = fmax(v, lane_xor<32>(v));
   v = fmax(v, lane_xor<16>(v));

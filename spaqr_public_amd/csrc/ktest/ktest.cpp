@@ -114,17 +114,15 @@ int ktest_qr(int m, int k, double* A, double* tau, double* Tb, int nc, double* C
   int* ds = dup(&zero, 1);
   int* err = dup<int>(nullptr, 1);
   for (int jb = 0; jb < kk; jb += nb) {
-    // register-form panel step over ceil((m - jb) / rows-per-workgroup) workgroups
-    const int nwg = (m - jb + panel_rows_per_wg() - 1) / panel_rows_per_wg();
+    const int nwg = panel_wgs<double>(m - jb);
     if (nwg > panel_r_capacity<double>()) { g_err = "nwg exceeds resident capacity"; return -1; }
-    double* part = dup<double>(nullptr, 2 * (size_t)nwg * 2 * nb);
-    unsigned int* sync = dup<unsigned int>(nullptr, barrier_words(nwg));
-    PanelDesc<double> pd{dA, dt, dT, m, m, k, nwg, part, sync, err};
+    double* part = dup<double>(nullptr, panel_slots(nwg));
+    PanelDesc<double> pd{dA, dt, dT, m, m, k, nwg, part, err};
     PanelDesc<double>* dpd = dup(&pd, 1);
-    const int rc = launch_panel_r<double>(0, dpd, ds, 1, nwg, jb, nwg > 1 ? 1 : 0);
+    const int rc = launch_panel_r<double>(0, dpd, ds, 1, nwg, jb, m - jb, nwg > 1 ? 1 : 0);
     if (rc != 0) { g_err = hipGetErrorString((hipError_t)rc); return -1; }
     KT(hipDeviceSynchronize());
-    for (void* q : {(void*)part, (void*)sync, (void*)dpd}) (void)hipFree(q);
+    for (void* q : {(void*)part, (void*)dpd}) (void)hipFree(q);
     const int w = (nb < kk - jb) ? nb : kk - jb, rows = m - jb;
     const double* Vb = dA + jb + (size_t)jb * m;
     const double* Tbb = dT + (size_t)jb * nb;
