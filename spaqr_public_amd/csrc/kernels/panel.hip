@@ -36,18 +36,6 @@ __device__ __forceinline__ void t_factor(const T (&Gs)[kNB][kNB], const T (&taus
   }
 }
 
-template <typename T>
-__device__ __forceinline__ void tcol_from_dots(T* Ts, int jj, T tau, const T* g) {
-  // Ts is NB x NB (ld NB) in LDS; column jj from dots g[0..jj)
-  if ((int)threadIdx.x < jj) {
-    const int r = threadIdx.x;
-    T s = 0;
-    for (int l = r; l < jj; ++l) s += Ts[r + l * kNB] * g[l];
-    Ts[r + jj * kNB] = -tau * s;
-  }
-  if ((int)threadIdx.x == jj) Ts[jj + jj * kNB] = tau;
-}
-
 // The panel step.  A wave holds 8 Q rows of the block's 32 columns in
 // registers: lane (c8, g) = (lane / 8, lane % 8) the columns 4 c8 .. 4 c8 + 3 of
 // the rows g, g + 8, ... of its 8-row groups, which are dealt to the NW waves
@@ -308,54 +296,66 @@ __global__ __launch_bounds__(NW * kWave) void k_panel_r(const PanelDesc<T>* __re
   if (wg == 0 && w == NW - 1) t_factor(Gs, taus, to_global_mut(d.Tb) + (int64_t)jb * kNB);
 }
 
-// Block T factors for an existing reflector set (QP3 output): one workgroup
-// per (descriptor, NB block).
+// Block T factors for an existing reflector set (RRQR output): one workgroup
+// per (descriptor, NB block).  G = V_b^T V_b on the matrix cores, the rows
+// dealt to the waves 16 at a time (a lane reads four consecutive rows of two
+// columns), summed in LDS; then one wave forms T from it.  Bound by latency:
+// one pass over V_b and the T recurrence; a reduction per column of T took
+// 160 us a launch at 64^3, 33^3 and 2-D alike.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_larft(const LarftDesc<T>* __restrict__ descs, const int* __restrict__ tstart,
                                                     int nd) {
+  using V4 = typename Mfma<T>::v4;
+  constexpr int NW = kThreads / kWave;
+  __shared__ __align__(16) T Gs[kNB][kNB];
+  __shared__ T part[NW][3][16][17];
+  __shared__ T taus[kNB];
   const int t = blockIdx.x;
   const int p = find_owner(tstart, nd, t);
   const LarftDesc<T> d = descs[p];
   const int jb = (t - tstart[p]) * kNB;
-  const int w = min(kNB, d.r - jb);
-  const int m = d.m, tid = threadIdx.x;
+  const int cols = min(kNB, d.r - jb), rows = d.m - jb;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave, c16 = lane & 15, k4 = lane >> 4;
   const int64_t ld = d.ldv;
-  __shared__ T red[kNB * (kThreads / kWave)];
-  __shared__ T Ts[kNB * kNB];
-  __shared__ T gsh[kNB];
-  for (int i = tid; i < kNB * kNB; i += kThreads) Ts[i] = T(0);
-  __syncthreads();
-  for (int jj = 0; jj < w; ++jj) {
-    const int j = jb + jj;
-    const T* __restrict__ vj = d.V + (int64_t)j * ld;
-    T acc[kNB];
+  const gptr<T> V = to_global(d.V) + jb + (int64_t)jb * ld;
+  if (tid < kNB) taus[tid] = tid < cols ? d.tau[jb + tid] : T(0);
+  V4 g[3];  // tiles (0, 0), (0, 1), (1, 1) of G
 #pragma unroll
-    for (int c = 0; c < kNB; ++c) acc[c] = T(0);
-    // v_c . v_j for c < jj: v_c(j) * 1 + sum_{i>j} v_c(i) v_j(i)
-    for (int i = j + 1 + tid; i < m; i += kThreads) {
-      const T vi = vj[i];
+  for (int q = 0; q < 3; ++q) g[q] = V4{T(0), T(0), T(0), T(0)};
+  for (int rb = 16 * w; rb < rows; rb += 16 * NW) {
+    T v[2][4];
 #pragma unroll
-      for (int c = 0; c < kNB; ++c)
-        if (c < jj) acc[c] += vi * d.V[i + (int64_t)(jb + c) * ld];
+    for (int h = 0; h < 2; ++h) {
+      const int c = 16 * h + c16;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int r = rb + 4 * k4 + u;
+        const bool in = (int)(r < rows) & (int)(c < cols);
+        const T x = in ? V[r + (int64_t)c * ld] : T(0);
+        v[h][u] = !in ? T(0) : (r > c ? x : (r == c ? T(1) : T(0)));
+      }
     }
-    // one reduce-scatter for all jj dots (entries c >= jj are zero), then
-    // the waves' partials
-    const int lane = tid & (kWave - 1), wv = tid / kWave;
-    const T sw = wave_reduce_scatter32_nolds(acc);
-    if ((lane & 1) == 0) red[wv * kNB + (lane >> 1)] = sw;
-    __syncthreads();
-    if (tid < kNB) {
-      T s = T(0);
 #pragma unroll
-      for (int q = 0; q < kThreads / kWave; ++q) s += red[q * kNB + tid];
-      gsh[tid] = (tid < jj) ? (d.V[j + (int64_t)(jb + tid) * ld] + s) : T(0);
+    for (int u = 0; u < 4; ++u) {
+      g[0] = Mfma<T>::mac(v[0][u], v[0][u], g[0]);
+      g[1] = Mfma<T>::mac(v[0][u], v[1][u], g[1]);
+      g[2] = Mfma<T>::mac(v[1][u], v[1][u], g[2]);
     }
-    __syncthreads();
-    tcol_from_dots(Ts, jj, d.tau[j], gsh);
-    __syncthreads();
   }
-  T* __restrict__ Tb = d.Tb + (int64_t)jb * kNB;
-  for (int i = tid; i < kNB * kNB; i += kThreads) Tb[i] = Ts[i];
+#pragma unroll
+  for (int q = 0; q < 3; ++q)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) part[w][q][Mfma<T>::row(k4, u)][c16] = g[q][u];
+  __syncthreads();
+  for (int e = tid; e < 3 * 256; e += kThreads) {
+    const int q = e / 256, r = e / 16 % 16, c = e % 16;
+    T s = part[0][q][r][c];
+#pragma unroll
+    for (int u = 1; u < NW; ++u) s += part[u][q][r][c];
+    Gs[r + (q == 2 ? 16 : 0)][c + (q > 0 ? 16 : 0)] = s;
+  }
+  __syncthreads();
+  if (w == 0) t_factor(Gs, taus, to_global_mut(d.Tb) + (int64_t)jb * kNB);
 }
 
 // B[:, jb:jb+w) <- B[:, jb:jb+w) * inv(R[jb:jb+w, jb:jb+w]) ; one row per thread.
