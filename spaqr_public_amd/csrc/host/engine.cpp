@@ -975,35 +975,36 @@ void Engine<T>::assemble(const CscMat& A) {  // tree.cpp:725-778
   for (int c : bottoms_[0])
     for (int i = cl_[c].rstart; i < cl_[c].rstart + cl_[c].rsize; ++i) rmap[i] = c;
   for (int c : bottoms_[0]) alloc_x(c, cl_[c].rsize);
-  // host-side dense blocks, uploaded in one batch
-  std::vector<T> host;
-  struct Pending { int edge; size_t off; };
-  std::vector<Pending> pend;
-  for (int self : bottoms_[0]) {
-    std::vector<int> nb;
-    const Clu& s = cl_[self];
-    for (int j = s.cstart; j < s.cstart + s.csize; ++j)
-      for (int q = App.p[j]; q < App.p[j + 1]; ++q) nb.push_back(rmap[App.i[q]]);
-    nb.push_back(self);
-    std::sort(nb.begin(), nb.end());
-    nb.erase(std::unique(nb.begin(), nb.end()), nb.end());
-    for (int n : nb) {
+  // the block structure: per cluster the row clusters its columns meet (and
+  // itself), found on the host pool; the edges then in creation order
+  const std::vector<int>& lev = bottoms_[0];
+  const int nl = (int)lev.size();
+  std::vector<std::vector<int>> nbs(nl);
+  parallel_for(nl, 64, [&](int, int b, int e) {
+    for (int i = b; i < e; ++i) {
+      const Clu& s = cl_[lev[i]];
+      std::vector<int>& nb = nbs[i];
+      for (int q = App.p[s.cstart]; q < App.p[s.cstart + s.csize]; ++q) nb.push_back(rmap[App.i[q]]);
+      nb.push_back(lev[i]);
+      std::sort(nb.begin(), nb.end());
+      nb.erase(std::unique(nb.begin(), nb.end()), nb.end());
+    }
+  });
+  std::vector<int64_t> cell(nl + 1, 0);  // first edge of each cluster
+  for (int i = 0; i < nl; ++i) cell[i + 1] = cell[i] + (int64_t)nbs[i].size();
+  std::vector<int64_t> off(cell[nl]);  // of each edge's block
+  int64_t total = 0;
+  for (int i = 0; i < nl; ++i) {
+    const int self = lev[i];
+    for (size_t q = 0; q < nbs[i].size(); ++q) {
+      const int n = nbs[i][q];
       Edge e;
       e.n1 = self; e.n2 = n;
-      e.a.rows = cl_[n].rsize; e.a.cols = s.csize; e.a.ld = std::max(1, e.a.rows);
-      const size_t off = host.size();
-      host.resize(off + (size_t)e.a.ld * e.a.cols, T(0));
-      const int r0 = cl_[n].rstart, r1 = r0 + cl_[n].rsize;
-      for (int col = 0; col < s.csize; ++col) {
-        const int j = s.cstart + col;
-        const int* beg = App.i.data() + App.p[j];
-        const int* end = App.i.data() + App.p[j + 1];
-        for (const int* it = std::lower_bound(beg, end, r0); it != end && *it < r1; ++it)
-          host[off + (size_t)(*it - r0) + (size_t)col * e.a.ld] = (T)App.x[it - App.i.data()];
-      }
+      e.a.rows = cl_[n].rsize; e.a.cols = cl_[self].csize; e.a.ld = std::max(1, e.a.rows);
+      off[cell[i] + q] = total;
+      total += (int64_t)e.a.ld * e.a.cols;
       ed_.push_back(e);
       const int id = (int)ed_.size() - 1;
-      pend.push_back({id, off});
       cl_[self].out.push_back(id);
       cl_[self].outn.push_back(n);
       if (self != n) {
@@ -1012,11 +1013,38 @@ void Engine<T>::assemble(const CscMat& A) {  // tree.cpp:725-778
       }
     }
     sort_out(self);
-    cl_[self].cnbrs = nb;
+    cl_[self].cnbrs = nbs[i];
   }
-  T* dev = alloc_perm(host.size());
-  SPQ_HIP(hipMemcpyAsync(dev, host.data(), sizeof(T) * host.size(), hipMemcpyHostToDevice, stream_));
-  for (auto& p : pend) ed_[p.edge].a.p = dev + p.off;
+  // the dense blocks are mostly zero (64^3: 1.2 GB for 1.8 M values): only the
+  // values travel, each with its place, and the device clears and fills the
+  // blocks.  A repeated (row, column) keeps its last value.
+  T* dev = alloc_perm(total);
+  const size_t nz = App.x.size();
+  std::vector<ScatterVal> vals(nz);
+  parallel_for(nl, 64, [&](int, int b, int e) {
+    for (int i = b; i < e; ++i) {
+      const Clu& s = cl_[lev[i]];
+      const std::vector<int>& nb = nbs[i];
+      for (int j = s.cstart; j < s.cstart + s.csize; ++j)
+        for (int q = App.p[j]; q < App.p[j + 1]; ++q) {
+          const int r = App.i[q], n = rmap[r];
+          const size_t at = std::lower_bound(nb.begin(), nb.end(), n) - nb.begin();
+          const bool last = q + 1 == App.p[j + 1] || App.i[q + 1] != r;
+          vals[q].at = last ? off[cell[i] + at] + (r - cl_[n].rstart) + (int64_t)(j - s.cstart) * std::max(1, cl_[n].rsize)
+                            : -1;
+          vals[q].v = App.x[q];
+        }
+    }
+  });
+  launch_zero(stream_, (int)sizeof(T), dev, total);
+  const size_t kPiece = size_t(1) << 20;  // values per upload, a quarter of the staging ring
+  for (size_t q = 0; q < nz; q += kPiece) {
+    const size_t n = std::min(kPiece, nz - q);
+    const ScatterVal* d = (const ScatterVal*)stager_.push_raw(vals.data() + q, sizeof(ScatterVal) * n);
+    stager_.flush();
+    launch_scatter_vals<T>(stream_, d, (int)n, dev);
+  }
+  for (size_t q = 0; q < off.size(); ++q) ed_[ed_.size() - off.size() + q].a.p = dev + off[q];
   sync();
   assembled_ = true;
   t_assemble_ = wall() - t0;

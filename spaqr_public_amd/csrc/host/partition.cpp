@@ -4,6 +4,8 @@
 // tree.cpp:46-163 (initPermutation, form_rmap).
 #include "partition.hpp"
 
+#include "parallel.hpp"
+
 #include <algorithm>
 #include <cmath>
 #include <limits>
@@ -36,22 +38,28 @@ CscMat csc_permute(const CscMat& A, const std::vector<int>* rperm, const std::ve
   B.m = A.m;
   B.n = A.n;
   B.p.assign(A.n + 1, 0);
-  B.i.reserve(A.nnz());
-  B.x.reserve(A.nnz());
+  B.i.resize(A.nnz());
+  B.x.resize(A.nnz());
   std::vector<int> rinv;
   if (rperm) {
     rinv.resize(A.m);
     for (int r = 0; r < A.m; ++r) rinv[(*rperm)[r]] = r;
   }
-  std::vector<std::pair<int, double>> col;
   for (int c = 0; c < A.n; ++c) {
     const int src = cperm ? (*cperm)[c] : c;
-    col.clear();
-    for (int q = A.p[src]; q < A.p[src + 1]; ++q) col.push_back({rperm ? rinv[A.i[q]] : A.i[q], A.x[q]});
-    if (rperm) std::sort(col.begin(), col.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
-    for (auto& e : col) { B.i.push_back(e.first); B.x.push_back(e.second); }
-    B.p[c + 1] = (int)B.i.size();
+    B.p[c + 1] = B.p[c] + (A.p[src + 1] - A.p[src]);
   }
+  parallel_for(A.n, 4096, [&](int, int b, int e) {
+    std::vector<std::pair<int, double>> col;
+    for (int c = b; c < e; ++c) {
+      const int src = cperm ? (*cperm)[c] : c;
+      col.clear();
+      for (int q = A.p[src]; q < A.p[src + 1]; ++q) col.push_back({rperm ? rinv[A.i[q]] : A.i[q], A.x[q]});
+      if (rperm) std::sort(col.begin(), col.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
+      int at = B.p[c];
+      for (auto& v : col) { B.i[at] = v.first; B.x[at++] = v.second; }
+    }
+  });
   return B;
 }
 

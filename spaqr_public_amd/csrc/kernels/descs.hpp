@@ -24,6 +24,12 @@ struct CopyDesc {
   int pad_;
 };
 
+// dst[at] = v (at < 0: no entry)
+struct ScatterVal {
+  int64_t at;
+  double v;
+};
+
 // Batched GEMM: C = alpha * op(A) * op(B) + beta * C, C is m x n.
 // flags: bit0 transA, bit1 transB, bits 4-5 A structure, bits 6-7 B structure
 // (structure applies to the stored matrix: 1 = unit lower trapezoidal,

@@ -12,6 +12,8 @@ namespace spq {
 void launch_copy(hipStream_t s, int elem_src, int elem_dst, const CopyDesc* d, const int* tstart, int nd, int ntiles);
 void launch_init_blocks(hipStream_t s, int elem, const CopyDesc* d, const int* tstart, int nd, int ntiles);
 void launch_zero(hipStream_t s, int elem, void* p, int64_t n);
+template <typename T>
+void launch_scatter_vals(hipStream_t s, const ScatterVal* v, int n, T* dst);
 int rowgather_tiles(int nrows, int cols);
 template <typename T>
 void launch_rownorm(hipStream_t s, const RowNormDesc<T>* d, const int* tstart, int nd, int ntiles);
