@@ -26,6 +26,15 @@ namespace {
 inline int iceil(int a, int b) { return (a + b - 1) / b; }
 }  // namespace
 
+// reflectors V (m x k, T factors Tb of its 32-column blocks) and W = V T^T
+template <typename U>
+struct WyJob {
+  const U* V;
+  const U* Tb;
+  U* W;
+  int ldv, m, k;
+};
+
 template <typename T>
 class Engine final : public EngineBase {
  public:
@@ -198,6 +207,7 @@ class Engine final : public EngineBase {
     const T* V = nullptr;
     const T* Tb = nullptr;
     int ldv = 0, m = 0, k = 0;
+    const void* W = nullptr;  // V T^T (m x k, ld m) for the dataflow apply; FP64 with V64
     std::vector<std::pair<int, int>> segs;  // (cluster, length)
     // backward data
     const T* R = nullptr;
@@ -768,7 +778,60 @@ class Engine final : public EngineBase {
   bool trial_ = false;  // inside an autotuner trial: no ledger, no logging
   void sparsify_extra_level(const std::vector<int>& cs);
   void build_solve_program();
-
+  // the dataflow form of the square apply (kernels/flow.hip)
+  struct FlowItem {
+    const Op* op;
+    int type;
+    bool trans;  // H instead of H^T
+  };
+  struct FlowStage {
+    std::vector<FlowItem> items;
+    bool chain = false;  // items sharing rows, in tape order (else independent)
+    // changes of the clusters' rows after the items: splits and merges undone
+    // (down) or made (up)
+    std::vector<const Op*> split, merge;
+    bool up = false;
+  };
+  template <typename U>
+  struct FlowProg {
+    FlowArgs<U> args{};
+    int grid = 0;
+    unsigned int* zero = nullptr;  // exchange slots and tickets, cleared before each run
+    int64_t nzero = 0;             // words
+  };
+  // places of x holding the rows of each cluster, as segments
+  struct FlowRows {
+    std::vector<std::vector<FlowSeg>> of;
+    std::vector<int> scratch;
+    int next = 0;  // places given out so far
+  };
+  bool flow_fits() const;
+  bool build_flow();
+  template <typename U>
+  void build_w(const std::vector<WyJob<U>>& jobs);
+  template <typename U>
+  bool flow_prog(const std::vector<FlowStage>& stages, FlowRows& rows, FlowProg<U>& out);
+  std::vector<int> flow_places(const FlowRows& rows, const std::vector<int>& clusters) const;
+  template <typename U>
+  void run_flow(const FlowProg<U>& p) {
+    launch_zero(stream_, 4, p.zero, p.nzero);
+    launch_flow<U>(stream_, p.args, p.grid);
+  }
+  // modes 0 and 2 (M^{-1}, M^{-T}): one program, or around the FP64 top of an
+  // FP32 tree one before and one after it
+  struct FlowMode {
+    std::vector<FlowProg<T>> run;
+    FlowProg<double> top;
+    const int* top_in = nullptr;   // the top's rows before, and in its own x after it
+    const int* top_out = nullptr;
+    int top_at = 0;                // their places afterwards
+    int xplaces = 0, x64places = 0;
+    const int* out = nullptr;      // places of the result
+  };
+  bool flow_ = false;
+  FlowMode flow_mode_[2];
+  int flow_top_n_ = 0;
+  const int *flow_rperm_ = nullptr, *flow_cperm_ = nullptr;  // rows and columns in cluster order
   // ------------------------------------------------------------ state
   int nlevels_, skip_, scale_ = 0, square_ = 0, verbose_ = 0, timing_ = 1;
   double tol_ = 0;
@@ -2745,10 +2808,452 @@ int Engine<T>::factorize() {  // tree.cpp:1309-1437
   return 0;
 }
 
+// ---------------------------------------------------------------------------
+// The square apply as a dataflow program.
+
+// Square trees without fine-cluster eliminations, in the sizes k_flow takes.
+// The others, and applies timed stage by stage, run the staged program.
+template <typename T>
+bool Engine<T>::flow_fits() const {
+  if (!square_ || !reflr_ || stage_prof_) return false;
+  auto too_long = [](int64_t ld, int64_t cols) { return ld * cols * 8 > int64_t(0xffffffffu); };  // 32-bit offsets
+  for (auto& o : ops_) {
+    if (o.kind == OpFineQR || o.kind == OpReassign) return false;
+    if (o.kind == OpSplitD && o.crows != o.ccols) return false;
+    if (o.kind != OpQR && o.kind != OpScaleD && o.kind != OpOrthoD) continue;
+    if (o.k > kFlowMaxK || o.kr > kFlowMaxK) return false;
+    if (o.m > kFlowMaxParts * kFlowMaxK || too_long(std::max(o.ldv, o.m), o.k) || too_long(o.ldr, std::max(o.kr, o.k)))
+      return false;
+  }
+  for (int c : bottoms_[0])
+    if (cl_[c].rsize_org != cl_[c].csize_org) return false;
+  return flow_capacity<T>() >= 2 * kFlowMaxParts && flow_capacity<double>() >= 2 * kFlowMaxParts;
+}
+
+// W = V T^T of the ops with reflectors.  With H = H_1 ... H_nb over blocks of
+// 32 columns, T_b their triangular factors and W_b the columns of block b,
+//   W_b = V_b T_b^T - W_{>b} (V_{>b}^T V_b T_b^T),
+// so everything but the sum over later blocks is three batched products over
+// all ops, and the sums follow from the last block to the first.
+template <typename T>
+template <typename U>
+void Engine<T>::build_w(const std::vector<WyJob<U>>& jobs) {
+  std::vector<GemmDesc<U>> w0, g, h;
+  std::vector<std::vector<GemmDesc<U>>> sums;
+  size_t gsz = 0;
+  for (auto& j : jobs)
+    for (int r = j.k - nb_; r > 0; r -= nb_) gsz += (size_t)r * nb_;
+  U* G = gsz ? (U*)scratch_.alloc(sizeof(U) * gsz) : nullptr;
+  U* H = gsz ? (U*)scratch_.alloc(sizeof(U) * gsz) : nullptr;
+  for (auto& j : jobs) {
+    for (int jb = 0; jb < j.k; jb += nb_) {
+      const int w = std::min(nb_, j.k - jb), kr = j.k - jb - nb_, r1 = jb + nb_;
+      const U* Vb = j.V + jb + (int64_t)jb * j.ldv;
+      const U* Tb = j.Tb + (int64_t)jb * nb_;
+      U* Wb = j.W + jb + (int64_t)jb * j.m;
+      w0.push_back(gd(Vb, j.ldv, Tb, nb_, Wb, j.m, j.m - jb, w, w, gemm_flags(false, true, kStructUnitLower, kStructNone),
+                      U(1), U(0)));
+      if (kr <= 0) continue;
+      const U* Vr = j.V + r1 + (int64_t)r1 * j.ldv;
+      g.push_back(gd(Vr, j.ldv, Vb + nb_, j.ldv, G, kr, kr, nb_, j.m - r1,
+                     gemm_flags(true, false, kStructUnitLower, kStructNone), U(1), U(0)));
+      h.push_back(gd((const U*)G, kr, Tb, nb_, H, kr, kr, nb_, nb_, gemm_flags(false, true, kStructNone, kStructNone),
+                     U(1), U(0)));
+      const size_t step = (size_t)(kr - 1) / nb_;  // blocks after the next
+      if (sums.size() <= step) sums.resize(step + 1);
+      sums[step].push_back(gd((const U*)(j.W + r1 + (int64_t)r1 * j.m), j.m, (const U*)H, kr, Wb + nb_, j.m, j.m - r1,
+                              nb_, kr, gemm_flags(false, false, kStructLower, kStructNone), U(-1), U(1)));
+      G += (size_t)kr * nb_;
+      H += (size_t)kr * nb_;
+    }
+  }
+  gemm_batch(w0, "wy");
+  gemm_batch(g, "wy");
+  gemm_batch(h, "wy");
+  for (auto& v : sums) gemm_batch(v, "wy");
+}
+
+// One launch of k_flow over the stages; false if an op has more input
+// segments than the kernel takes.
+template <typename T>
+template <typename U>
+bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, FlowProg<U>& p) {
+  std::vector<FlowOp<U>> parts;
+  std::vector<FlowSeg> segs;
+  std::vector<FlowBlk<U>> blks;
+  constexpr bool top = sizeof(U) > sizeof(T);  // the FP64 factors of an FP32 tree's top
+  std::vector<FlowDiag<U>> diags;
+  std::vector<int> diag_start{0};
+  size_t slots = 0;
+  std::vector<size_t> slot_at;  // by part
+  std::vector<int>& wave = R.scratch;  // of a chain: waves so far on a cluster
+  const int cap = std::min(flow_capacity<U>(), 2 * num_cus_);
+  auto add_seg = [](std::vector<FlowSeg>& v, size_t from, FlowSeg sg) {
+    if (sg.len <= 0) return;
+    if (v.size() > from && v.back().off + v.back().len == sg.off) v.back().len += sg.len;
+    else v.push_back(sg);
+  };
+  // the first n rows of a cluster
+  auto rows_of = [&](int c, int n, std::vector<FlowSeg>& v, size_t from) {
+    for (const FlowSeg& sg : R.of[c]) {
+      if (n <= 0) break;
+      add_seg(v, from, FlowSeg{sg.off, std::min(sg.len, n)});
+      n -= sg.len;
+    }
+    if (n > 0) throw Error(kErrState, "solve program: rows of a cluster are missing");
+  };
+  auto set_rows = [&](int c, int off, int n) {
+    R.of[c].clear();
+    if (n > 0) R.of[c].push_back(FlowSeg{off, n});
+  };
+  bool fits = true;
+  auto add_op = [&](FlowOp<U>& d, int nparts) {
+    fits = fits && d.nseg <= kFlowMaxSegs;
+    d.out = R.next;
+    R.next += d.m;
+    for (d.g = 0; d.g < nparts; ++d.g) {
+      parts.push_back(d);
+      slot_at.push_back(slots);
+    }
+    if (d.nwg > 1) slots += (size_t)d.nwg * d.k;
+  };
+  for (auto& st : stages) {
+    // ops side by side: all, or in a chain an average wave
+    int waves = 1;
+    if (st.chain) {
+      for (auto& it : st.items) {
+        int wv = 0;
+        for (auto& sg : it.op->segs) wv = std::max(wv, wave[sg.first] + 1);
+        for (auto& sg : it.op->segs) wave[sg.first] = wv;
+        waves = std::max(waves, wv);
+      }
+      for (auto& it : st.items)
+        for (auto& sg : it.op->segs) wave[sg.first] = 0;
+    }
+    // An op is cut where workgroups would idle: until a wave holds a tile or
+    // two of each factor, as long as the ops side by side stay within the
+    // resident workgroups
+    const int maxp = std::max(1, std::min(kFlowMaxParts, cap / std::max(1, (int)st.items.size() / waves)));
+    std::vector<std::pair<int, std::pair<int, FlowBlk<U>>>> pulls;  // target; rows of it; block
+    for (auto& it : st.items) {
+      const Op& o = *it.op;
+      FlowOp<U> d{};
+      d.type = it.type;
+      d.seg0 = (int)segs.size();
+      d.blk0 = (int)blks.size();
+      if (it.type == kFlowWY) {
+        const U* V = top ? (const U*)o.V64 : (const U*)o.V;
+        const U* W = (const U*)o.W;
+        d.m = o.m; d.k = o.k;
+        d.A = it.trans ? W : V; d.lda = it.trans ? o.m : o.ldv; d.unit_a = !it.trans;
+        d.B = it.trans ? V : W; d.ldb = it.trans ? o.ldv : o.m; d.unit_b = it.trans;
+        for (auto& sg : o.segs) rows_of(sg.first, sg.second, segs, d.seg0);
+        d.nseg = (int)segs.size() - d.seg0;
+        const int rp = o.k <= 32 ? 256 : (o.k <= 64 ? 128 : 64);
+        d.rows_per = std::min(kFlowMaxK, std::max(rp, iceil(iceil(o.m, maxp), 64) * 64));
+        d.nwg = std::max(1, iceil(o.m, d.rows_per));
+        solve_bytes_ += sizeof(U) * (2.0 * o.m * o.k - (double)o.k * o.k + 2.0 * o.m);
+        add_op(d, d.nwg);
+        int off = d.out;
+        for (auto& sg : o.segs) {
+          set_rows(sg.first, off, sg.second);
+          off += sg.second;
+        }
+        continue;
+      }
+      const bool sc = o.kind == OpScaleD;
+      d.A = top ? (const U*)o.V64 : (const U*)o.R;
+      d.lda = top ? o.ldv : o.ldr;
+      d.m = d.k = sc ? o.k : o.kr;
+      rows_of(o.c, d.k, segs, d.seg0);
+      d.nseg = (int)segs.size() - d.seg0;
+      d.nwg = 1;
+      double by = 0;
+      if (!sc && !top)
+        for (auto& q : o.r12) {
+          const int sn = q.second.second, n = q.second.first;
+          by += (double)sizeof(U) * d.k * sn;
+          if (it.type == kFlowBack) {
+            // tiles of up to 32 columns, cut where x_n's segments end
+            int j = 0;
+            for (const FlowSeg& sg : R.of[n])
+              for (int t = 0; t < sg.len && j < sn; t += 32) {
+                const int nn = std::min({32, sg.len - t, sn - j});
+                blks.push_back(FlowBlk<U>{(const U*)q.first.p + (int64_t)j * q.first.ld, q.first.ld, nn, sg.off + t, 0});
+                j += nn;
+              }
+            if (j < sn) throw Error(kErrState, "solve program: rows of a cluster are missing");
+          } else if (sn > 0) {
+            for (int r = 0; r < d.k; r += 64)
+              pulls.push_back({n, {sn, FlowBlk<U>{(const U*)q.first.p + r, q.first.ld, std::min(64, d.k - r), R.next + r, 0}}});
+          }
+        }
+      d.nblk = (int)blks.size() - d.blk0;
+      if (it.type == kFlowBack) d.nwg = std::max(1, std::min({maxp, d.nblk, d.nblk * iceil(d.k, 64) / 8}));
+      solve_bytes_ += by + sizeof(U) * (0.5 * d.k * d.k + 2.0 * d.k);
+      const int nb = iceil(d.k, nb_);
+      U* D = (U*)perm_.alloc(sizeof(U) * (size_t)nb * nb_ * (nb_ + 1));
+      diags.push_back(FlowDiag<U>{d.A, D, d.lda, d.k, it.type == kFlowSolveT, 0});
+      diag_start.push_back(diag_start.back() + nb);
+      d.B = D;
+      add_op(d, d.nwg);
+      set_rows(o.c, d.out, d.k);
+    }
+    // the products x_n - sum A^T x_c after the transposed solves, by target
+    std::stable_sort(pulls.begin(), pulls.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
+    for (size_t i = 0; i < pulls.size();) {
+      FlowOp<U> d{};
+      const int n = pulls[i].first;
+      d.type = kFlowPull;
+      d.m = pulls[i].second.first;
+      d.k = 32; d.nwg = 1;
+      d.seg0 = (int)segs.size();
+      d.blk0 = (int)blks.size();
+      rows_of(n, d.m, segs, d.seg0);
+      d.nseg = (int)segs.size() - d.seg0;
+      for (; i < pulls.size() && pulls[i].first == n; ++i) {
+        if (pulls[i].second.first != d.m) throw Error(kErrState, "solve program: blocks of different widths");
+        blks.push_back(pulls[i].second.second);
+      }
+      d.nblk = (int)blks.size() - d.blk0;
+      add_op(d, iceil(d.m, 32));
+      set_rows(n, d.out, d.m);
+    }
+    // rows handed over between clusters
+    if (st.up) {
+      for (const Op* o : st.split) {
+        // the fine cluster takes the rows past the rank
+        std::vector<FlowSeg> keep, fine;
+        int n = o->rank;
+        for (const FlowSeg& sg : R.of[o->c]) {
+          const int h = std::max(0, std::min(sg.len, n));
+          add_seg(keep, 0, FlowSeg{sg.off, h});
+          add_seg(fine, 0, FlowSeg{sg.off + h, sg.len - h});
+          n -= h;
+        }
+        R.of[o->c] = std::move(keep);
+        R.of[o->f] = std::move(fine);
+      }
+      for (const Op* o : st.merge) {
+        std::vector<FlowSeg> v;
+        for (int ch : cl_[o->c].children) rows_of(ch, cl_[ch].rsize, v, 0);
+        R.of[o->c] = std::move(v);
+      }
+    } else {
+      for (const Op* o : st.merge) {
+        size_t q = 0;
+        int used = 0;
+        const auto& par = R.of[o->c];
+        for (int ch : cl_[o->c].children) {
+          std::vector<FlowSeg> v;
+          for (int n = cl_[ch].rsize; n > 0;) {
+            if (q >= par.size()) throw Error(kErrState, "solve program: rows of a cluster are missing");
+            const int h = std::min(n, par[q].len - used);
+            add_seg(v, 0, FlowSeg{par[q].off + used, h});
+            n -= h;
+            used += h;
+            if (used == par[q].len) { ++q; used = 0; }
+          }
+          R.of[ch] = std::move(v);
+        }
+      }
+      for (const Op* o : st.split)
+        for (const FlowSeg& sg : R.of[o->f]) add_seg(R.of[o->c], 0, sg);
+    }
+  }
+  if (!fits) return false;
+  const size_t slot_words = slots * sizeof(U) / 4;
+  p.nzero = (int64_t)(slot_words + 64);
+  p.zero = (unsigned int*)perm_.alloc(4 * (size_t)p.nzero);
+  for (size_t i = 0; i < parts.size(); ++i)
+    if (parts[i].nwg > 1) parts[i].slots = (U*)p.zero + slot_at[i];
+  p.grid = cap;
+  p.args.nparts = (int)parts.size();
+  const FlowDiag<U>* dd = stager_.push(diags);
+  const int* ds = stager_.push(diag_start);
+  timed("wy", 0.0, 0.0, [&] { launch_flow_diag<U>(stream_, dd, ds, (int)diags.size(), diag_start.back()); });
+  p.args.parts = stager_.upload(perm_, parts);
+  p.args.segs = stager_.upload(perm_, segs);
+  p.args.blks = stager_.upload(perm_, blks);
+  p.args.ctl = p.zero + slot_words;
+  p.args.err = solve_err_;
+  return true;
+}
+
+// places of the clusters' rows, one after the other
+template <typename T>
+std::vector<int> Engine<T>::flow_places(const FlowRows& R, const std::vector<int>& clusters) const {
+  std::vector<int> at;
+  for (int c : clusters)
+    for (const FlowSeg& sg : R.of[c])
+      for (int i = 0; i < sg.len; ++i) at.push_back(sg.off + i);
+  return at;
+}
+
+template <typename T>
+bool Engine<T>::build_flow() {
+  solve_err_ = (int*)perm_.alloc(256);
+  launch_zero(stream_, 4, solve_err_, 64);
+  scratch_.rewind();
+  // W of every op with reflectors
+  std::vector<WyJob<T>> wj;
+  std::vector<WyJob<double>> wj64;
+  for (auto& o : ops_) {
+    if (o.kind == OpSplitD || o.kind == OpMerge || o.k <= 0) continue;
+    if (o.V64) {
+      double* W = (double*)perm_.alloc(sizeof(double) * (size_t)o.m * o.k);
+      o.W = W;
+      wj64.push_back(WyJob<double>{o.V64, o.Tb64, W, o.ldv, o.m, o.k});
+    } else {
+      T* W = alloc_perm((size_t)o.m * o.k);
+      o.W = W;
+      wj.push_back(WyJob<T>{o.V, o.Tb, W, o.ldv, o.m, o.k});
+    }
+  }
+  build_w(wj);
+  build_w(wj64);
+  // stages of the forward and the backward tape; the FP64 top apart
+  std::vector<std::vector<const Op*>> by_level(nlevels_);
+  for (auto& o : ops_) by_level[o.level].push_back(&o);
+  std::vector<FlowStage> fwd, bwd;
+  const Op* top = nullptr;
+  for (auto& lv : by_level) {
+    FlowStage qr, sc, od;
+    qr.chain = od.up = true;
+    for (auto o : lv) {
+      if (o->kind == OpQR) {
+        if (o->V64) {
+          if (top || !o->r12.empty() || o->segs.size() != 1)
+            throw Error(kErrState, "FP64 top separator: unexpected op structure");
+          top = o;
+        } else if (o->k > 0) {
+          qr.items.push_back(FlowItem{o, kFlowWY, false});
+        }
+      } else if (o->kind == OpScaleD && o->k > 0) {
+        sc.items.push_back(FlowItem{o, kFlowWY, false});
+      } else if (o->kind == OpOrthoD && o->k > 0 && !o->nofwd) {
+        od.items.push_back(FlowItem{o, kFlowWY, false});
+      } else if (o->kind == OpSplitD) {
+        od.split.push_back(o);
+      } else if (o->kind == OpMerge) {
+        od.merge.push_back(o);
+      }
+    }
+    // the factorization's order: elimination wave, then creation
+    std::stable_sort(qr.items.begin(), qr.items.end(),
+                     [](const FlowItem& a, const FlowItem& b) { return a.op->wave < b.op->wave; });
+    fwd.push_back(std::move(qr));
+    fwd.push_back(std::move(sc));
+    fwd.push_back(std::move(od));
+  }
+  for (int l = nlevels_ - 1; l >= 0; --l) {
+    FlowStage dn, qr, sc, od;
+    for (auto o : by_level[l]) {
+      if (o->kind == OpOrthoD && o->k > 0) od.items.push_back(FlowItem{o, kFlowWY, true});
+      else if (o->kind == OpScaleD && o->k > 0) sc.items.push_back(FlowItem{o, kFlowBack, false});
+      else if (o->kind == OpQR && !o->V64 && o->kr > 0) qr.items.push_back(FlowItem{o, kFlowBack, false});
+      else if (o->kind == OpSplitD) dn.split.push_back(o);
+      else if (o->kind == OpMerge) dn.merge.push_back(o);
+    }
+    bwd.push_back(std::move(dn));
+    bwd.push_back(std::move(od));
+    bwd.push_back(std::move(sc));
+    bwd.push_back(std::move(qr));
+  }
+  // M^{-T}: the stages in reverse, each transposed (a stage that hands rows
+  // over does so after its items, the reverse one before them)
+  auto transpose = [](const std::vector<FlowStage>& src) {
+    std::vector<FlowStage> dst;
+    for (auto it = src.rbegin(); it != src.rend(); ++it) {
+      FlowStage st, mv;
+      st.items = it->items;
+      st.chain = it->chain;
+      mv.split = it->split;
+      mv.merge = it->merge;
+      mv.up = !it->up;
+      if (st.chain) std::reverse(st.items.begin(), st.items.end());
+      for (auto& q : st.items) {
+        q.trans = !q.trans;
+        if (q.type != kFlowWY) q.type = kFlowSolveT;
+      }
+      dst.push_back(std::move(mv));
+      dst.push_back(std::move(st));
+    }
+    return dst;
+  };
+  auto join = [](std::vector<FlowStage> a, const std::vector<FlowStage>& b) {
+    a.insert(a.end(), b.begin(), b.end());
+    return a;
+  };
+  const std::vector<FlowStage> first[2] = {fwd, transpose(bwd)}, second[2] = {bwd, transpose(fwd)};
+  const double bytes0 = solve_bytes_;
+  for (int t = 1; t >= 0; --t) {
+    solve_bytes_ = bytes0;  // in the end those of the forward apply
+    FlowMode& M = flow_mode_[t];
+    FlowRows R;
+    R.of.resize(cl_.size());
+    R.scratch.assign(cl_.size(), 0);
+    for (int c : bottoms_[0]) {
+      if (cl_[c].rsize_org > 0) R.of[c].push_back(FlowSeg{R.next, cl_[c].rsize_org});
+      R.next += cl_[c].rsize_org;
+    }
+    M.run.clear();
+    if (top) {
+      M.run.resize(2);
+      if (!flow_prog<T>(first[t], R, M.run[0])) return false;
+      const int c = top->c;
+      flow_top_n_ = top->m;
+      M.top_in = stager_.upload(perm_, flow_places(R, {c}));
+      FlowRows R64;
+      R64.of.resize(cl_.size());
+      R64.scratch.assign(cl_.size(), 0);
+      R64.of[c].push_back(FlowSeg{0, top->m});
+      R64.next = top->m;
+      std::vector<FlowStage> tf(1), tb(1);
+      tf[0].items.push_back(FlowItem{top, kFlowWY, false});
+      tb[0].items.push_back(FlowItem{top, kFlowBack, false});
+      if (!flow_prog<double>(t ? join(transpose(tb), transpose(tf)) : join(tf, tb), R64, M.top)) return false;
+      M.top_out = stager_.upload(perm_, flow_places(R64, {c}));
+      M.x64places = R64.next;
+      M.top_at = R.next;
+      R.of[c].assign(1, FlowSeg{R.next, top->m});
+      R.next += top->m;
+      if (!flow_prog<T>(second[t], R, M.run[1])) return false;
+    } else {
+      M.run.resize(1);
+      if (!flow_prog<T>(join(first[t], second[t]), R, M.run[0])) return false;
+    }
+    M.xplaces = R.next;
+    M.out = stager_.upload(perm_, flow_places(R, bottoms_[0]));
+  }
+  xsize_ = std::max(flow_mode_[0].xplaces, flow_mode_[1].xplaces);
+  SPQ_HIP(dev_malloc((void**)&xbuf_, sizeof(T) * std::max<int64_t>(xsize_, 1)));
+  if (top) SPQ_HIP(dev_malloc((void**)&x64_, sizeof(double) * std::max(flow_mode_[0].x64places, flow_mode_[1].x64places)));
+  SPQ_HIP(dev_malloc((void**)&bin_, sizeof(double) * std::max(nrows_, 1)));
+  SPQ_HIP(dev_malloc((void**)&xout_, sizeof(double) * std::max(ncols_, 1)));
+  for (auto& M : flow_mode_) {
+    for (auto& r : M.run) r.args.x = xbuf_;
+    M.top.args.x = x64_;
+  }
+  std::vector<int> rp, cp;
+  for (int c : bottoms_[0])
+    for (int i = 0; i < cl_[c].rsize_org; ++i) {
+      rp.push_back(rperm_[cl_[c].rstart + i]);
+      cp.push_back(cperm_[cl_[c].cstart + i]);
+    }
+  flow_rperm_ = stager_.upload(perm_, rp);
+  flow_cperm_ = stager_.upload(perm_, cp);
+  flow_ = true;
+  return true;
+}
+
 // Solve program: per level, forward stages QR (waves) -> ScaleD -> OrthogonalD
 // -> SplitD -> Merge, backward stages in the reverse order (tree.cpp:1440-1466).
 template <typename T>
 void Engine<T>::build_solve_program() {
+  const double bytes0 = solve_bytes_;
+  if (flow_fits() && build_flow()) return;
+  solve_bytes_ = bytes0;
   layout_x();
   // temporary segments for SplitD moves whose ranges overlap (least-squares
   // clusters with extra rows)
@@ -3340,6 +3845,22 @@ void Engine<T>::build_solve_program() {
 
 template <typename T>
 void Engine<T>::run_program(const double* b, double* x, bool prof, int mode) {
+  if (flow_) {
+    // M^{-T}: b enters through the exit map and leaves through the entry map
+    const FlowMode& M = flow_mode_[mode == 2];
+    launch_zero(stream_, sizeof(T), xbuf_, M.xplaces);
+    launch_flow_in<T>(stream_, mode == 2 ? flow_cperm_ : flow_rperm_, nrows_, b, xbuf_, 0);
+    run_flow(M.run[0]);
+    if (M.run.size() > 1) {
+      launch_zero(stream_, 8, x64_, M.x64places);
+      launch_flow_cvt<T, double>(stream_, M.top_in, flow_top_n_, xbuf_, x64_, 0);
+      run_flow(M.top);
+      launch_flow_cvt<double, T>(stream_, M.top_out, flow_top_n_, x64_, xbuf_, M.top_at);
+      run_flow(M.run[1]);
+    }
+    launch_flow_out<T>(stream_, M.out, nrows_, xbuf_, mode == 2 ? flow_rperm_ : flow_cperm_, x);
+    return;
+  }
   launch_zero(stream_, sizeof(T), xbuf_, xsize_);
   if (n_solve_sync_ > 0) launch_zero(stream_, 4, solve_sync_, n_solve_sync_);
   std::vector<hipEvent_t> ev;

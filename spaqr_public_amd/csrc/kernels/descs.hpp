@@ -268,6 +268,54 @@ struct R12Chunk {
   int ld, k, nc, trans;
 };
 
+// The dataflow apply (flow.hip).  Ops in tape order; an op has nwg parts, each
+// drawn by one workgroup.  Inputs are segments [seg0, seg0 + nseg) of earlier
+// outputs in x, outputs the places from `out` on.
+//   kFlowWY      x - B (A^T x) on m rows, A and B m x k: (V, W) for H^T, (W, V)
+//                for H; parts of rows_per rows
+//   kFlowBack    R^{-1} (x_c - sum_n A_n x_n), R = A (k x k); blocks [blk0,
+//                blk0 + nblk) are up to 32 columns of an A_n with the places of
+//                their x values
+//   kFlowSolveT  R^{-T} x_c
+//   kFlowPull    x_n - sum_c A_c^T x_c on m rows; blocks are up to 64 rows of an
+//                A_c with the places of their x values; parts of 32 rows
+enum : int { kFlowWY = 0, kFlowBack = 1, kFlowSolveT = 2, kFlowPull = 3 };
+constexpr int kFlowMaxK = 1024;     // columns of an op, rows of a part
+constexpr int kFlowMaxSegs = 1024;  // input segments of an op
+constexpr int kFlowMaxParts = 32;   // parts of an op that wait for each other
+template <typename T>
+struct FlowOp {
+  const T* A;
+  const T* B;          // triangular ops: the diagonal blocks as k_flow_diag leaves them
+  T* slots;            // nwg x k exchange slots, zero on entry
+  int lda, ldb, m, k;
+  int unit_a, unit_b;  // 1: unit lower trapezoidal (V), 0: lower trapezoidal (W)
+  int type, nwg, rows_per, g;  // g: this part (the table has an entry for each)
+  int seg0, nseg, blk0, nblk, out, pad_;
+};
+template <typename T>
+struct FlowDiag {
+  const T* R;
+  T* D;
+  int ld, k, tr, pad_;
+};
+struct FlowSeg { int off, len; };  // places in x
+template <typename T>
+struct FlowBlk {
+  const T* A;
+  int ld, n, off, pad_;
+};
+template <typename T>
+struct FlowArgs {
+  const FlowOp<T>* parts;
+  const FlowSeg* segs;
+  const FlowBlk<T>* blks;
+  T* x;               // zero where no value is yet
+  unsigned int* ctl;  // tickets; zero on entry
+  int* err;
+  int nparts;
+};
+
 // Vector segment move dst[0:len] = src[0:len] (x-buffer offsets).
 struct MoveDesc {
   int64_t src, dst;

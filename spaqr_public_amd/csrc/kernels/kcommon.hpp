@@ -162,6 +162,14 @@ __device__ __forceinline__ void store_at(T* base, unsigned byte_off, T v) {
   *(gmut<T>)((__attribute__((address_space(1))) char*)to_global_mut(base) + byte_off) = v;
 }
 
+// a pointer every lane of the wave holds alike, as a scalar
+template <typename T>
+__device__ __forceinline__ const T* uniform_ptr(const T* p) {
+  const unsigned long long b = (unsigned long long)p;
+  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
+  return (const T*)(((unsigned long long)hi << 32) | lo);
+}
 // Value of v in lane l (l uniform) for every lane of the wave.
 __device__ __forceinline__ double lane_bcast(double v, int l) {
   const unsigned long long b = __double_as_longlong(v);
@@ -411,6 +419,65 @@ __device__ __forceinline__ void group_barrier2_rx(unsigned int* sync, int g, int
     barrier_wait_rx(sync, phase * (unsigned int)ngrp, err);
   }
   __syncthreads();
+}
+
+// ---------------------------------------------------------------------------
+// Values handed over without a barrier: a slot holds the value's complement and
+// is zero until then (the host clears it), so a reader polls the values
+// themselves: one trip through memory for the store and one for the load,
+// where a counter in between takes three.
+template <int BYTES>
+struct Bits;
+template <>
+struct Bits<4> { using type = unsigned int; };
+template <>
+struct Bits<8> { using type = unsigned long long; };
+template <typename T>
+__device__ __forceinline__ void slot_put(T* slots, int64_t at, bool on, T v) {
+  using B = typename Bits<sizeof(T)>::type;
+  B b;
+  __builtin_memcpy(&b, &v, sizeof(T));
+  b = ~b;
+  if (b == 0) b = 1;  // the NaN of all ones becomes its neighbour
+  if (on) __hip_atomic_store(to_global_mut((B*)slots) + at, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Sum over the first `cnt` of nwg slots `stride` apart, in order, waiting for
+// each, U loads in flight.  The wait is bounded as in barrier_wait_rx.
+template <typename T, int U>
+__device__ __forceinline__ T slot_sum(const T* slots, int stride, int cnt, int nwg, int* err) {
+  using B = typename Bits<sizeof(T)>::type;
+  const gmut<B> at = to_global_mut((B*)const_cast<T*>(slots));
+  T sum = T(0);
+  unsigned int spins = 0;
+  for (int q0 = 0; q0 < nwg; q0 += U) {
+    B b[U];
+    for (;;) {
+      bool ok = true;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        b[u] = q0 + u < cnt
+                   ? __hip_atomic_load(at + (int64_t)(q0 + u) * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                   : B(1);
+#pragma unroll
+      for (int u = 0; u < U; ++u) ok = ok & (b[u] != 0);
+      if (ok) break;
+      __builtin_amdgcn_s_sleep(1);
+      ++spins;
+      if ((spins & 255u) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
+      if (spins > (1u << 20)) {
+        atomicOr(err, 1);
+        break;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const B v = ~b[u];
+      T x;
+      __builtin_memcpy(&x, &v, sizeof(T));
+      sum += (q0 + u < cnt) ? x : T(0);
+    }
+  }
+  return sum;
 }
 
 // Find the descriptor owning flattened tile `t` given exclusive prefix sums

@@ -117,6 +117,23 @@ void launch_gather_in(hipStream_t s, const int64_t* dst, const int* src, int n, 
 template <typename T>
 void launch_scatter_out(hipStream_t s, const int64_t* src, const int* dst, int n, const T* xbuf, double* x);
 
+// flow.hip: the dataflow apply on `grid` workgroups (flow_capacity at most)
+template <typename T>
+int flow_capacity();
+template <typename T>
+void launch_flow(hipStream_t s, const FlowArgs<T>& a, int grid);
+// the diagonal blocks of triangular factors as k_flow reads them (flow_diag_elems
+// entries each); start: exclusive prefix sums of ceil(k / 32)
+template <typename T>
+void launch_flow_diag(hipStream_t s, const FlowDiag<T>* d, const int* start, int nd, int nblocks);
+// values into places [at, at + n) of a dataflow x, and out of places loc
+template <typename T>
+void launch_flow_in(hipStream_t s, const int* src, int n, const double* b, T* x, int at);
+template <typename T>
+void launch_flow_out(hipStream_t s, const int* loc, int n, const T* x, const int* dst, double* y);
+template <typename T, typename D>
+void launch_flow_cvt(hipStream_t s, const int* loc, int n, const T* x, D* y, int at);
+
 // smin.hip
 int smin_max_k();
 size_t smin_work_elems(int k);

@@ -61,61 +61,6 @@ __device__ __forceinline__ void t_factor(const T (&Gs)[kNB][kNB], const T (&taus
 // complement and is zero until then, so a reader polls the values themselves
 // (one trip through memory for the store and one for the load; a counter
 // barrier between them takes three).  Every step has its own slots.
-template <int BYTES>
-struct Bits;
-template <>
-struct Bits<4> { using type = unsigned int; };
-template <>
-struct Bits<8> { using type = unsigned long long; };
-template <typename T>
-__device__ __forceinline__ void exchange_put(T* slots, int64_t at, bool on, T v) {
-  using B = typename Bits<sizeof(T)>::type;
-  B b;
-  __builtin_memcpy(&b, &v, sizeof(T));
-  b = ~b;
-  if (b == 0) b = 1;  // the NaN of all ones becomes its neighbour
-  if (on) __hip_atomic_store((gmut<B>)to_global_mut((B*)slots) + at, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// sum over the first `cnt` of nwg slots 64 apart, waiting for each; all lanes of
-// the wave take part.  The wait is bounded as in barrier_wait_rx.
-template <typename T>
-__device__ __forceinline__ T exchange_sum(const T* slots, int cnt, int nwg, int* err) {
-  using B = typename Bits<sizeof(T)>::type;
-  const gmut<B> at = to_global_mut((B*)const_cast<T*>(slots));
-  T sum = T(0);
-  unsigned int spins = 0;
-  for (int q0 = 0; q0 < nwg; q0 += 8) {
-    B b[8];
-    for (;;) {
-      bool ok = true;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        b[u] = q0 + u < cnt ? __hip_atomic_load(at + (int64_t)(q0 + u) * (2 * kNB), __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT)
-                            : B(1);
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) ok = ok & (b[u] != 0);
-      if (__ballot(!ok) == 0) break;
-      __builtin_amdgcn_s_sleep(1);
-      ++spins;
-      if ((spins & 255u) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
-      if (spins > (1u << 20)) {
-        atomicOr(err, 1);
-        break;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const B v = ~b[u];
-      T x;
-      __builtin_memcpy(&x, &v, sizeof(T));
-      sum += (q0 + u < cnt) ? x : T(0);
-    }
-  }
-  return sum;
-}
-
 template <typename T>
 __device__ __forceinline__ T panel_rcp(T v) {
   if constexpr (sizeof(T) == 8) return rcp_nr(v);
@@ -218,10 +163,11 @@ __global__ __launch_bounds__(NW * kWave) void k_panel_r(const PanelDesc<T>* __re
     if (nwg > 1) {
       // wave 0 exchanges the sums (lanes < 32) and row j (lanes >= 32)
       if (w == 0) {
-        exchange_put(d.part, (jj * nwg + wg) * (2 * kNB) + lane, wg == 0 || lane < kNB,
-                     lane < kNB ? dot : rowv[buf][lc]);
+        slot_put(d.part, (int64_t)(jj * nwg + wg) * (2 * kNB) + lane, wg == 0 || lane < kNB,
+                 lane < kNB ? dot : rowv[buf][lc]);
         // the sums of all workgroups in workgroup order; row j from the first
-        const T v = exchange_sum(d.part + (int64_t)jj * nwg * (2 * kNB) + lane, lane < kNB ? nwg : 1, nwg, d.err);
+        const T v = slot_sum<T, 8>(d.part + (int64_t)jj * nwg * (2 * kNB) + lane, 2 * kNB, lane < kNB ? nwg : 1, nwg,
+                                   d.err);
         if (lane < kNB) dsh[lane] = v;
         else if (wg != 0) rowv[buf][lc] = v;
       }

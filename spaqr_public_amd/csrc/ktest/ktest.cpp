@@ -276,7 +276,86 @@ int rrqr_one(int k, int N, X* Ct, X* V, X* tau, double tol, int nd, int* perm, i
   return h.next;
 }
 }  // namespace
+namespace {
+// One dataflow op (kernels/flow.hip) on x (m values) and, for the triangular
+// and the pull form, xn (n values) with the block Bn: the inputs lie in two
+// segments in reverse order, the blocks' tiles start with a short one.
+//   WY: A, B m x k (lda, ldb), parts of rows_per rows; unit: A is V, B is W
+//   Back: R = A (k x k, m = k), Bn k x n (ldb), nwg parts; SolveT: R alone
+//   Pull: Bn = B n x m (ldb)
+template <typename T>
+int flow_one(int type, int m, int k, int par, int unit, const T* A, int lda, const T* B, int ldb, int n,
+             const double* x, const double* xn, double* out) {
+  const int h = m / 3, total = 2 * m + n + 7;
+  std::vector<FlowSeg> segs;
+  if (m - h > 0) segs.push_back(FlowSeg{h, m - h});  // rows 0 .. m-h-1 of x lie after the others
+  if (h > 0) segs.push_back(FlowSeg{0, h});
+  std::vector<double> xin(m + n);
+  for (int i = 0; i < m; ++i) xin[i < m - h ? h + i : i - (m - h)] = x[i];
+  for (int i = 0; i < n; ++i) xin[m + i] = xn[i];
+  const bool tri = type == kFlowBack || type == kFlowSolveT, wy = type == kFlowWY;
+  T* dA = A ? dup(A, (size_t)lda * k) : nullptr;
+  T* dB = B ? dup(B, (size_t)ldb * (wy ? k : (type == kFlowPull ? m : n))) : nullptr;
+  std::vector<FlowBlk<T>> blks;
+  if (type == kFlowBack)
+    for (int j = 0; j < n;) {
+      const int w = std::min(j == 0 ? 5 : 32, n - j);
+      blks.push_back(FlowBlk<T>{dB + (size_t)j * ldb, ldb, w, m + j, 0});
+      j += w;
+    }
+  if (type == kFlowPull)
+    for (int r = 0; r < n;) {
+      const int w = std::min(r == 0 ? 7 : 64, n - r);
+      blks.push_back(FlowBlk<T>{dB + r, ldb, w, m + r, 0});
+      r += w;
+    }
+  FlowOp<T> d{};
+  d.type = type; d.m = m; d.k = wy || tri ? k : 32;
+  d.A = dA; d.lda = lda; d.B = dB; d.ldb = ldb;
+  d.unit_a = unit; d.unit_b = !unit;
+  d.rows_per = par;
+  d.nwg = wy ? (m + par - 1) / par : (tri ? par : 1);
+  d.nseg = (int)segs.size(); d.nblk = (int)blks.size(); d.out = m + n + 7;
+  const int nb = (k + 31) / 32, np = type == kFlowPull ? (m + 31) / 32 : d.nwg;
+  d.slots = dup<T>(nullptr, (size_t)d.nwg * d.k);
+  T* dx = dup<T>(nullptr, total);
+  unsigned int* ctl = dup<unsigned int>(nullptr, 64);
+  int* err = dup<int>(nullptr, 64);
+  if (tri) {
+    T* D = dup<T>(nullptr, (size_t)nb * 32 * 33);
+    FlowDiag<T> fd{dA, D, lda, k, type == kFlowSolveT, 0};
+    const int st[2] = {0, nb};
+    launch_flow_diag<T>(0, dup(&fd, 1), dup(st, 2), 1, nb);
+    d.B = D;
+  }
+  std::vector<FlowOp<T>> parts;
+  for (int g = 0; g < np; ++g) { d.g = g; parts.push_back(d); }
+  FlowArgs<T> a{};
+  a.parts = dup(parts.data(), parts.size());
+  a.segs = dup(segs.data(), segs.size());
+  a.blks = blks.empty() ? nullptr : dup(blks.data(), blks.size());
+  a.x = dx; a.ctl = ctl; a.err = err; a.nparts = np;
+  launch_flow_in<T>(0, nullptr, m + n, dup(xin.data(), xin.size()), dx, 0);
+  launch_flow<T>(0, a, std::min(np, flow_capacity<T>()));
+  std::vector<int> loc(m);
+  for (int i = 0; i < m; ++i) loc[i] = d.out + i;
+  double* dy = dup<double>(nullptr, m);
+  launch_flow_out<T>(0, dup(loc.data(), loc.size()), m, dx, nullptr, dy);
+  KT(hipMemcpy(out, dy, sizeof(double) * m, hipMemcpyDeviceToHost));
+  int e = 0;
+  KT(hipMemcpy(&e, err, sizeof(int), hipMemcpyDeviceToHost));
+  return e;
+}
+}  // namespace
 extern "C" {
+int ktest_flow(int type, int m, int k, int par, int unit, const double* A, int lda, const double* B, int ldb, int n,
+               const double* x, const double* xn, double* out) {
+  return flow_one<double>(type, m, k, par, unit, A, lda, B, ldb, n, x, xn, out);
+}
+int ktest_flow_f32(int type, int m, int k, int par, int unit, const float* A, int lda, const float* B, int ldb, int n,
+                   const double* x, const double* xn, double* out) {
+  return flow_one<float>(type, m, k, par, unit, A, lda, B, ldb, n, x, xn, out);
+}
 int ktest_rrqr(int k, int N, double* Ct, double* V, double* tau, double tol, int nd, int* perm, int* rounds) {
   return rrqr_one<double>(k, N, Ct, V, tau, tol, nd, perm, rounds);
 }
