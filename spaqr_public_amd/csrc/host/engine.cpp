@@ -796,7 +796,7 @@ class Engine final : public EngineBase {
   struct FlowProg {
     FlowArgs<U> args{};
     int grid = 0;
-    unsigned int* zero = nullptr;  // exchange slots and tickets, cleared before each run
+    unsigned int* zero = nullptr;  // exchange slots and tickets, cleared before each apply
     int64_t nzero = 0;             // words
   };
   // places of x holding the rows of each cluster, as segments
@@ -812,11 +812,7 @@ class Engine final : public EngineBase {
   template <typename U>
   bool flow_prog(const std::vector<FlowStage>& stages, FlowRows& rows, FlowProg<U>& out);
   std::vector<int> flow_places(const FlowRows& rows, const std::vector<int>& clusters) const;
-  template <typename U>
-  void run_flow(const FlowProg<U>& p) {
-    launch_zero(stream_, 4, p.zero, p.nzero);
-    launch_flow<U>(stream_, p.args, p.grid);
-  }
+  void run_flow(const double* b, double* x, bool transposed);
   // modes 0 and 2 (M^{-1}, M^{-T}): one program, or around the FP64 top of an
   // FP32 tree one before and one after it
   struct FlowMode {
@@ -830,6 +826,8 @@ class Engine final : public EngineBase {
   };
   bool flow_ = false;
   FlowMode flow_mode_[2];
+  T* flow_x_ = nullptr;
+  double* flow_x64_ = nullptr;
   int flow_top_n_ = 0;
   const int *flow_rperm_ = nullptr, *flow_cperm_ = nullptr;  // rows and columns in cluster order
   // ------------------------------------------------------------ state
@@ -2786,7 +2784,7 @@ int Engine<T>::factorize() {  // tree.cpp:1309-1437
   build_solve_program();
   // the apply's graph is instantiated here, so solves (and the Krylov drivers
   // around them) allocate nothing on the device
-  if (solve_graph_ && !stage_prof_) {
+  if (solve_graph_ && !stage_prof_ && !flow_) {
     if (square_) graph_exec_fwd_ = capture_program(0);
     else graph_exec_nrml_ = capture_program(1);
   }
@@ -3227,13 +3225,12 @@ bool Engine<T>::build_flow() {
     M.out = stager_.upload(perm_, flow_places(R, bottoms_[0]));
   }
   xsize_ = std::max(flow_mode_[0].xplaces, flow_mode_[1].xplaces);
-  SPQ_HIP(dev_malloc((void**)&xbuf_, sizeof(T) * std::max<int64_t>(xsize_, 1)));
-  if (top) SPQ_HIP(dev_malloc((void**)&x64_, sizeof(double) * std::max(flow_mode_[0].x64places, flow_mode_[1].x64places)));
-  SPQ_HIP(dev_malloc((void**)&bin_, sizeof(double) * std::max(nrows_, 1)));
-  SPQ_HIP(dev_malloc((void**)&xout_, sizeof(double) * std::max(ncols_, 1)));
+  flow_x_ = alloc_perm((size_t)xsize_);
+  if (top)
+    flow_x64_ = (double*)perm_.alloc(sizeof(double) * (size_t)std::max(flow_mode_[0].x64places, flow_mode_[1].x64places));
   for (auto& M : flow_mode_) {
-    for (auto& r : M.run) r.args.x = xbuf_;
-    M.top.args.x = x64_;
+    for (auto& r : M.run) r.args.x = flow_x_;
+    M.top.args.x = flow_x64_;
   }
   std::vector<int> rp, cp;
   for (int c : bottoms_[0])
@@ -3843,24 +3840,38 @@ void Engine<T>::build_solve_program() {
   }
 }
 
+// An apply of the dataflow program: three launches (seven around an FP64 top)
+// on the stream.  b is read by the first only, so it may alias x; a graph would
+// need both at fixed addresses, and two copies with it.
+template <typename T>
+void Engine<T>::run_flow(const double* b, double* x, bool transposed) {
+  const FlowMode& M = flow_mode_[transposed];
+  FlowClear c{};
+  auto clear = [&, i = 0](void* p, int64_t words) mutable {
+    c.p[i] = (unsigned int*)p;
+    c.n[i++] = words;
+  };
+  clear(flow_x_ + nrows_, (int64_t)(M.xplaces - nrows_) * (int64_t)(sizeof(T) / 4));
+  for (auto& r : M.run) clear(r.zero, r.nzero);
+  const bool top = M.run.size() > 1;
+  if (top) {
+    clear(flow_x64_, 2 * (int64_t)M.x64places);
+    clear(M.top.zero, M.top.nzero);
+  }
+  // M^{-T}: b enters through the exit map and leaves through the entry map
+  launch_flow_begin<T>(stream_, transposed ? flow_cperm_ : flow_rperm_, nrows_, b, flow_x_, c);
+  launch_flow<T>(stream_, M.run[0].args, M.run[0].grid);
+  if (top) {
+    launch_flow_cvt<T, double>(stream_, M.top_in, flow_top_n_, flow_x_, flow_x64_, 0);
+    launch_flow<double>(stream_, M.top.args, M.top.grid);
+    launch_flow_cvt<double, T>(stream_, M.top_out, flow_top_n_, flow_x64_, flow_x_, M.top_at);
+    launch_flow<T>(stream_, M.run[1].args, M.run[1].grid);
+  }
+  launch_flow_out<T>(stream_, M.out, nrows_, flow_x_, transposed ? flow_rperm_ : flow_cperm_, x);
+}
+
 template <typename T>
 void Engine<T>::run_program(const double* b, double* x, bool prof, int mode) {
-  if (flow_) {
-    // M^{-T}: b enters through the exit map and leaves through the entry map
-    const FlowMode& M = flow_mode_[mode == 2];
-    launch_zero(stream_, sizeof(T), xbuf_, M.xplaces);
-    launch_flow_in<T>(stream_, mode == 2 ? flow_cperm_ : flow_rperm_, nrows_, b, xbuf_, 0);
-    run_flow(M.run[0]);
-    if (M.run.size() > 1) {
-      launch_zero(stream_, 8, x64_, M.x64places);
-      launch_flow_cvt<T, double>(stream_, M.top_in, flow_top_n_, xbuf_, x64_, 0);
-      run_flow(M.top);
-      launch_flow_cvt<double, T>(stream_, M.top_out, flow_top_n_, x64_, xbuf_, M.top_at);
-      run_flow(M.run[1]);
-    }
-    launch_flow_out<T>(stream_, M.out, nrows_, xbuf_, mode == 2 ? flow_rperm_ : flow_cperm_, x);
-    return;
-  }
   launch_zero(stream_, sizeof(T), xbuf_, xsize_);
   if (n_solve_sync_ > 0) launch_zero(stream_, 4, solve_sync_, n_solve_sync_);
   std::vector<hipEvent_t> ev;
@@ -3945,6 +3956,10 @@ template <typename T>
 void Engine<T>::solve_dev(const double* b, double* x) {
   if (!factored_) throw Error(kErrState, "solve before factorize");
   if (!square_) throw Error(kErrState, "solve: rectangular (least-squares) tree; use solve_nrml");
+  if (flow_) {
+    timed("apply", 0.0, solve_bytes_, [&] { run_flow(b, x, false); });
+    return;
+  }
   // b is taken by value (tree.cpp:1440): copy into the program's fixed input,
   // replay the captured apply, copy the fixed output out.
   SPQ_HIP(hipMemcpyAsync(bin_, b, sizeof(double) * nrows_, hipMemcpyDeviceToDevice, stream_));
@@ -3980,6 +3995,10 @@ template <typename T>
 void Engine<T>::solve_t_dev(const double* b, double* x) {
   if (!factored_) throw Error(kErrState, "solve_transpose before factorize");
   if (!square_) throw Error(kErrState, "solve_transpose: rectangular (least-squares) tree");
+  if (flow_) {
+    timed("apply", 0.0, solve_bytes_, [&] { run_flow(b, x, true); });
+    return;
+  }
   SPQ_HIP(hipMemcpyAsync(bin_, b, sizeof(double) * ncols_, hipMemcpyDeviceToDevice, stream_));
   if (stage_prof_ || !solve_graph_) {
     timed("apply", 0.0, solve_bytes_, [&] { run_program(bin_, xout_, stage_prof_, 2); });

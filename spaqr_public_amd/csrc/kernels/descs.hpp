@@ -293,6 +293,11 @@ struct FlowOp {
   int type, nwg, rows_per, g;  // g: this part (the table has an entry for each)
   int seg0, nseg, blk0, nblk, out, pad_;
 };
+// what an apply clears before it runs: words of 4 bytes
+struct FlowClear {
+  unsigned int* p[5];
+  int64_t n[5];
+};
 template <typename T>
 struct FlowDiag {
   const T* R;

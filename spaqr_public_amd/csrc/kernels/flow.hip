@@ -24,7 +24,8 @@
 // what could not be fetched ahead; a part that exchanges sums 1.2 us more; a
 // triangular block of 32 rows 0.9 us (3.3 us as k_bwdr's block step).  Whole
 // applies, against one kernel per stage with a graph around them: 2-D 64^2 472
-// -> 165 us, 3-D 40^3 2.9 -> 0.8 ms, 52^3 5.3 -> 1.6 ms.
+// -> 146 us, 3-D 40^3 2.9 -> 0.8 ms, 52^3 5.3 -> 1.6 ms (the first with the launches
+// of launch_flow_begin; 165 us inside a graph of seven nodes).
 //
 // Progress: a workgroup waits only for ops with earlier tickets and for the
 // other parts of its own op.  Tickets are drawn when a workgroup is running
@@ -589,13 +590,14 @@ template int flow_capacity<float>();
 template void launch_flow<double>(hipStream_t, const FlowArgs<double>&, int);
 template void launch_flow<float>(hipStream_t, const FlowArgs<float>&, int);
 
-// places [at, at + n) of x from b, and y from places of x (sources and
-// destinations through index lists, identity where null)
-template <typename T, typename S>
-__global__ __launch_bounds__(256) void k_flow_in(const int* __restrict__ src, int n, const S* __restrict__ b, T* x,
-                                                 int at) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) slot_put(x, (int64_t)at + i, true, (T)b[src ? src[i] : i]);
+template <typename T>
+__global__ __launch_bounds__(256) void k_flow_begin(const int* __restrict__ src, int n, const double* __restrict__ b,
+                                                    T* x, FlowClear c) {
+  const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+  for (int64_t i = i0; i < n; i += step) slot_put(x, i, true, (T)b[src ? src[i] : i]);
+#pragma unroll
+  for (int q = 0; q < 5; ++q)
+    for (int64_t i = i0; i < c.n[q]; i += step) c.p[q][i] = 0;
 }
 template <typename T, typename D>
 __global__ __launch_bounds__(256) void k_flow_out(const int* __restrict__ loc, int n, const T* __restrict__ x,
@@ -608,7 +610,7 @@ __global__ __launch_bounds__(256) void k_flow_out(const int* __restrict__ loc, i
   __builtin_memcpy(&v, &b, sizeof(T));
   y[dst ? dst[i] : i] = (D)v;
 }
-// the same from places of one x to places of another
+// values of places of one x in places of another
 template <typename T, typename D>
 __global__ __launch_bounds__(256) void k_flow_cvt(const int* __restrict__ loc, int n, const T* __restrict__ x, D* y,
                                                   int at) {
@@ -621,8 +623,12 @@ __global__ __launch_bounds__(256) void k_flow_cvt(const int* __restrict__ loc, i
   slot_put(y, (int64_t)at + i, true, (D)v);
 }
 template <typename T>
-void launch_flow_in(hipStream_t s, const int* src, int n, const double* b, T* x, int at) {
-  if (n > 0) hipLaunchKernelGGL((k_flow_in<T, double>), dim3((n + 255) / 256), dim3(256), 0, s, src, n, b, x, at);
+void launch_flow_begin(hipStream_t s, const int* src, int n, const double* b, T* x, const FlowClear& c) {
+  int64_t most = n;
+  for (int64_t w : c.n) most = std::max(most, w);
+  if (most <= 0) return;
+  hipLaunchKernelGGL((k_flow_begin<T>), dim3(std::min<int64_t>((most + 255) / 256, 2048)), dim3(256), 0, s, src, n, b, x,
+                     c);
 }
 template <typename T>
 void launch_flow_out(hipStream_t s, const int* loc, int n, const T* x, const int* dst, double* y) {
@@ -632,8 +638,8 @@ template <typename T, typename D>
 void launch_flow_cvt(hipStream_t s, const int* loc, int n, const T* x, D* y, int at) {
   if (n > 0) hipLaunchKernelGGL((k_flow_cvt<T, D>), dim3((n + 255) / 256), dim3(256), 0, s, loc, n, x, y, at);
 }
-template void launch_flow_in<double>(hipStream_t, const int*, int, const double*, double*, int);
-template void launch_flow_in<float>(hipStream_t, const int*, int, const double*, float*, int);
+template void launch_flow_begin<double>(hipStream_t, const int*, int, const double*, double*, const FlowClear&);
+template void launch_flow_begin<float>(hipStream_t, const int*, int, const double*, float*, const FlowClear&);
 template void launch_flow_out<double>(hipStream_t, const int*, int, const double*, const int*, double*);
 template void launch_flow_out<float>(hipStream_t, const int*, int, const float*, const int*, double*);
 template void launch_flow_cvt<float, double>(hipStream_t, const int*, int, const float*, double*, int);
