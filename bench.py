@@ -28,7 +28,7 @@ FAMILY_KERNEL = {
     "qp3s": "spq::k_qp3<{T}>", "rrqr_init": "spq::k_rrqr_init<{T}>", "rrqr_upd": "spq::k_rrqr_update<{T}>",
     "panel": "spq::k_panel_r<{T}>", "gemm": "spq::k_gemm<{T}>", "larft": "spq::k_larft<{T}>",
     "trsm": "spq::k_trsm_block<{T}>", "copy": "spq::k_copy", "init": "spq::k_init_blocks",
-    "apply": "solve program (hipGraph of k_refl/k_bwd/k_move)",
+    "larfb": "spq::k_larfb<{T}>", "wy": "spq::k_gemm<{T}>", "apply": "spq::k_flow<{T}>",
 }
 
 

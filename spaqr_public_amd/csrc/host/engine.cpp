@@ -623,14 +623,8 @@ class Engine final : public EngineBase {
           if (rc != 0) throw Error(kErrHip, std::string("panel launch failed: ") + hipGetErrorString((hipError_t)rc));
         });
       }
-      // trailing matrices: C -= (V_b T_b^T)(V_b^T C).  W = V_b T_b^T is formed
-      // once per problem in the same launch as the Y = V_b^T C of its
-      // targets (W and Y live in ws_, rewound per step); T_b's strict lower
-      // part is stored as zeros, so it enters as a dense factor
-      auto& bufs = larfb_bufs<U>();
-      auto &g1 = bufs.g1, &g3 = bufs.g3;
       // the step's targets of job q: its trailing columns, then its extra
-      // matrices with columns, in that order (larfb_step_descs' order)
+      // matrices with columns
       auto targets = [&](int q, std::vector<LarfbTarget<U>>& tg) {
         auto& j = jobs[q];
         tg.clear();
@@ -639,69 +633,115 @@ class Engine final : public EngineBase {
         for (auto& b : j.extra)
           if (b.cols > 0) tg.push_back({b.p + jb, b.ld, b.cols});
       };
-      // pass 1: per live job its descriptor counts and the bytes of its W
-      // and Y products (each allocation 256-aligned, as the arena places
-      // them), so every job's tables and scratch have fixed offsets
-      const int nl = (int)live.size();
-      std::vector<size_t> n1(nl + 1, 0), n3(nl + 1, 0), nby(nl + 1, 0);
-      auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-      parallel_for(nl, 256, [&](int, int b, int e) {
-        std::vector<LarfbTarget<U>> tg;
-        for (int i = b; i < e; ++i) {
-          targets(live[i], tg);
-          if (tg.empty()) continue;
-          const int rows = jobs[live[i]].m - jb;
-          size_t by = al(sizeof(U) * (size_t)std::max<int64_t>((int64_t)std::max(rows, 1) * nb_, 1));
-          for (auto& t : tg) by += al(sizeof(U) * (size_t)std::max<int64_t>((int64_t)nb_ * t.cols, 1));
-          n1[i + 1] = 1 + tg.size();
-          n3[i + 1] = tg.size();
-          nby[i + 1] = by;
-        }
-      });
-      for (int i = 0; i < nl; ++i) { n1[i + 1] += n1[i]; n3[i + 1] += n3[i]; nby[i + 1] += nby[i]; }
-      if (g1.size() < n1[nl]) g1.resize(n1[nl]);
-      if (g3.size() < n3[nl]) g3.resize(n3[nl]);
-      char* wbase = nby[nl] ? (char*)ws_.alloc(nby[nl]) : nullptr;
-      // pass 2: the descriptors, written at those offsets
-      parallel_for(nl, 64, [&](int, int b, int e) {
-        std::vector<LarfbTarget<U>> tg;
-        struct Out {
-          GemmDesc<U>* p;
-          void push_back(const GemmDesc<U>& d) { *p++ = d; }
-        };
-        for (int i = b; i < e; ++i) {
-          const int q = live[i];
-          auto& j = jobs[q];
-          targets(q, tg);
-          if (tg.empty()) continue;
-          const int w = std::min(nb_, std::min(j.m, j.k) - jb);
-          const int rows = j.m - jb;
-          const U* Vb = j.P + jb + (int64_t)jb * j.ld;
-          const U* Tb = j.Tb + (int64_t)jb * nb_;
-          char* cur = wbase + nby[i];
-          auto alloc = [&](int64_t elems) {
-            U* p = (U*)cur;
-            cur += al(sizeof(U) * (size_t)std::max<int64_t>(elems, 1));
-            return p;
-          };
-          Out o1{g1.data() + n1[i]}, o3{g3.data() + n3[i]};
-          larfb_step_descs<U>(Vb, j.ld, Tb, nb_, rows, w, tg.data(), (int)tg.size(), alloc, o1, o3);
-        }
-      });
-      const GemmLaunch<U> l1 = gemm_plan(g1.data(), n1[nl], "gemm_y");
-      const GemmLaunch<U> l3 = gemm_plan(g3.data(), n3[nl], "gemm_c");
-      run.push_back([this, l1, l3] {
-        gemm_launch(l1);
-        gemm_launch(l3);
-      });
+      // targets: k_larfb, in the least form that holds the rows (a form with
+      // few tiles joins the next used one: a launch costs more than its empty
+      // row tiles), and two GEMMs for more rows than its largest form holds
+      const int nf = larfb_forms();
+      std::vector<std::vector<int>> by_form(nf + 1);
+      std::vector<size_t> form_tiles(nf + 1, 0);
+      for (int q : live) {
+        const int rows = jobs[q].m - jb;
+        int f = 0;
+        while (f < nf && rows > larfb_form_rows(f)) ++f;
+        by_form[f].push_back(q);
+        const int c0 = jb + std::min(nb_, jobs[q].k - jb);
+        form_tiles[f] += larfb_tiles(jobs[q].k - c0);
+        for (auto& b : jobs[q].extra) form_tiles[f] += larfb_tiles(b.cols);
+      }
+      for (int f = 0; f + 1 < nf; ++f) {
+        if (by_form[f].empty() || form_tiles[f] >= (size_t)8 * num_cus_) continue;
+        int g = f + 1;
+        while (g < nf && by_form[g].empty()) ++g;
+        if (g == nf) continue;
+        by_form[g].insert(by_form[g].end(), by_form[f].begin(), by_form[f].end());
+        form_tiles[g] += form_tiles[f];
+        by_form[f].clear();
+      }
+      size_t planned = 0;
+      for (int f = 0; f < nf; ++f)
+        if (!by_form[f].empty()) planned += larfb_plan<U>(jobs, by_form[f], f, jb, targets, run);
+      if (!by_form[nf].empty()) larfb_gemms<U>(jobs, by_form[nf], jb, targets, run);
       // a step whose planning costs more host time than an upload (the
       // batches of many small problems) is launched at once, so the next
       // step is planned while it runs
-      if (n1[nl] + n3[nl] >= 4096) {
+      if (planned >= 2048) {
         for (auto& f : run) f();
         run.clear();
       }
     }
+  }
+
+  // k_larfb over the targets of jobs `qs` in form f; returns their number
+  template <typename U, typename Targets>
+  size_t larfb_plan(std::vector<QrJobT<U>>& jobs, const std::vector<int>& qs, int f, int jb, Targets&& targets, Run& run) {
+    auto& ds = larfb_bufs<U>().ds;
+    const int nq = (int)qs.size();
+    std::vector<size_t> at(nq + 1, 0);
+    parallel_for(nq, 256, [&](int, int b, int e) {
+      for (int i = b; i < e; ++i) {
+        auto& j = jobs[qs[i]];
+        at[i + 1] = j.k > jb + std::min(nb_, j.k - jb) ? 1 : 0;
+        for (auto& x : j.extra) at[i + 1] += x.cols > 0;
+      }
+    });
+    for (int i = 0; i < nq; ++i) at[i + 1] += at[i];
+    const size_t nd = at[nq];
+    if (nd == 0) return 0;
+    if (ds.size() < nd) ds.resize(nd);
+    std::vector<int>& cnt = tile_bufs().cnt;
+    cnt.resize(nd);
+    std::vector<double> fl(plan_chunks(nq, 64) + 1, 0.0), by(plan_chunks(nq, 64) + 1, 0.0);
+    parallel_for(nq, 64, [&](int ch, int b, int e) {
+      std::vector<LarfbTarget<U>> tg;
+      for (int i = b; i < e; ++i) {
+        auto& j = jobs[qs[i]];
+        targets(qs[i], tg);
+        const int w = std::min(nb_, std::min(j.m, j.k) - jb), rows = j.m - jb;
+        size_t o = at[i];
+        for (auto& t : tg) {
+          ds[o] = LarfbDesc<U>{j.P + jb + (int64_t)jb * j.ld, j.Tb + (int64_t)jb * nb_, t.C, j.ld, t.ld, rows, t.cols, w, 0};
+          cnt[o++] = larfb_tiles(t.cols);
+          fl[ch] += 4.0 * rows * t.cols * w;
+          by[ch] += sizeof(U) * (2.0 * rows * t.cols + (double)rows * w);
+        }
+      }
+    });
+    double flops = 0, bytes = 0;
+    for (double v : fl) flops += v;
+    for (double v : by) bytes += v;
+    std::vector<int>& st = tile_bufs().st;
+    const int nt = prefix_tiles(cnt, st);
+    const LarfbDesc<U>* dd = (const LarfbDesc<U>*)stager_.push_raw(ds.data(), sizeof(LarfbDesc<U>) * nd);
+    const int* dst = stager_.push(st);
+    run.push_back([this, flops, bytes, dd, dst, nd, nt, f] {
+      timed("larfb", flops, bytes, [&] { launch_larfb<U>(stream_, dd, dst, (int)nd, nt, f); });
+    });
+    return nd;
+  }
+
+  // The same step as GEMMs, C -= (V_b T_b^T)(V_b^T C), for panels of more rows
+  // than k_larfb holds.  W = V_b T_b^T is formed once per problem in the same
+  // launch as the Y = V_b^T C of its targets (W and Y live in ws_, rewound per
+  // step); T_b's strict lower part is stored as zeros, so it enters as a dense
+  // factor.
+  template <typename U, typename Targets>
+  void larfb_gemms(std::vector<QrJobT<U>>& jobs, const std::vector<int>& qs, int jb, Targets&& targets, Run& run) {
+    std::vector<GemmDesc<U>> g1, g3;
+    std::vector<LarfbTarget<U>> tg;
+    auto alloc = [&](int64_t elems) { return (U*)ws_.alloc(sizeof(U) * (size_t)std::max<int64_t>(elems, 1)); };
+    for (int q : qs) {
+      auto& j = jobs[q];
+      targets(q, tg);
+      const int w = std::min(nb_, std::min(j.m, j.k) - jb);
+      larfb_step_descs<U>(j.P + jb + (int64_t)jb * j.ld, j.ld, j.Tb + (int64_t)jb * nb_, nb_, j.m - jb, w, tg.data(),
+                          (int)tg.size(), alloc, g1, g3);
+    }
+    const GemmLaunch<U> l1 = gemm_plan(g1.data(), g1.size(), "gemm_y");
+    const GemmLaunch<U> l3 = gemm_plan(g3.data(), g3.size(), "gemm_c");
+    run.push_back([this, l1, l3] {
+      gemm_launch(l1);
+      gemm_launch(l3);
+    });
   }
 
   // tables of the larfb block steps and gemm_batch's tile counts, kept per
@@ -710,8 +750,7 @@ class Engine final : public EngineBase {
   // filling it.  The memory is held until the thread ends.
   template <typename U>
   struct LarfbBufs {
-    std::vector<GemmDesc<U>> g1, g3;
-    std::vector<LarfbTarget<U>> tg;
+    std::vector<LarfbDesc<U>> ds;
   };
   template <typename U>
   static LarfbBufs<U>& larfb_bufs() {

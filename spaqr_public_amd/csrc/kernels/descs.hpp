@@ -107,6 +107,16 @@ void larfb_step_descs(const U* Vb, int ldv, const U* Tb, int ldt, int rows, int 
   }
 }
 
+// The same step on one target as k_larfb takes it (larfb.hip): rows x cols, up to
+// the rows of its largest form
+template <typename T>
+struct LarfbDesc {
+  const T* V;
+  const T* Tb;  // ld 32
+  T* C;
+  int ldv, ldc, rows, cols, w, pad_;
+};
+
 // Householder panel block: factor columns [jb, jb+w) of P (m x k, ld), writing
 // reflectors below the diagonal, R on/above it, tau[j] and the nb x nb block
 // T factor of this block into Tb + jb*nb (ld nb).  Rows [jb, m) beyond one

@@ -117,6 +117,13 @@ void launch_gather_in(hipStream_t s, const int64_t* dst, const int* src, int n, 
 template <typename T>
 void launch_scatter_out(hipStream_t s, const int64_t* src, const int* dst, int n, const T* xbuf, double* x);
 
+// larfb.hip: forms 0 .. larfb_forms() - 1 take up to larfb_form_rows rows
+int larfb_forms();
+int larfb_form_rows(int form);
+int larfb_tiles(int cols);
+template <typename T>
+void launch_larfb(hipStream_t s, const LarfbDesc<T>* d, const int* tstart, int nd, int ntiles, int form);
+
 // flow.hip: the dataflow apply on `grid` workgroups (flow_capacity at most)
 template <typename T>
 int flow_capacity();

@@ -277,6 +277,23 @@ int rrqr_one(int k, int N, X* Ct, X* V, X* tau, double tol, int nd, int* perm, i
 }
 }  // namespace
 namespace {
+template <typename T>
+int larfb_one(int form, int rows, int cols, int nt, int w, const T* V, int ldv, const T* Tb, T* Cm, int ldc) {
+  if (form < 0 || form >= larfb_forms() || rows > larfb_form_rows(form)) { g_err = "rows exceed the form"; return -1; }
+  T *dV = dup(V, (size_t)ldv * w), *dT = dup(Tb, 32 * 32), *dC = dup(Cm, (size_t)ldc * cols * nt);
+  std::vector<LarfbDesc<T>> ds;
+  std::vector<int> st{0};
+  for (int t = 0; t < nt; ++t) {
+    ds.push_back(LarfbDesc<T>{dV, dT, dC + (size_t)ldc * cols * t, ldv, ldc, rows, cols, w, 0});
+    st.push_back(st.back() + larfb_tiles(cols));
+  }
+  launch_larfb<T>(0, dup(ds.data(), ds.size()), dup(st.data(), st.size()), nt, st.back(), form);
+  KT(hipDeviceSynchronize());
+  back(Cm, dC, (size_t)ldc * cols * nt);
+  return 0;
+}
+}  // namespace
+namespace {
 // One dataflow op (kernels/flow.hip) on x (m values) and, for the triangular
 // and the pull form, xn (n values) with the block Bn: the inputs lie in two
 // segments in reverse order, the blocks' tiles start with a short one.
@@ -352,6 +369,17 @@ int ktest_flow(int type, int m, int k, int par, int unit, const double* A, int l
                const double* x, const double* xn, double* out) {
   return flow_one<double>(type, m, k, par, unit, A, lda, B, ldb, n, x, xn, out);
 }
+// One k_larfb step of `form` on nt targets of cols columns each (C: ldc x nt
+// cols, target t at its column t cols)
+int ktest_larfb(int form, int rows, int cols, int nt, int w, const double* V, int ldv, const double* Tb, double* Cm,
+                int ldc) {
+  return larfb_one<double>(form, rows, cols, nt, w, V, ldv, Tb, Cm, ldc);
+}
+int ktest_larfb_f32(int form, int rows, int cols, int nt, int w, const float* V, int ldv, const float* Tb, float* Cm,
+                    int ldc) {
+  return larfb_one<float>(form, rows, cols, nt, w, V, ldv, Tb, Cm, ldc);
+}
+int ktest_larfb_rows(int form) { return form < larfb_forms() ? larfb_form_rows(form) : 0; }
 int ktest_flow_f32(int type, int m, int k, int par, int unit, const float* A, int lda, const float* B, int ldb, int n,
                    const double* x, const double* xn, double* out) {
   return flow_one<float>(type, m, k, par, unit, A, lda, B, ldb, n, x, xn, out);
