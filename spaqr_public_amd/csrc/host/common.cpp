@@ -28,14 +28,12 @@ void* Arena::alloc(size_t bytes, size_t align) {
     ++cur_;
   }
   size_t sz = bytes > chunk_ ? (bytes + align) : chunk_;
-  void* p = nullptr;
   const double t0 = wall();
-  hipError_t e = dev_malloc(&p, sz);
+  if (chunks_.empty()) SPQ_HIP(hipGetDevice(&dev_));
+  char* p = pool_take(false, sz);
   t_chunks += wall() - t0;
   ++n_chunks;
-  if (e != hipSuccess)
-    throw Error(kErrOom, "device allocation of " + std::to_string(sz) + " bytes failed: " + hipGetErrorString(e));
-  chunks_.push_back({(char*)p, sz, 0});
+  chunks_.push_back({p, sz, 0});
   reserved_ += sz;
   cur_ = chunks_.size() - 1;
   Chunk& c = chunks_.back();
@@ -51,7 +49,7 @@ void Arena::rewind() {
 }
 
 void Arena::release() {
-  for (auto& c : chunks_) dev_free(c.p);
+  for (auto& c : chunks_) pool_give(false, c.p, c.size, dev_);
   chunks_.clear();
   cur_ = 0;
   used_ = 0;
@@ -60,7 +58,10 @@ void Arena::release() {
 
 namespace {
 struct PoolEntry { int dev; bool host; size_t bytes; char* p; };
-constexpr size_t kPoolBytes = size_t(2) << 30;
+// kept per device: pinned host memory, and device memory (the arenas of a
+// tree of a million unknowns; 3% of the device's)
+constexpr size_t kPoolBytes[2] = {size_t(8) << 30, size_t(2) << 30};
+constexpr size_t kPoolStreams = 16;
 std::mutex& pool_mu() {
   static std::mutex m;
   return m;
@@ -82,6 +83,7 @@ char* pool_take(bool host, size_t& bytes, bool largest) {
     int best = -1;
     for (size_t i = 0; i < v.size(); ++i)
       if (v[i].dev == dev && v[i].host == host && v[i].bytes >= bytes &&
+          (largest || v[i].bytes <= 2 * bytes + (size_t(1) << 20)) &&  // no large chunk for a small request
           (best < 0 || (largest ? v[i].bytes > v[best].bytes : v[i].bytes < v[best].bytes)))
         best = (int)i;
     if (best >= 0) {
@@ -92,9 +94,81 @@ char* pool_take(bool host, size_t& bytes, bool largest) {
     }
   }
   void* p = nullptr;
-  if (host) SPQ_HIP(host_malloc(&p, bytes));
-  else SPQ_HIP(dev_malloc(&p, bytes));
+  if (host) {
+    SPQ_HIP(host_malloc(&p, bytes));
+    return (char*)p;
+  }
+  const hipError_t e = dev_malloc(&p, bytes);
+  if (e != hipSuccess)
+    throw Error(kErrOom, "device allocation of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
   return (char*)p;
+}
+
+// Device memory; when there is none left, what the pool keeps is given back
+// and the allocation tried again.
+hipError_t dev_malloc(void** p, size_t bytes) {
+  std::lock_guard<std::recursive_mutex> lk(capture_lock());
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return e;
+  std::vector<PoolEntry> drop;
+  {
+    std::lock_guard<std::mutex> lk2(pool_mu());
+    auto& v = pool();
+    for (size_t i = 0; i < v.size();)
+      if (v[i].dev == dev && !v[i].host) {
+        drop.push_back(v[i]);
+        v.erase(v.begin() + i);
+      } else {
+        ++i;
+      }
+  }
+  if (drop.empty()) return e;
+  (void)hipGetLastError();
+  for (auto& d : drop) (void)hipFree(d.p);
+  return hipMalloc(p, bytes);
+}
+
+namespace {
+std::vector<std::pair<int, hipStream_t>>& stream_pool() {
+  static auto* v = new std::vector<std::pair<int, hipStream_t>>();
+  return *v;
+}
+}  // namespace
+
+hipStream_t stream_take() {
+  int dev = 0;
+  SPQ_HIP(hipGetDevice(&dev));
+  {
+    std::lock_guard<std::mutex> lk(pool_mu());
+    auto& v = stream_pool();
+    for (size_t i = 0; i < v.size(); ++i)
+      if (v[i].first == dev) {
+        const hipStream_t s = v[i].second;
+        v.erase(v.begin() + i);
+        return s;
+      }
+  }
+  hipStream_t s = nullptr;
+  SPQ_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+  return s;
+}
+
+void stream_give(hipStream_t s, int dev) {
+  if (!s) return;
+  {
+    std::lock_guard<std::mutex> lk(pool_mu());
+    auto& v = stream_pool();
+    size_t n = 0;
+    for (auto& e : v) n += e.first == dev;
+    if (n < kPoolStreams) {
+      v.push_back({dev, s});
+      return;
+    }
+  }
+  std::lock_guard<std::recursive_mutex> lk(capture_lock());
+  (void)hipStreamDestroy(s);
 }
 
 void pool_give(bool host, char* p, size_t bytes, int dev) {
@@ -113,7 +187,7 @@ void pool_give(bool host, char* p, size_t bytes, int dev) {
         tot += v[i].bytes;
         if (small < 0 || v[i].bytes < v[small].bytes) small = (int)i;
       }
-      if (tot <= kPoolBytes || small < 0) break;
+      if (tot <= kPoolBytes[host] || small < 0) break;
       drop.push_back(v[small]);
       v.erase(v.begin() + small);
     }

@@ -41,10 +41,7 @@ inline void host_free(void* p) {
   std::lock_guard<std::recursive_mutex> lk(capture_lock());
   (void)hipHostFree(p);
 }
-inline hipError_t dev_malloc(void** p, size_t bytes) {
-  std::lock_guard<std::recursive_mutex> lk(capture_lock());
-  return hipMalloc(p, bytes);
-}
+hipError_t dev_malloc(void** p, size_t bytes);
 inline hipError_t host_malloc(void** p, size_t bytes) {
   std::lock_guard<std::recursive_mutex> lk(capture_lock());
   return hipHostMalloc(p, bytes, hipHostMallocDefault);
@@ -102,7 +99,7 @@ class Arena {
   Arena& operator=(const Arena&) = delete;
   void* alloc(size_t bytes, size_t align = 256);
   void rewind();  // keep chunks, reset offsets
-  void release();
+  void release();  // chunks go back to the pool: the stream work on them is complete
   size_t used() const { return used_; }
   // chunk allocations of all arenas: count and host seconds (diagnostics)
   static long n_chunks;
@@ -114,17 +111,26 @@ class Arena {
   size_t chunk_;
   std::vector<Chunk> chunks_;
   size_t cur_ = 0, used_ = 0, reserved_ = 0;
+  int dev_ = 0;
 };
 
-// Process-wide pool of staging buffers (pinned host or device memory of the
+// Process-wide pool of buffers (pinned host or device memory of the
 // current device), so trees created one after another reuse them instead of
 // allocating and pinning again.  pool_take returns a buffer of at least
 // `bytes` (the smallest pooled one that fits, or the largest with `largest`,
 // else a new one) and sets `bytes` to its size; pool_give returns it to the pool of device `dev` (the device
 // current when it was taken; the caller's stream work on it must be
-// complete).  At most 2 GiB per kind and device stay pooled.
+// complete).  At most 8 GiB of device and 2 GiB of pinned memory per device stay
+// pooled, and none of it once an allocation finds no memory left.  A tree of a
+// small problem spent a fifth of its life in hipMalloc and hipFree (2-D 40^2:
+// 1.0 of 4.7 ms), and after some hundred trees in a process the driver made
+// single allocations wait for 20 ms to seconds.
 char* pool_take(bool host, size_t& bytes, bool largest = false);
 void pool_give(bool host, char* p, size_t bytes, int dev);
+// The same for streams (default priority, non-blocking, idle when given back;
+// at most 16 per device are kept).
+hipStream_t stream_take();
+void stream_give(hipStream_t s, int dev);
 
 // Pinned host staging + device ring for descriptor tables.  push() copies a
 // table into the pinned ring, enqueues the H2D copy on the stream and returns

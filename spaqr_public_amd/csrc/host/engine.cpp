@@ -41,14 +41,15 @@ class Engine final : public EngineBase {
   Engine(int nlevels, int skip, int device) : nlevels_(nlevels), skip_(skip), perm_(size_t(512) << 20),
                                                scratch_(size_t(256) << 20), ws_(size_t(64) << 20) {
     SPQ_HIP(hipSetDevice(device));
-    SPQ_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+    device_ = device;
+    stream_ = stream_take();
     stager_.init(stream_, size_t(64) << 20);
     bottoms_.resize(nlevels);
     info_.resize(nlevels);
     nb_ = panel_nb();
     for (auto& row : qp3r_cap_)
       for (int& c : row) c = -1;
-    SPQ_HIP(host_malloc((void**)&rank_host_, sizeof(int) * 65536));
+    rank_host_ = (int*)pool_take(true, rank_bytes_);
     qp3_err_ = (int*)perm_.alloc(256);
     SPQ_HIP(hipMemset(qp3_err_, 0, 256));
     if (const char* e = std::getenv("SPAQR_QP3_MAX_WG")) qp3_max_wg_ = std::max(1, std::atoi(e));
@@ -80,11 +81,11 @@ class Engine final : public EngineBase {
     if (graph_exec_t_) hipGraphExecDestroy(graph_exec_t_);
     dev_free(xtbuf_);
     dev_free(x64_);
-    host_free(rank_host_);
+    pool_give(true, (char*)rank_host_, rank_bytes_, device_);
     dev_free(xbuf_);
     dev_free(bin_);
     dev_free(xout_);
-    hipStreamDestroy(stream_);
+    stream_give(stream_, device_);
   }
 
   void set_tol(double t) override { tol_ = t; }
@@ -900,6 +901,8 @@ class Engine final : public EngineBase {
   int qp3_max_wg_ = 64;
   Stager stager_;
   int* rank_host_ = nullptr;
+  size_t rank_bytes_ = sizeof(int) * 65536;
+  int device_ = 0;
   bool partitioned_ = false, assembled_ = false, factored_ = false;
   bool factorizing_ = false;  // set for good once factorize starts (a failed run leaves the tree unusable)
   bool kprof_ = false;

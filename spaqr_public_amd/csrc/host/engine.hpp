@@ -96,7 +96,7 @@ class EngineBase {
   virtual void reset_kernel_stats() = 0;
 
  private:
-  struct Work { double* p = nullptr; size_t cap = 0; };
+  struct Work { double* p = nullptr; size_t cap = 0, bytes = 0; int dev = 0; };
   std::vector<Work> work_dev_, work_host_;
 };
 

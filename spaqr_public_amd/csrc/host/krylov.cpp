@@ -10,8 +10,9 @@
 namespace spq {
 
 EngineBase::~EngineBase() {
-  for (auto& w : work_dev_) dev_free(w.p);
-  for (auto& w : work_host_) host_free(w.p);
+  // the engine's own destructor has waited for its stream
+  for (auto& w : work_dev_) pool_give(false, (char*)w.p, w.bytes, w.dev);
+  for (auto& w : work_host_) pool_give(true, (char*)w.p, w.bytes, w.dev);
 }
 
 double* EngineBase::work_dev(int slot, size_t elems) {
@@ -19,11 +20,14 @@ double* EngineBase::work_dev(int slot, size_t elems) {
   Work& w = work_dev_[slot];
   elems = std::max<size_t>(elems, 1);
   if (w.cap < elems) {
-    dev_free(w.p);
+    SPQ_HIP(hipStreamSynchronize(stream()));  // the pool hands it to other streams
+    pool_give(false, (char*)w.p, w.bytes, w.dev);
     w.p = nullptr;
     w.cap = 0;
-    SPQ_HIP(dev_malloc((void**)&w.p, sizeof(double) * elems));
-    w.cap = elems;
+    w.bytes = sizeof(double) * elems;
+    SPQ_HIP(hipGetDevice(&w.dev));
+    w.p = (double*)pool_take(false, w.bytes);
+    w.cap = w.bytes / sizeof(double);
   }
   return w.p;
 }
@@ -33,38 +37,47 @@ double* EngineBase::work_host(int slot, size_t elems) {
   Work& w = work_host_[slot];
   elems = std::max<size_t>(elems, 1);
   if (w.cap < elems) {
-    host_free(w.p);
+    SPQ_HIP(hipStreamSynchronize(stream()));
+    pool_give(true, (char*)w.p, w.bytes, w.dev);
     w.p = nullptr;
     w.cap = 0;
-    SPQ_HIP(host_malloc((void**)&w.p, sizeof(double) * elems));
-    w.cap = elems;
+    w.bytes = sizeof(double) * elems;
+    SPQ_HIP(hipGetDevice(&w.dev));
+    w.p = (double*)pool_take(true, w.bytes);
+    w.cap = w.bytes / sizeof(double);
   }
   return w.p;
 }
 
 DevMatrix::~DevMatrix() {
-  for (void* p : {(void*)rp, (void*)ci, (void*)v, (void*)rpt, (void*)cit, (void*)vt}) dev_free(p);
+  dev_free(mem);
 }
-
-namespace {
-void up(void** d, const void* h, size_t bytes) {
-  SPQ_HIP(dev_malloc(d, bytes > 0 ? bytes : 8));
-  if (bytes) SPQ_HIP(hipMemcpy(*d, h, bytes, hipMemcpyHostToDevice));
-}
-}  // namespace
 
 DevMatrix* upload_matrix(const CscMat& A, bool with_transpose) {
   DevMatrix* M = new DevMatrix;
   M->m = A.m; M->n = A.n; M->nnz = A.nnz();
   // CSR of A == CSC of A^T
   CscMat At = csc_transpose(A);
-  up((void**)&M->rp, At.p.data(), sizeof(int) * At.p.size());
-  up((void**)&M->ci, At.i.data(), sizeof(int) * At.i.size());
-  up((void**)&M->v, At.x.data(), sizeof(double) * At.x.size());
+  // one allocation for all arrays
+  struct Part { void** d; const void* h; size_t bytes, off; };
+  std::vector<Part> parts;
+  size_t total = 0;
+  auto add = [&](void** d, const void* h, size_t bytes) {
+    parts.push_back({d, h, bytes, total});
+    total += (std::max<size_t>(bytes, 8) + 255) / 256 * 256;
+  };
+  add((void**)&M->rp, At.p.data(), sizeof(int) * At.p.size());
+  add((void**)&M->ci, At.i.data(), sizeof(int) * At.i.size());
+  add((void**)&M->v, At.x.data(), sizeof(double) * At.x.size());
   if (with_transpose) {
-    up((void**)&M->rpt, A.p.data(), sizeof(int) * A.p.size());
-    up((void**)&M->cit, A.i.data(), sizeof(int) * A.i.size());
-    up((void**)&M->vt, A.x.data(), sizeof(double) * A.x.size());
+    add((void**)&M->rpt, A.p.data(), sizeof(int) * A.p.size());
+    add((void**)&M->cit, A.i.data(), sizeof(int) * A.i.size());
+    add((void**)&M->vt, A.x.data(), sizeof(double) * A.x.size());
+  }
+  SPQ_HIP(dev_malloc(&M->mem, total));
+  for (auto& q : parts) {
+    *q.d = (char*)M->mem + q.off;
+    if (q.bytes) SPQ_HIP(hipMemcpy(*q.d, q.h, q.bytes, hipMemcpyHostToDevice));
   }
   return M;
 }

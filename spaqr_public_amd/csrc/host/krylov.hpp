@@ -11,6 +11,7 @@ struct DevMatrix {
   double* v = nullptr;
   int *rpt = nullptr, *cit = nullptr;  // CSR of A^T
   double* vt = nullptr;
+  void* mem = nullptr;  // holds them all
   ~DevMatrix();
 };
 DevMatrix* upload_matrix(const CscMat& A, bool with_transpose);
