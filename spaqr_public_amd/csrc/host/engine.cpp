@@ -828,9 +828,10 @@ class Engine final : public EngineBase {
     std::vector<FlowItem> items;
     bool chain = false;  // items sharing rows, in tape order (else independent)
     // changes of the clusters' rows after the items: splits and merges undone
-    // (down) or made (up)
+    // (down) or made (up), then (least squares) what `moves` do
     std::vector<const Op*> split, merge;
     bool up = false;
+    std::vector<std::function<void()>> moves;
   };
   template <typename U>
   struct FlowProg {
@@ -839,14 +840,53 @@ class Engine final : public EngineBase {
     unsigned int* zero = nullptr;  // exchange slots and tickets, cleared before each apply
     int64_t nzero = 0;             // words
   };
-  // places of x holding the rows of each cluster, as segments
+  // places of x holding the rows of each cluster, as segments (least squares:
+  // zeros, off -1, where nothing was written)
+  using FlowList = std::vector<FlowSeg>;
   struct FlowRows {
-    std::vector<std::vector<FlowSeg>> of;
+    std::vector<FlowList> of;
     std::vector<int> scratch;
-    int next = 0;  // places given out so far
+    int next = 0;   // places given out so far
+    int zero = -1;  // least squares: first of kFlowZeros places holding zeros
   };
+  static constexpr int kFlowZeros = 1024;
+  static void flow_add(FlowList& v, size_t from, FlowSeg sg) {
+    if (sg.len <= 0) return;
+    if (v.size() > from && (sg.off < 0 ? v.back().off < 0 : v.back().off >= 0 && v.back().off + v.back().len == sg.off))
+      v.back().len += sg.len;
+    else
+      v.push_back(sg);
+  }
+  // rows [a, a + n), zeros past the end
+  static FlowList flow_slice(const FlowList& v, int a, int n) {
+    FlowList r;
+    for (const FlowSeg& sg : v) {
+      if (n <= 0) break;
+      const int skip = std::min(a, sg.len), len = std::min(sg.len - skip, n);
+      a -= skip;
+      flow_add(r, 0, FlowSeg{sg.off < 0 ? -1 : sg.off + skip, len});
+      n -= len;
+    }
+    flow_add(r, 0, FlowSeg{-1, n});
+    return r;
+  }
+  static int flow_len(const FlowList& v) {
+    int n = 0;
+    for (const FlowSeg& sg : v) n += sg.len;
+    return n;
+  }
+  // rows from a on replaced by r
+  static void flow_splice(FlowList& v, int a, const FlowList& r) {
+    const int n = flow_len(r), m = flow_len(v);
+    FlowList o = flow_slice(v, 0, a);
+    for (const FlowSeg& sg : r) flow_add(o, 0, sg);
+    if (m > a + n)
+      for (const FlowSeg& sg : flow_slice(v, a + n, m - a - n)) flow_add(o, 0, sg);
+    v = std::move(o);
+  }
   bool flow_fits() const;
   bool build_flow();
+  bool build_flow_ls(const std::vector<std::vector<const Op*>>& by_level);
   template <typename U>
   void build_w(const std::vector<WyJob<U>>& jobs);
   template <typename U>
@@ -2856,22 +2896,23 @@ int Engine<T>::factorize() {  // tree.cpp:1309-1437
 // ---------------------------------------------------------------------------
 // The square apply as a dataflow program.
 
-// Square trees without fine-cluster eliminations, in the sizes k_flow takes.
-// The others, and applies timed stage by stage, run the staged program.
+// Trees without fine-cluster eliminations, in the sizes k_flow takes; least
+// squares in one precision.  The others, and applies timed stage by stage, run
+// the staged program.
 template <typename T>
 bool Engine<T>::flow_fits() const {
-  if (!square_ || !reflr_ || stage_prof_) return false;
+  if (!reflr_ || stage_prof_) return false;
   auto too_long = [](int64_t ld, int64_t cols) { return ld * cols * 8 > int64_t(0xffffffffu); };  // 32-bit offsets
   for (auto& o : ops_) {
-    if (o.kind == OpFineQR || o.kind == OpReassign) return false;
-    if (o.kind == OpSplitD && o.crows != o.ccols) return false;
+    if (o.kind == OpFineQR || (!square_ && o.V64)) return false;
+    if (square_ && (o.kind == OpReassign || (o.kind == OpSplitD && o.crows != o.ccols))) return false;
     if (o.kind != OpQR && o.kind != OpScaleD && o.kind != OpOrthoD) continue;
     if (o.k > kFlowMaxK || o.kr > kFlowMaxK) return false;
     if (o.m > kFlowMaxParts * kFlowMaxK || too_long(std::max(o.ldv, o.m), o.k) || too_long(o.ldr, std::max(o.kr, o.k)))
       return false;
   }
   for (int c : bottoms_[0])
-    if (cl_[c].rsize_org != cl_[c].csize_org) return false;
+    if (square_ && cl_[c].rsize_org != cl_[c].csize_org) return false;
   return flow_capacity<T>() >= 2 * kFlowMaxParts && flow_capacity<double>() >= 2 * kFlowMaxParts;
 }
 
@@ -2933,21 +2974,30 @@ bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, Flo
   std::vector<size_t> slot_at;  // by part
   std::vector<int>& wave = R.scratch;  // of a chain: waves so far on a cluster
   const int cap = std::min(flow_capacity<U>(), 2 * num_cus_);
-  auto add_seg = [](std::vector<FlowSeg>& v, size_t from, FlowSeg sg) {
-    if (sg.len <= 0) return;
-    if (v.size() > from && v.back().off + v.back().len == sg.off) v.back().len += sg.len;
-    else v.push_back(sg);
-  };
+  auto add_seg = [](FlowList& v, size_t from, FlowSeg sg) { flow_add(v, from, sg); };
   // the first n rows of a cluster
-  auto rows_of = [&](int c, int n, std::vector<FlowSeg>& v, size_t from) {
+  auto rows_of = [&](int c, int n, FlowList& v, size_t from) {
+    if (R.zero >= 0) {
+      for (const FlowSeg& sg : flow_slice(R.of[c], 0, n)) {
+        if (sg.off >= 0) flow_add(v, from, sg);
+        else
+          for (int t = 0; t < sg.len; t += kFlowZeros) v.push_back(FlowSeg{R.zero, std::min(kFlowZeros, sg.len - t)});
+      }
+      return;
+    }
     for (const FlowSeg& sg : R.of[c]) {
       if (n <= 0) break;
-      add_seg(v, from, FlowSeg{sg.off, std::min(sg.len, n)});
+      flow_add(v, from, FlowSeg{sg.off, std::min(sg.len, n)});
       n -= sg.len;
     }
     if (n > 0) throw Error(kErrState, "solve program: rows of a cluster are missing");
   };
+  // (least squares: the rows past the first n stay)
   auto set_rows = [&](int c, int off, int n) {
+    if (R.zero >= 0) {
+      flow_splice(R.of[c], 0, FlowList{FlowSeg{off, n}});
+      return;
+    }
     R.of[c].clear();
     if (n > 0) R.of[c].push_back(FlowSeg{off, n});
   };
@@ -3021,7 +3071,9 @@ bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, Flo
           if (it.type == kFlowBack) {
             // tiles of up to 32 columns, cut where x_n's segments end
             int j = 0;
-            for (const FlowSeg& sg : R.of[n])
+            FlowList at;
+            rows_of(n, sn, at, 0);
+            for (const FlowSeg& sg : at)
               for (int t = 0; t < sg.len && j < sn; t += 32) {
                 const int nn = std::min({32, sg.len - t, sn - j});
                 blks.push_back(FlowBlk<U>{(const U*)q.first.p + (int64_t)j * q.first.ld, q.first.ld, nn, sg.off + t, 0});
@@ -3105,6 +3157,7 @@ bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, Flo
       for (const Op* o : st.split)
         for (const FlowSeg& sg : R.of[o->f]) add_seg(R.of[o->c], 0, sg);
     }
+    for (auto& f : st.moves) f();
   }
   if (!fits) return false;
   const size_t slot_words = slots * sizeof(U) / 4;
@@ -3144,7 +3197,8 @@ bool Engine<T>::build_flow() {
   std::vector<WyJob<T>> wj;
   std::vector<WyJob<double>> wj64;
   for (auto& o : ops_) {
-    if (o.kind == OpSplitD || o.kind == OpMerge || o.k <= 0) continue;
+    if (o.kind != OpOrthoD && !(square_ && (o.kind == OpQR || o.kind == OpScaleD))) continue;
+    if (o.k <= 0) continue;
     if (o.V64) {
       double* W = (double*)perm_.alloc(sizeof(double) * (size_t)o.m * o.k);
       o.W = W;
@@ -3157,9 +3211,10 @@ bool Engine<T>::build_flow() {
   }
   build_w(wj);
   build_w(wj64);
-  // stages of the forward and the backward tape; the FP64 top apart
   std::vector<std::vector<const Op*>> by_level(nlevels_);
   for (auto& o : ops_) by_level[o.level].push_back(&o);
+  if (!square_) return build_flow_ls(by_level);
+  // stages of the forward and the backward tape; the FP64 top apart
   std::vector<FlowStage> fwd, bwd;
   const Op* top = nullptr;
   for (auto& lv : by_level) {
@@ -3287,6 +3342,132 @@ bool Engine<T>::build_flow() {
     }
   flow_rperm_ = stager_.upload(perm_, rp);
   flow_cperm_ = stager_.upload(perm_, cp);
+  flow_ = true;
+  return true;
+}
+
+// (W^T W)^{-1} of a least-squares tree (tree.cpp:1471-1517): R^{-T} and the
+// interfaces' reflectors up the tree on xt, row permutations down and up again,
+// and the backward tape on x.  Only list entries move in the permutations.
+template <typename T>
+bool Engine<T>::build_flow_ls(const std::vector<std::vector<const Op*>>& by_level) {
+  FlowMode& M = flow_mode_[0];
+  FlowRows R;
+  R.of.resize(cl_.size());
+  R.scratch.assign(cl_.size(), 0);
+  std::vector<int> cp;
+  for (int c : bottoms_[0]) {
+    if (cl_[c].csize_org > 0) R.of[c].push_back(FlowSeg{R.next, cl_[c].csize_org});
+    R.next += cl_[c].csize_org;
+    for (int i = 0; i < cl_[c].csize_org; ++i) cp.push_back(cperm_[cl_[c].cstart + i]);
+  }
+  R.zero = R.next;
+  R.next += kFlowZeros;
+  // SplitD (operations.cpp:120-131): x_f = x[rk:cc), x[rk:rk+rest) = x[cc:cr)
+  auto split_up = [&](const Op* o) {
+    FlowList& v = R.of[o->c];
+    const int rest = o->crows - o->ccols;
+    const FlowList fine = flow_slice(v, o->rank, o->ccols - o->rank), tail = flow_slice(v, o->ccols, rest);
+    flow_splice(R.of[o->f], 0, fine);
+    flow_splice(v, o->rank, tail);
+  };
+  auto split_down = [&](const Op* o) {
+    FlowList& v = R.of[o->c];
+    const int rest = o->crows - o->ccols;
+    const FlowList tail = flow_slice(v, o->rank, rest);
+    flow_splice(v, o->ccols, tail);
+    flow_splice(v, o->rank, flow_slice(R.of[o->f], 0, o->ccols - o->rank));
+  };
+  auto merge = [&](const Op* o, bool up, bool rows) {
+    int k = 0;
+    for (int ch : cl_[o->c].children) {
+      const int len = rows ? cl_[ch].rsize : cl_[ch].csize;
+      if (up) flow_splice(R.of[o->c], k, flow_slice(R.of[ch], 0, len));
+      else flow_splice(R.of[ch], 0, flow_slice(R.of[o->c], k, len));
+      k += len;
+    }
+  };
+  // Reassign: x_f[nstart + t] = x_c[idx[t]] (up) and back
+  auto reassign = [&](const Op* o, bool up) {
+    for (size_t t = 0; t < o->idx.size(); ++t) {
+      const int f = o->nstart + (int)t;
+      if (up) flow_splice(R.of[o->f], f, flow_slice(R.of[o->c], o->idx[t], 1));
+      else flow_splice(R.of[o->c], o->idx[t], flow_slice(R.of[o->f], f, 1));
+    }
+  };
+  std::vector<FlowStage> st;
+  for (auto& lv : by_level) {
+    FlowStage qr, sc, od;
+    for (auto o : lv) {
+      if (o->kind == OpQR && o->kr > 0) qr.items.push_back(FlowItem{o, kFlowSolveT, true});
+      else if (o->kind == OpScaleD && o->k > 0) sc.items.push_back(FlowItem{o, kFlowSolveT, true});
+      else if (o->kind == OpOrthoD && o->k > 0) od.items.push_back(FlowItem{o, kFlowWY, false});
+    }
+    od.moves.push_back([&, split_up, merge] {
+      for (auto o : lv)
+        if (o->kind == OpSplitD) split_up(o);
+      for (auto o : lv)
+        if (o->kind == OpMerge) merge(o, true, false);
+    });
+    st.push_back(std::move(qr));
+    st.push_back(std::move(sc));
+    st.push_back(std::move(od));
+  }
+  FlowStage perm;
+  perm.moves.push_back([&, split_up, split_down, merge, reassign] {
+    for (int l = nlevels_ - 1; l >= 0; --l) {
+      for (auto o : by_level[l])
+        if (o->kind == OpMerge) merge(o, false, true);
+      for (auto o : by_level[l])
+        if (o->kind == OpSplitD) split_down(o);
+      for (auto o : by_level[l])
+        if (o->kind == OpReassign) reassign(o, false);
+    }
+    // xt -> x at the leaves
+    std::vector<FlowList> x(cl_.size());
+    for (int c : bottoms_[0]) x[c] = flow_slice(R.of[c], 0, cl_[c].rsize_org);
+    R.of = std::move(x);
+    for (auto& lv : by_level) {
+      for (auto o : lv)
+        if (o->kind == OpReassign) reassign(o, true);
+      for (auto o : lv)
+        if (o->kind == OpSplitD) split_up(o);
+      for (auto o : lv)
+        if (o->kind == OpMerge) merge(o, true, true);
+    }
+  });
+  st.push_back(std::move(perm));
+  for (int l = nlevels_ - 1; l >= 0; --l) {
+    const auto& lv = by_level[l];
+    FlowStage dn, qr, sc, od;
+    dn.moves.push_back([&, split_down, merge] {
+      for (auto o : lv)
+        if (o->kind == OpMerge) merge(o, false, false);
+      for (auto o : lv)
+        if (o->kind == OpSplitD) split_down(o);
+    });
+    for (auto o : lv) {
+      if (o->kind == OpOrthoD && o->k > 0) od.items.push_back(FlowItem{o, kFlowWY, true});
+      else if (o->kind == OpScaleD && o->k > 0) sc.items.push_back(FlowItem{o, kFlowBack, false});
+      else if (o->kind == OpQR && o->kr > 0) qr.items.push_back(FlowItem{o, kFlowBack, false});
+    }
+    st.push_back(std::move(dn));
+    st.push_back(std::move(od));
+    st.push_back(std::move(sc));
+    st.push_back(std::move(qr));
+  }
+  M.run.resize(1);
+  if (!flow_prog<T>(st, R, M.run[0])) return false;
+  M.xplaces = R.next;
+  std::vector<int> out;
+  for (int c : bottoms_[0])
+    for (const FlowSeg& sg : flow_slice(R.of[c], 0, cl_[c].csize_org))
+      for (int i = 0; i < sg.len; ++i) out.push_back(sg.off < 0 ? R.zero : sg.off + i);
+  M.out = stager_.upload(perm_, out);
+  flow_cperm_ = flow_rperm_ = stager_.upload(perm_, cp);
+  xsize_ = M.xplaces;
+  flow_x_ = alloc_perm((size_t)xsize_);
+  M.run[0].args.x = flow_x_;
   flow_ = true;
   return true;
 }
@@ -3893,12 +4074,13 @@ void Engine<T>::build_solve_program() {
 template <typename T>
 void Engine<T>::run_flow(const double* b, double* x, bool transposed) {
   const FlowMode& M = flow_mode_[transposed];
+  const int nz = square_ ? 0 : kFlowZeros;  // least squares: places of zeros after b's
   FlowClear c{};
   auto clear = [&, i = 0](void* p, int64_t words) mutable {
     c.p[i] = (unsigned int*)p;
     c.n[i++] = words;
   };
-  clear(flow_x_ + nrows_, (int64_t)(M.xplaces - nrows_) * (int64_t)(sizeof(T) / 4));
+  clear(flow_x_ + ncols_ + nz, (int64_t)(M.xplaces - ncols_ - nz) * (int64_t)(sizeof(T) / 4));
   for (auto& r : M.run) clear(r.zero, r.nzero);
   const bool top = M.run.size() > 1;
   if (top) {
@@ -3906,7 +4088,7 @@ void Engine<T>::run_flow(const double* b, double* x, bool transposed) {
     clear(M.top.zero, M.top.nzero);
   }
   // M^{-T}: b enters through the exit map and leaves through the entry map
-  launch_flow_begin<T>(stream_, transposed ? flow_cperm_ : flow_rperm_, nrows_, b, flow_x_, c);
+  launch_flow_begin<T>(stream_, transposed ? flow_cperm_ : flow_rperm_, ncols_, b, flow_x_, nz, c);
   launch_flow<T>(stream_, M.run[0].args, M.run[0].grid);
   if (top) {
     launch_flow_cvt<T, double>(stream_, M.top_in, flow_top_n_, flow_x_, flow_x64_, 0);
@@ -3914,7 +4096,7 @@ void Engine<T>::run_flow(const double* b, double* x, bool transposed) {
     launch_flow_cvt<double, T>(stream_, M.top_out, flow_top_n_, flow_x64_, flow_x_, M.top_at);
     launch_flow<T>(stream_, M.run[1].args, M.run[1].grid);
   }
-  launch_flow_out<T>(stream_, M.out, nrows_, flow_x_, transposed ? flow_rperm_ : flow_cperm_, x);
+  launch_flow_out<T>(stream_, M.out, ncols_, flow_x_, transposed ? flow_rperm_ : flow_cperm_, x);
 }
 
 template <typename T>
@@ -4026,6 +4208,10 @@ template <typename T>
 void Engine<T>::solve_nrml_dev(const double* b, double* x) {
   if (!factored_) throw Error(kErrState, "solve_nrml before factorize");
   if (square_) throw Error(kErrState, "solve_nrml: the tree was factored as a square system (set_square(0) first)");
+  if (flow_) {
+    timed("apply", 0.0, solve_bytes_, [&] { run_flow(b, x, false); });
+    return;
+  }
   SPQ_HIP(hipMemcpyAsync(bin_, b, sizeof(double) * ncols_, hipMemcpyDeviceToDevice, stream_));
   if (stage_prof_ || !solve_graph_) {
     timed("apply", 0.0, solve_bytes_, [&] { run_program(bin_, xout_, stage_prof_, 1); });

@@ -1,4 +1,4 @@
-// The preconditioner apply of a square tree as one dataflow kernel (gfx950).
+// The preconditioner apply of a tree as one dataflow kernel (gfx950).
 //
 // The tape is a chain of 50-250 dependent steps, most of a few small ops (the
 // elimination waves of a level: 1-24 ops of 250-500 rows), so an apply is bound
@@ -592,9 +592,9 @@ template void launch_flow<float>(hipStream_t, const FlowArgs<float>&, int);
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_flow_begin(const int* __restrict__ src, int n, const double* __restrict__ b,
-                                                    T* x, FlowClear c) {
+                                                    T* x, int nz, FlowClear c) {
   const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
-  for (int64_t i = i0; i < n; i += step) slot_put(x, i, true, (T)b[src ? src[i] : i]);
+  for (int64_t i = i0; i < n + nz; i += step) slot_put(x, i, true, i < n ? (T)b[src ? src[i] : i] : T(0));
 #pragma unroll
   for (int q = 0; q < 5; ++q)
     for (int64_t i = i0; i < c.n[q]; i += step) c.p[q][i] = 0;
@@ -623,12 +623,12 @@ __global__ __launch_bounds__(256) void k_flow_cvt(const int* __restrict__ loc, i
   slot_put(y, (int64_t)at + i, true, (D)v);
 }
 template <typename T>
-void launch_flow_begin(hipStream_t s, const int* src, int n, const double* b, T* x, const FlowClear& c) {
-  int64_t most = n;
+void launch_flow_begin(hipStream_t s, const int* src, int n, const double* b, T* x, int nz, const FlowClear& c) {
+  int64_t most = n + nz;
   for (int64_t w : c.n) most = std::max(most, w);
   if (most <= 0) return;
   hipLaunchKernelGGL((k_flow_begin<T>), dim3(std::min<int64_t>((most + 255) / 256, 2048)), dim3(256), 0, s, src, n, b, x,
-                     c);
+                     nz, c);
 }
 template <typename T>
 void launch_flow_out(hipStream_t s, const int* loc, int n, const T* x, const int* dst, double* y) {
@@ -638,8 +638,8 @@ template <typename T, typename D>
 void launch_flow_cvt(hipStream_t s, const int* loc, int n, const T* x, D* y, int at) {
   if (n > 0) hipLaunchKernelGGL((k_flow_cvt<T, D>), dim3((n + 255) / 256), dim3(256), 0, s, loc, n, x, y, at);
 }
-template void launch_flow_begin<double>(hipStream_t, const int*, int, const double*, double*, const FlowClear&);
-template void launch_flow_begin<float>(hipStream_t, const int*, int, const double*, float*, const FlowClear&);
+template void launch_flow_begin<double>(hipStream_t, const int*, int, const double*, double*, int, const FlowClear&);
+template void launch_flow_begin<float>(hipStream_t, const int*, int, const double*, float*, int, const FlowClear&);
 template void launch_flow_out<double>(hipStream_t, const int*, int, const double*, const int*, double*);
 template void launch_flow_out<float>(hipStream_t, const int*, int, const float*, const int*, double*);
 template void launch_flow_cvt<float, double>(hipStream_t, const int*, int, const float*, double*, int);

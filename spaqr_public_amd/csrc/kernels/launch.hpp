@@ -133,11 +133,11 @@ void launch_flow(hipStream_t s, const FlowArgs<T>& a, int grid);
 // entries each); start: exclusive prefix sums of ceil(k / 32)
 template <typename T>
 void launch_flow_diag(hipStream_t s, const FlowDiag<T>* d, const int* start, int nd, int nblocks);
-// the start of an apply: n values of b (through src, or in order) into the first
-// places of x and zeros into what c lists, in one launch; and its end, values out
-// of places loc
+// the start of an apply: n values of b (through src, or in order) and nz zeros
+// into the first places of x, and what c lists cleared, in one launch; and its
+// end, values out of places loc
 template <typename T>
-void launch_flow_begin(hipStream_t s, const int* src, int n, const double* b, T* x, const FlowClear& c);
+void launch_flow_begin(hipStream_t s, const int* src, int n, const double* b, T* x, int nz, const FlowClear& c);
 template <typename T>
 void launch_flow_out(hipStream_t s, const int* loc, int n, const T* x, const int* dst, double* y);
 // places loc of x into places [at, at + n) of y

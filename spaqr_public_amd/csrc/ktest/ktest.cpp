@@ -352,7 +352,7 @@ int flow_one(int type, int m, int k, int par, int unit, const T* A, int lda, con
   a.segs = dup(segs.data(), segs.size());
   a.blks = blks.empty() ? nullptr : dup(blks.data(), blks.size());
   a.x = dx; a.ctl = ctl; a.err = err; a.nparts = np;
-  launch_flow_begin<T>(0, nullptr, m + n, dup(xin.data(), xin.size()), dx, FlowClear{});
+  launch_flow_begin<T>(0, nullptr, m + n, dup(xin.data(), xin.size()), dx, 0, FlowClear{});
   launch_flow<T>(0, a, std::min(np, flow_capacity<T>()));
   std::vector<int> loc(m);
   for (int i = 0; i < m; ++i) loc[i] = d.out + i;

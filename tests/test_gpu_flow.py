@@ -128,3 +128,29 @@ def test_against_staged_program(monkeypatch, n, d, precision, tol):
     for a, c in zip(*got):
         assert np.linalg.norm(a - c) <= 1e4 * eps * np.linalg.norm(a)
     assert np.array_equal(got[1][0], got[1][2])  # no order of arrival in the sums
+
+
+@pytest.mark.parametrize("n,precision,tol", [(16, 8, 1e-2), (24, 8, 0.0), (40, 4, 1e-2), (57, 8, 1e-1)])
+def test_least_squares_against_staged_program(monkeypatch, n, precision, tol):
+    from spaqr_public_amd import gen
+    A, _ = sq.colscale(gen.laplacian_gradient_ls(n, 1e-2))
+    b = np.random.default_rng(n).standard_normal(A.shape[1])
+    got = []
+    for reg in ("0", "1"):
+        monkeypatch.setenv("SPAQR_REFL_REGISTER", reg)
+        t = sq.Tree(sq.default_levels(A.shape[1]), 0, precision)
+        t.set_scale(1)
+        t.set_tol(tol)
+        t.set_square(0)
+        t.set_tensor_coordinates(n, 2)
+        t.partition(A)
+        t.assemble(A)
+        t.factorize()
+        got.append([t.solve_nrml(b), t.solve_nrml(b)])
+        t.close()
+    # R^{-1} R^{-T} b by two routes, each backward stable; the column-scaled
+    # matrix with its regularising rows has a condition below 1e4, squared here
+    eps = np.finfo(np.float32 if precision == 4 else np.float64).eps
+    for a, c in zip(*got):
+        assert np.linalg.norm(a - c) <= (1e8 if precision == 8 else 1e5) * eps * np.linalg.norm(a)
+    assert precision == 4 or np.array_equal(got[1][0], got[1][1])
