@@ -79,28 +79,59 @@ std::vector<double> tensor_coordinates(int n, int dim) {
 
 namespace {
 
-// Median split of `dofs` along the coordinate with the largest range (first
-// such coordinate on ties); X <= median value goes to part `lo`, else lo + 1.
-void split_geo(const std::vector<int>& dofs, std::vector<int>& part, const std::vector<double>& X, int dim, int lo) {
-  if (dofs.empty()) return;
+// Median split of the columns [b, e) of `ord` along the coordinate with the
+// largest range (first such coordinate on ties): X <= median value goes to the
+// front, else to the back, each in its order; returns where the back begins.
+int split_geo(std::vector<int>& ord, int b, int e, const std::vector<double>& X, int dim, std::vector<double>& vals,
+              std::vector<int>& back) {
+  if (b == e) return b;
   int best = -1;
   double range = -1.0;
   for (int d = 0; d < dim; ++d) {
     double mx = std::numeric_limits<double>::lowest(), mn = std::numeric_limits<double>::max();
-    for (int v : dofs) {
-      const double c = X[(size_t)v * dim + d];
+    for (int q = b; q < e; ++q) {
+      const double c = X[(size_t)ord[q] * dim + d];
       mx = std::max(mx, c);
       mn = std::min(mn, c);
     }
     if (mx - mn > range) { range = mx - mn; best = d; }
   }
-  std::vector<double> vals;
-  vals.reserve(dofs.size());
-  for (int v : dofs) vals.push_back(X[(size_t)v * dim + best]);
-  const size_t mid = dofs.size() / 2;
+  vals.clear();
+  for (int q = b; q < e; ++q) vals.push_back(X[(size_t)ord[q] * dim + best]);
+  const size_t mid = vals.size() / 2;
   std::nth_element(vals.begin(), vals.begin() + mid, vals.end());
   const double cut = vals[mid];
-  for (int v : dofs) part[v] = (X[(size_t)v * dim + best] <= cut) ? lo : lo + 1;
+  back.clear();
+  int at = b;
+  for (int q = b; q < e; ++q) {
+    const int v = ord[q];
+    if (X[(size_t)v * dim + best] <= cut) ord[at++] = v;
+    else back.push_back(v);
+  }
+  std::copy(back.begin(), back.end(), ord.begin() + at);
+  return at;
+}
+
+// Pattern of A^T: the columns of each row, sorted.  Chunks of rows are filled
+// by a scan of all columns each.
+struct Pattern { std::vector<int> p, i; };
+Pattern row_pattern(const CscMat& A) {
+  Pattern T;
+  T.p.assign(A.m + 1, 0);
+  for (int r : A.i) T.p[r + 1]++;
+  std::partial_sum(T.p.begin(), T.p.end(), T.p.begin());
+  T.i.resize(A.nnz());
+  const int nch = A.nnz() < 65536 ? 1 : std::min(host_threads(), 8);
+  std::vector<int> fill(T.p.begin(), T.p.end() - 1);
+  parallel_for(nch, 1, [&](int, int b, int e) {
+    const int r0 = (int)((int64_t)b * A.m / nch), r1 = (int)((int64_t)e * A.m / nch);
+    for (int c = 0; c < A.n; ++c)
+      for (int q = A.p[c]; q < A.p[c + 1]; ++q) {
+        const int r = A.i[q];
+        if (r >= r0 && r < r1) T.i[fill[r]++] = c;
+      }
+  });
+  return T;
 }
 
 SepID climb_common(SepID a, SepID b) {  // partition.cpp:63-86
@@ -139,43 +170,66 @@ void rows_by_weight(const CscMat& A, const std::vector<CID>& cpermed, const std:
 
 std::vector<CID> geometric_labels(const CscMat& A, int nlevels, const std::vector<double>& X, int dim) {
   const int n = A.n;
-  const CscMat R = csc_transpose(A);  // R.p/R.i: columns of each row, sorted
-  // recursive bisection of all columns (nlevels - 1 times)
-  std::vector<int> part(n, 0);
+  const Pattern R = row_pattern(A);
+  constexpr int grain = 4096;
+  // recursive bisection of all columns (nlevels - 1 times): `ord` holds them
+  // part after part, in column order
+  std::vector<int> part(n, 0), ord(n), at{0, n};
+  std::iota(ord.begin(), ord.end(), 0);
   for (int depth = 0; depth < nlevels - 1; ++depth) {
     const int nparts = 1 << depth;
-    std::vector<std::vector<int>> groups(nparts);
-    for (int v = 0; v < n; ++v) groups[part[v]].push_back(v);
-    for (int g = 0; g < nparts; ++g) split_geo(groups[g], part, X, dim, 2 * g);
+    std::vector<int> next(2 * nparts + 1, n);
+    parallel_for(nparts, 1, [&](int, int b, int e) {
+      std::vector<double> vals;
+      std::vector<int> back;
+      for (int g = b; g < e; ++g) {
+        next[2 * g] = at[g];
+        next[2 * g + 1] = split_geo(ord, at[g], at[g + 1], X, dim, vals, back);
+      }
+    });
+    at = std::move(next);
   }
+  parallel_for((int)at.size() - 1, 16, [&](int, int b, int e) {
+    for (int g = b; g < e; ++g)
+      for (int q = at[g]; q < at[g + 1]; ++q) part[ord[q]] = g;
+  });
   // separators: from the top level down, a still-unlabelled column in an even
   // subtree becomes a separator of level l when an unlabelled column of the
-  // adjacent odd subtree is its neighbour in the graph of A^T A.
+  // adjacent odd subtree is its neighbour in the graph of A^T A.  (Columns of
+  // odd subtrees keep their state within a level, so the columns of one can be
+  // looked at in any order.)
   std::vector<CID> lab(n);
-  std::vector<int> stamp(n, -1);
+  std::vector<int> slvl(n, -1);
   for (int depth = 0; depth < nlevels - 1; ++depth) {
     const int l = nlevels - depth - 1;
-    for (int v = 0; v < n; ++v) {
-      if (lab[v].self.lvl != -1) continue;
-      const int pv = part[v] >> (l - 1);
-      if (pv & 1) continue;
-      bool sep = false;
-      for (int q = A.p[v]; q < A.p[v + 1] && !sep; ++q) {
-        const int row = A.i[q];
-        for (int t = R.p[row]; t < R.p[row + 1]; ++t) {
-          const int u = R.i[t];
-          if (lab[u].self.lvl == -1 && (part[u] >> (l - 1)) == pv + 1) { sep = true; break; }
+    parallel_for(n, grain, [&](int, int b, int e) {
+      for (int v = b; v < e; ++v) {
+        if (slvl[v] != -1) continue;
+        const int pv = part[v] >> (l - 1);
+        if (pv & 1) continue;
+        bool sep = false;
+        for (int q = A.p[v]; q < A.p[v + 1] && !sep; ++q) {
+          const int row = A.i[q];
+          for (int t = R.p[row]; t < R.p[row + 1]; ++t) {
+            const int u = R.i[t];
+            if ((part[u] >> (l - 1)) == pv + 1 && slvl[u] == -1) { sep = true; break; }
+          }
+        }
+        if (sep) {
+          slvl[v] = l;
+          lab[v].self = SepID(l, pv / 2);
         }
       }
-      if (sep) lab[v].self = SepID(l, pv / 2);
-    }
+    });
   }
-  for (int v = 0; v < n; ++v)
-    if (lab[v].self.lvl == -1) {
-      lab[v].self = SepID(0, part[v]);
-      lab[v].l = lab[v].self;
-      lab[v].r = lab[v].self;
-    }
+  parallel_for(n, grain, [&](int, int b, int e) {
+    for (int v = b; v < e; ++v)
+      if (slvl[v] == -1) {
+        lab[v].self = SepID(0, part[v]);
+        lab[v].l = lab[v].self;
+        lab[v].r = lab[v].self;
+      }
+  });
   // row labels
   std::vector<CID> rlab(A.m);
   if (A.m != A.n) {
@@ -189,39 +243,43 @@ std::vector<CID> geometric_labels(const CscMat& A, int nlevels, const std::vecto
     rlab = lab;
   }
   // interfaces (partition.cpp:506-578): pass 1 from lower-level neighbours
-  for (int r = 0; r < A.m; ++r) {
-    const SepID self = rlab[r].self;
-    if (self.lvl <= 0) continue;
-    SepID left, right;
-    for (int t = R.p[r]; t < R.p[r + 1]; ++t) {
-      const SepID nb = lab[R.i[t]].self;
-      if (nb.lvl >= self.lvl) continue;
-      const int side = (int)(nb.sep / std::pow(2.0, self.lvl - nb.lvl - 1));
-      if (side % 2 == 0) left = (left.lvl == -1) ? nb : lower_of(nb, left);
-      else right = (right.lvl == -1) ? nb : lower_of(nb, right);
+  parallel_for(A.m, grain, [&](int, int b, int e) {
+    for (int r = b; r < e; ++r) {
+      const SepID self = rlab[r].self;
+      if (self.lvl <= 0) continue;
+      SepID left, right;
+      for (int t = R.p[r]; t < R.p[r + 1]; ++t) {
+        const SepID nb = lab[R.i[t]].self;
+        if (nb.lvl >= self.lvl) continue;
+        const int side = nb.sep >> (self.lvl - nb.lvl - 1);
+        if (side % 2 == 0) left = (left.lvl == -1) ? nb : lower_of(nb, left);
+        else right = (right.lvl == -1) ? nb : lower_of(nb, right);
+      }
+      rlab[r].l = left;
+      rlab[r].r = right;
     }
-    rlab[r].l = left;
-    rlab[r].r = right;
-  }
+  });
   std::vector<CID> clab = rlab;  // row i matched to column i
   // pass 2: a missing side is borrowed from same-separator neighbours
-  for (int r = 0; r < A.m; ++r) {
-    const SepID self = rlab[r].self;
-    SepID left = rlab[r].l, right = rlab[r].r;
-    if (right == SepID()) {
-      for (int t = R.p[r]; t < R.p[r + 1]; ++t) {
-        const CID& c = clab[R.i[t]];
-        if (c.self == self && c.r != SepID()) right = (right == SepID()) ? c.r : climb_common(right, c.r);
+  parallel_for(A.m, grain, [&](int, int b, int e) {
+    for (int r = b; r < e; ++r) {
+      const SepID self = rlab[r].self;
+      SepID left = rlab[r].l, right = rlab[r].r;
+      if (right == SepID()) {
+        for (int t = R.p[r]; t < R.p[r + 1]; ++t) {
+          const CID& c = clab[R.i[t]];
+          if (c.self == self && c.r != SepID()) right = (right == SepID()) ? c.r : climb_common(right, c.r);
+        }
+      } else if (left == SepID()) {
+        for (int t = R.p[r]; t < R.p[r + 1]; ++t) {
+          const CID& c = clab[R.i[t]];
+          if (c.self == self && c.l != SepID()) left = (left == SepID()) ? c.l : climb_common(left, c.l);
+        }
       }
-    } else if (left == SepID()) {
-      for (int t = R.p[r]; t < R.p[r + 1]; ++t) {
-        const CID& c = clab[R.i[t]];
-        if (c.self == self && c.l != SepID()) left = (left == SepID()) ? c.l : climb_common(left, c.l);
-      }
+      rlab[r].l = left;
+      rlab[r].r = right;
     }
-    rlab[r].l = left;
-    rlab[r].r = right;
-  }
+  });
   for (auto& c : rlab) {
     if (c.l == SepID()) c.l = c.self;
     if (c.r == SepID()) c.r = c.self;
@@ -229,14 +287,62 @@ std::vector<CID> geometric_labels(const CscMat& A, int nlevels, const std::vecto
   return rlab;
 }
 
+// Columns by their labels: the order that stable sorts by the label and then by
+// its merged form at each level leave, so the last level's form counts first.
+// There are far fewer labels than columns: those are sorted, and the columns
+// counted into their places.
 void order_columns(int nlevels, const std::vector<CID>& labels, std::vector<int>& cperm) {
-  std::vector<CID> key = labels;
-  auto by_key = [&key](int a, int b) { return key[a] < key[b]; };
-  std::stable_sort(cperm.begin(), cperm.end(), by_key);
-  for (int lvl = 1; lvl < nlevels; ++lvl) {
-    for (auto& c : key) c = cid_merge_if(c, lvl);
-    std::stable_sort(cperm.begin(), cperm.end(), by_key);
+  const int n = (int)cperm.size();
+  auto mix = [](const CID& c) {
+    size_t h = 1469598103934665603ull;
+    for (int v : {c.self.lvl, c.self.sep, c.l.lvl, c.l.sep, c.r.lvl, c.r.sep, c.part, c.section})
+      h = (h ^ (size_t)(unsigned)v) * 1099511628211ull;
+    return h ^ (h >> 29);
+  };
+  // distinct labels, in order of appearance
+  std::vector<CID> key;
+  std::vector<int> id(labels.size()), table(1024, -1);
+  std::vector<size_t> hash;
+  for (size_t v = 0; v < labels.size(); ++v) {
+    if (v > 0 && labels[v] == labels[v - 1]) { id[v] = id[v - 1]; continue; }
+    const size_t h = mix(labels[v]);
+    size_t q = h & (table.size() - 1);
+    while (table[q] >= 0 && !(hash[table[q]] == h && key[table[q]] == labels[v])) q = (q + 1) & (table.size() - 1);
+    if (table[q] < 0) {
+      table[q] = (int)key.size();
+      key.push_back(labels[v]);
+      hash.push_back(h);
+      if (2 * key.size() > table.size()) {
+        table.assign(2 * table.size(), -1);
+        for (size_t d = 0; d < key.size(); ++d) {
+          size_t t = hash[d] & (table.size() - 1);
+          while (table[t] >= 0) t = (t + 1) & (table.size() - 1);
+          table[t] = (int)d;
+        }
+        id[v] = (int)key.size() - 1;
+        continue;
+      }
+    }
+    id[v] = table[q];
   }
+  const int nd = (int)key.size();
+  std::vector<int> order(nd);
+  std::iota(order.begin(), order.end(), 0);
+  auto by_key = [&key](int a, int b) { return key[a] < key[b]; };
+  std::sort(order.begin(), order.end(), by_key);
+  for (int lvl = 1; lvl < nlevels; ++lvl) {
+    parallel_for(nd, 1024, [&](int, int b, int e) {
+      for (int d = b; d < e; ++d) key[d] = cid_merge_if(key[d], lvl);
+    });
+    if (!std::is_sorted(order.begin(), order.end(), by_key)) std::stable_sort(order.begin(), order.end(), by_key);
+  }
+  // cperm's columns by rank, in cperm's order
+  std::vector<int> rank(nd), at(nd + 1, 0), out(n);
+  for (int q = 0; q < nd; ++q) rank[order[q]] = q;
+  for (int c : cperm) at[rank[id[c]] + 1]++;
+  std::partial_sum(at.begin(), at.end(), at.begin());
+  for (int c : cperm) out[at[rank[id[c]]]++] = c;
+  cperm = std::move(out);
 }
 
 void order_rows_ls(const CscMat& Ap, const std::vector<CID>& cpermed, std::vector<int>& rperm,
