@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <exception>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -38,8 +39,12 @@ namespace {
 // use and never destroyed (its threads sleep through process exit).
 class Pool {
  public:
+  // (fewer workers where the system grants no more threads)
   explicit Pool(int workers) {
-    for (int i = 0; i < workers; ++i) th_.emplace_back([this] { work(); });
+    try {
+      for (int i = 0; i < workers; ++i) th_.emplace_back([this] { work(); });
+    } catch (const std::system_error&) {
+    }
   }
   std::mutex run_mu;  // held by the thread whose job the pool is running
 
