@@ -886,7 +886,8 @@ class Engine final : public EngineBase {
   }
   bool flow_fits() const;
   bool build_flow();
-  bool build_flow_ls(const std::vector<std::vector<const Op*>>& by_level);
+  bool build_flow_mode(int t);
+  bool build_flow_ls();
   template <typename U>
   void build_w(const std::vector<WyJob<U>>& jobs);
   template <typename U>
@@ -902,12 +903,12 @@ class Engine final : public EngineBase {
     const int* top_out = nullptr;
     int top_at = 0;                // their places afterwards
     int xplaces = 0, x64places = 0;
+    T* x = nullptr;
+    double* x64 = nullptr;
     const int* out = nullptr;      // places of the result
   };
-  bool flow_ = false;
+  bool flow_ = false, flow_off_ = false;
   FlowMode flow_mode_[2];
-  T* flow_x_ = nullptr;
-  double* flow_x64_ = nullptr;
   int flow_top_n_ = 0;
   const int *flow_rperm_ = nullptr, *flow_cperm_ = nullptr;  // rows and columns in cluster order
   // ------------------------------------------------------------ state
@@ -2901,7 +2902,7 @@ int Engine<T>::factorize() {  // tree.cpp:1309-1437
 // the staged program.
 template <typename T>
 bool Engine<T>::flow_fits() const {
-  if (!reflr_ || stage_prof_) return false;
+  if (!reflr_ || stage_prof_ || flow_off_) return false;
   auto too_long = [](int64_t ld, int64_t cols) { return ld * cols * 8 > int64_t(0xffffffffu); };  // 32-bit offsets
   for (auto& o : ops_) {
     if (o.kind == OpFineQR || (!square_ && o.V64)) return false;
@@ -3211,9 +3212,15 @@ bool Engine<T>::build_flow() {
   }
   build_w(wj);
   build_w(wj64);
+  return square_ ? build_flow_mode(0) : build_flow_ls();
+}
+
+// The program of M^{-1} (t = 0), built with the factors, or of M^{-T} (1), built
+// when it is first asked for.
+template <typename T>
+bool Engine<T>::build_flow_mode(int t) {
   std::vector<std::vector<const Op*>> by_level(nlevels_);
   for (auto& o : ops_) by_level[o.level].push_back(&o);
-  if (!square_) return build_flow_ls(by_level);
   // stages of the forward and the backward tape; the FP64 top apart
   std::vector<FlowStage> fwd, bwd;
   const Op* top = nullptr;
@@ -3285,11 +3292,9 @@ bool Engine<T>::build_flow() {
     a.insert(a.end(), b.begin(), b.end());
     return a;
   };
-  const std::vector<FlowStage> first[2] = {fwd, transpose(bwd)}, second[2] = {bwd, transpose(fwd)};
-  const double bytes0 = solve_bytes_;
-  for (int t = 1; t >= 0; --t) {
-    solve_bytes_ = bytes0;  // in the end those of the forward apply
-    FlowMode& M = flow_mode_[t];
+  const std::vector<FlowStage> first = t ? transpose(bwd) : std::move(fwd), second = t ? transpose(fwd) : std::move(bwd);
+  FlowMode& M = flow_mode_[t];
+  {
     FlowRows R;
     R.of.resize(cl_.size());
     R.scratch.assign(cl_.size(), 0);
@@ -3300,7 +3305,7 @@ bool Engine<T>::build_flow() {
     M.run.clear();
     if (top) {
       M.run.resize(2);
-      if (!flow_prog<T>(first[t], R, M.run[0])) return false;
+      if (!flow_prog<T>(first, R, M.run[0])) return false;
       const int c = top->c;
       flow_top_n_ = top->m;
       M.top_in = stager_.upload(perm_, flow_places(R, {c}));
@@ -3318,22 +3323,18 @@ bool Engine<T>::build_flow() {
       M.top_at = R.next;
       R.of[c].assign(1, FlowSeg{R.next, top->m});
       R.next += top->m;
-      if (!flow_prog<T>(second[t], R, M.run[1])) return false;
+      if (!flow_prog<T>(second, R, M.run[1])) return false;
     } else {
       M.run.resize(1);
-      if (!flow_prog<T>(join(first[t], second[t]), R, M.run[0])) return false;
+      if (!flow_prog<T>(join(first, second), R, M.run[0])) return false;
     }
     M.xplaces = R.next;
     M.out = stager_.upload(perm_, flow_places(R, bottoms_[0]));
   }
-  xsize_ = std::max(flow_mode_[0].xplaces, flow_mode_[1].xplaces);
-  flow_x_ = alloc_perm((size_t)xsize_);
-  if (top)
-    flow_x64_ = (double*)perm_.alloc(sizeof(double) * (size_t)std::max(flow_mode_[0].x64places, flow_mode_[1].x64places));
-  for (auto& M : flow_mode_) {
-    for (auto& r : M.run) r.args.x = flow_x_;
-    M.top.args.x = flow_x64_;
-  }
+  M.x = alloc_perm((size_t)M.xplaces);
+  for (auto& r : M.run) r.args.x = M.x;
+  if (top) M.top.args.x = M.x64 = (double*)perm_.alloc(sizeof(double) * (size_t)M.x64places);
+  if (t) return true;
   std::vector<int> rp, cp;
   for (int c : bottoms_[0])
     for (int i = 0; i < cl_[c].rsize_org; ++i) {
@@ -3350,7 +3351,9 @@ bool Engine<T>::build_flow() {
 // interfaces' reflectors up the tree on xt, row permutations down and up again,
 // and the backward tape on x.  Only list entries move in the permutations.
 template <typename T>
-bool Engine<T>::build_flow_ls(const std::vector<std::vector<const Op*>>& by_level) {
+bool Engine<T>::build_flow_ls() {
+  std::vector<std::vector<const Op*>> by_level(nlevels_);
+  for (auto& o : ops_) by_level[o.level].push_back(&o);
   FlowMode& M = flow_mode_[0];
   FlowRows R;
   R.of.resize(cl_.size());
@@ -3465,9 +3468,8 @@ bool Engine<T>::build_flow_ls(const std::vector<std::vector<const Op*>>& by_leve
       for (int i = 0; i < sg.len; ++i) out.push_back(sg.off < 0 ? R.zero : sg.off + i);
   M.out = stager_.upload(perm_, out);
   flow_cperm_ = flow_rperm_ = stager_.upload(perm_, cp);
-  xsize_ = M.xplaces;
-  flow_x_ = alloc_perm((size_t)xsize_);
-  M.run[0].args.x = flow_x_;
+  M.x = alloc_perm((size_t)M.xplaces);
+  M.run[0].args.x = M.x;
   flow_ = true;
   return true;
 }
@@ -4080,23 +4082,23 @@ void Engine<T>::run_flow(const double* b, double* x, bool transposed) {
     c.p[i] = (unsigned int*)p;
     c.n[i++] = words;
   };
-  clear(flow_x_ + ncols_ + nz, (int64_t)(M.xplaces - ncols_ - nz) * (int64_t)(sizeof(T) / 4));
+  clear(M.x + ncols_ + nz, (int64_t)(M.xplaces - ncols_ - nz) * (int64_t)(sizeof(T) / 4));
   for (auto& r : M.run) clear(r.zero, r.nzero);
   const bool top = M.run.size() > 1;
   if (top) {
-    clear(flow_x64_, 2 * (int64_t)M.x64places);
+    clear(M.x64, 2 * (int64_t)M.x64places);
     clear(M.top.zero, M.top.nzero);
   }
   // M^{-T}: b enters through the exit map and leaves through the entry map
-  launch_flow_begin<T>(stream_, transposed ? flow_cperm_ : flow_rperm_, ncols_, b, flow_x_, nz, c);
+  launch_flow_begin<T>(stream_, transposed ? flow_cperm_ : flow_rperm_, ncols_, b, M.x, nz, c);
   launch_flow<T>(stream_, M.run[0].args, M.run[0].grid);
   if (top) {
-    launch_flow_cvt<T, double>(stream_, M.top_in, flow_top_n_, flow_x_, flow_x64_, 0);
+    launch_flow_cvt<T, double>(stream_, M.top_in, flow_top_n_, M.x, M.x64, 0);
     launch_flow<double>(stream_, M.top.args, M.top.grid);
-    launch_flow_cvt<double, T>(stream_, M.top_out, flow_top_n_, flow_x64_, flow_x_, M.top_at);
+    launch_flow_cvt<double, T>(stream_, M.top_out, flow_top_n_, M.x64, M.x, M.top_at);
     launch_flow<T>(stream_, M.run[1].args, M.run[1].grid);
   }
-  launch_flow_out<T>(stream_, M.out, ncols_, flow_x_, transposed ? flow_rperm_ : flow_cperm_, x);
+  launch_flow_out<T>(stream_, M.out, ncols_, M.x, transposed ? flow_rperm_ : flow_cperm_, x);
 }
 
 template <typename T>
@@ -4228,6 +4230,17 @@ template <typename T>
 void Engine<T>::solve_t_dev(const double* b, double* x) {
   if (!factored_) throw Error(kErrState, "solve_transpose before factorize");
   if (!square_) throw Error(kErrState, "solve_transpose: rectangular (least-squares) tree");
+  if (flow_) {
+    if (flow_mode_[1].run.empty()) {
+      const double bytes = solve_bytes_;
+      flow_ = build_flow_mode(1);
+      if (!flow_) {  // an op with too many input segments: this tree's applies are staged from here on
+        flow_off_ = true;
+        build_solve_program();
+      }
+      solve_bytes_ = bytes;
+    }
+  }
   if (flow_) {
     timed("apply", 0.0, solve_bytes_, [&] { run_flow(b, x, true); });
     return;
