@@ -10,8 +10,9 @@
 // and as the accumulators of the update alike.  (As two GEMMs C was read twice,
 // Y made a round through memory, and long sums over few tiles had to be split:
 // 64^3, 640 steps of 106 GB of C in all: 98.8 -> 50.3 ms; 33^3 16.4 -> 5.5 ms;
-// 2-D 128^2 2.57 -> 0.79 ms.)  What is left beside HBM is V, which every 16
-// columns read twice from L2: 2.1-2.4 TB/s of C in forms of 128 rows and more.
+// 2-D 128^2 2.57 -> 0.79 ms.)  Forms of 128 rows and more move 2.1-2.4 TB/s of
+// C: a workgroup waits for memory twice and at three barriers, with 3-7 of
+// them on a CU.  32 columns a workgroup, which halve V's reads, took as long.
 //
 // A lane (k4 = lane / 16, c16 = lane % 16) holds rows 4 k4 .. 4 k4 + 3 of a tile
 // in column c16, which are 16-byte loads along the column.  The contraction over
