@@ -486,8 +486,8 @@ def main():
     fac = float(np.mean(fac_t))
     kry = float(np.mean(kry_t))
     # dominant kernel over the timed steps: timing families grouped by the
-    # kernel they launch (the GEMM roles all run k_gemm); the solve program
-    # ("apply", a graph of many kernels) is reported separately
+    # kernel they launch (the GEMM roles all run k_gemm); the applies
+    # ("apply") are reported separately
     tname = "double" if precision == sq.FP64 else "float"
     per_kernel = {}
     for fam, v in stats_acc.items():

@@ -30,7 +30,12 @@ void* Arena::alloc(size_t bytes, size_t align) {
   size_t sz = bytes > chunk_ ? (bytes + align) : chunk_;
   const double t0 = wall();
   if (chunks_.empty()) SPQ_HIP(hipGetDevice(&dev_));
-  char* p = pool_take(false, sz);
+  char* p = nullptr;
+  try {
+    p = pool_take(false, sz);
+  } catch (const Error& e) {
+    throw Error(kErrOom, "device allocation of " + std::to_string(sz) + " bytes failed: " + e.what());
+  }
   t_chunks += wall() - t0;
   ++n_chunks;
   chunks_.push_back({p, sz, 0});
@@ -94,13 +99,8 @@ char* pool_take(bool host, size_t& bytes, bool largest) {
     }
   }
   void* p = nullptr;
-  if (host) {
-    SPQ_HIP(host_malloc(&p, bytes));
-    return (char*)p;
-  }
-  const hipError_t e = dev_malloc(&p, bytes);
-  if (e != hipSuccess)
-    throw Error(kErrOom, "device allocation of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
+  if (host) SPQ_HIP(host_malloc(&p, bytes));
+  else SPQ_HIP(dev_malloc(&p, bytes));
   return (char*)p;
 }
 

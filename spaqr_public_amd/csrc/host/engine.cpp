@@ -533,8 +533,7 @@ class Engine final : public EngineBase {
   // Blocked Householder QR of a batch of panels.  For every block step the
   // panel kernel factors NB columns, then the block reflector is applied to the
   // panel's trailing columns and to every extra matrix `extra[p]` (same row
-  // space as the panel, ld given) with three batched GEMMs:
-  //   Y = V_b^T C ; Z = T_b^T Y ; C -= V_b Z.
+  // space as the panel, ld given): C -= V_b (T_b^T (V_b^T C)).
   template <typename U>
   struct QrJobT {
     U* P; int ld, m, k;
@@ -745,9 +744,8 @@ class Engine final : public EngineBase {
     });
   }
 
-  // tables of the larfb block steps and gemm_batch's tile counts, kept per
-  // host thread across block steps and trees: a level-0 step plans ~300k
-  // descriptors, and fresh memory costs more host time (page faults) than
+  // tables of the larfb block steps, kept per host thread across block steps
+  // and trees: a level-0 step plans more than 100k descriptors, and fresh memory costs more host time (page faults) than
   // filling it.  The memory is held until the thread ends.
   template <typename U>
   struct LarfbBufs {
@@ -2870,8 +2868,8 @@ int Engine<T>::factorize() {  // tree.cpp:1309-1437
   }
   const double tbp = wall();
   build_solve_program();
-  // the apply's graph is instantiated here, so solves (and the Krylov drivers
-  // around them) allocate nothing on the device
+  // a staged apply's graph is instantiated here (a dataflow apply has none), so
+  // solves and the Krylov drivers around them allocate nothing on the device
   if (solve_graph_ && !stage_prof_ && !flow_) {
     if (square_) graph_exec_fwd_ = capture_program(0);
     else graph_exec_nrml_ = capture_program(1);

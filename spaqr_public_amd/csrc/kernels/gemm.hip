@@ -1,5 +1,6 @@
-// Batched uneven GEMM with structured operands for the block-reflector
-// updates (larfb), T assembly and blocked TRSM of the spaQR phases.
+// Batched uneven GEMM with structured operands: blocked TRSM, Q^T on
+// neighbours, W = V T^T of the applies, and the block-reflector updates
+// (larfb) of panels with more rows than k_larfb holds.
 //   C = alpha * op(A) * op(B) + beta * C
 // Structure masks (unit-lower V, triangular T/R) are applied while staging,
 // so the stored upper triangle of a Householder panel (which holds R) is

@@ -5,7 +5,7 @@
 // tau = (beta - alpha) / beta, v(0) = 1), the reflector applied to the
 // remaining columns of the block, and the block's compact-WY factor T
 // (forward, columnwise: T(0:j,j) = -tau_j T(0:j,0:j) V^T v_j).  The caller
-// applies the block to the trailing columns with the batched GEMM.
+// applies the block to the trailing columns (k_larfb).
 #include "kcommon.hpp"
 #include "descs.hpp"
 #include "launch.hpp"

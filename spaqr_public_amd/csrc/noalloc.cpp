@@ -10,8 +10,8 @@
 // The kernels write every scratch element before reading it (partial sums,
 // basis columns, residuals), so nothing needs clearing between calls.  Every
 // call on one GPU shares its array: calls that overlap on one GPU race.  The
-// solve graph is instantiated by factorize, so the preconditioner applies
-// inside allocate nothing either.
+// solve program and its work space are made by factorize, so the preconditioner
+// applies inside allocate nothing either.
 #include <mutex>
 #include <string>
 
