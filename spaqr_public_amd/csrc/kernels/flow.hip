@@ -181,6 +181,9 @@ __device__ __forceinline__ T flow_poll(const T* X, int at, int* err) {
 // lane's registers and one exchange between the half waves, where a row in each
 // lane needs a 32-way reduction over the wave (2.4 -> 0.6 us an op, masks at the
 // trapezoids' edges included: they are applied while x is still awaited).
+// Two workgroups a CU: bounded to three, FP64 spills 109 registers, and with as
+// many more parts to fill them an apply is 1.3-1.5x slower (2D n = 64: 147 -> 189
+// us, 3D n = 52: 1575 -> 2222 us; bound and part count were changed together).
 template <typename T>
 __global__ __launch_bounds__(kFT, 2) void k_flow(const FlowArgs<T> P) {
   constexpr int KM = kFlowMaxK;
