@@ -838,6 +838,23 @@ class Engine final : public EngineBase {
     unsigned int* zero = nullptr;  // exchange slots and tickets, cleared before each apply
     int64_t nzero = 0;             // words
   };
+  // its tables before they have a place on the device
+  template <typename U>
+  struct FlowPlan {
+    std::vector<FlowOp<U>> parts;
+    std::vector<FlowSeg> segs;
+    std::vector<FlowBlk<U>> blks;
+    std::vector<FlowDiag<U>> diags;
+    std::vector<int> diag_start{0};
+    // by part: its exchange slots; where its diagonal blocks begin (-1: none)
+    std::vector<size_t> slot_at;
+    std::vector<int64_t> diag_at;
+    size_t slots = 0;
+    int64_t diag_elems = 0;
+    int grid = 0;
+    double bytes = 0;  // the factors and vectors an apply streams
+    bool fits = true;  // no op has more input segments than the kernel takes
+  };
   // places of x holding the rows of each cluster, as segments (least squares:
   // zeros, off -1, where nothing was written)
   using FlowList = std::vector<FlowSeg>;
@@ -884,16 +901,16 @@ class Engine final : public EngineBase {
   }
   bool flow_fits() const;
   bool build_flow();
-  bool build_flow_mode(int t);
-  bool build_flow_ls();
   template <typename U>
   void build_w(const std::vector<WyJob<U>>& jobs);
   template <typename U>
-  bool flow_prog(const std::vector<FlowStage>& stages, FlowRows& rows, FlowProg<U>& out);
+  void flow_plan(const std::vector<FlowStage>& stages, FlowRows& rows, int grid, FlowPlan<U>& plan) const;
+  template <typename U>
+  void flow_place(FlowPlan<U>& plan, FlowProg<U>& prog);
   std::vector<int> flow_places(const FlowRows& rows, const std::vector<int>& clusters) const;
   void run_flow(const double* b, double* x, bool transposed);
-  // modes 0 and 2 (M^{-1}, M^{-T}): one program, or around the FP64 top of an
-  // FP32 tree one before and one after it
+  // M^{-1} and M^{-T} (flow_mode_[0], [1]): one program, or around the FP64 top
+  // of an FP32 tree one before and one after it
   struct FlowMode {
     std::vector<FlowProg<T>> run;
     FlowProg<double> top;
@@ -901,12 +918,25 @@ class Engine final : public EngineBase {
     const int* top_out = nullptr;
     int top_at = 0;                // their places afterwards
     int xplaces = 0, x64places = 0;
-    T* x = nullptr;
-    double* x64 = nullptr;
     const int* out = nullptr;      // places of the result
   };
-  bool flow_ = false, flow_off_ = false;
+  struct FlowModePlan {
+    std::vector<FlowPlan<T>> run;
+    FlowPlan<double> top;
+    std::vector<int> top_in, top_out, out;
+    int top_n = 0, top_at = 0, xplaces = 0, x64places = 0;
+    bool fits() const {
+      bool f = top.fits;
+      for (auto& r : run) f = f && r.fits;
+      return f;
+    }
+  };
+  void plan_flow_mode(int t, int grid, int grid64, FlowModePlan& P) const;
+  void plan_flow_ls(int grid, FlowModePlan& P) const;
+  bool flow_ = false;  // applies run the dataflow programs
   FlowMode flow_mode_[2];
+  T* flow_x_ = nullptr;
+  double* flow_x64_ = nullptr;
   int flow_top_n_ = 0;
   const int *flow_rperm_ = nullptr, *flow_cperm_ = nullptr;  // rows and columns in cluster order
   // ------------------------------------------------------------ state
@@ -2900,7 +2930,7 @@ int Engine<T>::factorize() {  // tree.cpp:1309-1437
 // the staged program.
 template <typename T>
 bool Engine<T>::flow_fits() const {
-  if (!reflr_ || stage_prof_ || flow_off_) return false;
+  if (!reflr_ || stage_prof_) return false;
   auto too_long = [](int64_t ld, int64_t cols) { return ld * cols * 8 > int64_t(0xffffffffu); };  // 32-bit offsets
   for (auto& o : ops_) {
     if (o.kind == OpFineQR || (!square_ && o.V64)) return false;
@@ -2958,21 +2988,31 @@ void Engine<T>::build_w(const std::vector<WyJob<U>>& jobs) {
   for (auto& v : sums) gemm_batch(v, "wy");
 }
 
-// One launch of k_flow over the stages; false if an op has more input
-// segments than the kernel takes.
+// One launch of k_flow over the stages on `cap` workgroups (host work only).
 template <typename T>
 template <typename U>
-bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, FlowProg<U>& p) {
-  std::vector<FlowOp<U>> parts;
-  std::vector<FlowSeg> segs;
-  std::vector<FlowBlk<U>> blks;
+void Engine<T>::flow_plan(const std::vector<FlowStage>& stages, FlowRows& R, int cap, FlowPlan<U>& p) const {
+  auto &parts = p.parts;
+  auto &segs = p.segs;
+  auto &blks = p.blks;
+  auto &diags = p.diags;
+  auto &diag_start = p.diag_start;
   constexpr bool top = sizeof(U) > sizeof(T);  // the FP64 factors of an FP32 tree's top
-  std::vector<FlowDiag<U>> diags;
-  std::vector<int> diag_start{0};
-  size_t slots = 0;
-  std::vector<size_t> slot_at;  // by part
   std::vector<int>& wave = R.scratch;  // of a chain: waves so far on a cluster
-  const int cap = std::min(flow_capacity<U>(), 2 * num_cus_);
+  p.grid = cap;
+  // (fresh memory costs more host time than filling it: no tables that grow by
+  // copying)
+  size_t items = 0, links = 0;
+  for (auto& st : stages) {
+    items += st.items.size();
+    for (auto& it : st.items)
+      if (it.type != kFlowWY) links += it.op->r12.size();
+  }
+  parts.reserve(2 * items + links);
+  p.slot_at.reserve(parts.capacity());
+  p.diag_at.reserve(parts.capacity());
+  segs.reserve(2 * items + links);
+  blks.reserve(3 * links);
   auto add_seg = [](FlowList& v, size_t from, FlowSeg sg) { flow_add(v, from, sg); };
   // the first n rows of a cluster
   auto rows_of = [&](int c, int n, FlowList& v, size_t from) {
@@ -3000,16 +3040,16 @@ bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, Flo
     R.of[c].clear();
     if (n > 0) R.of[c].push_back(FlowSeg{off, n});
   };
-  bool fits = true;
-  auto add_op = [&](FlowOp<U>& d, int nparts) {
-    fits = fits && d.nseg <= kFlowMaxSegs;
+  auto add_op = [&](FlowOp<U>& d, int nparts, int64_t diag = -1) {
+    p.fits = p.fits && d.nseg <= kFlowMaxSegs;
     d.out = R.next;
     R.next += d.m;
     for (d.g = 0; d.g < nparts; ++d.g) {
       parts.push_back(d);
-      slot_at.push_back(slots);
+      p.slot_at.push_back(p.slots);
+      p.diag_at.push_back(diag);
     }
-    if (d.nwg > 1) slots += (size_t)d.nwg * d.k;
+    if (d.nwg > 1) p.slots += (size_t)d.nwg * d.k;
   };
   for (auto& st : stages) {
     // ops side by side: all, or in a chain an average wave
@@ -3046,7 +3086,7 @@ bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, Flo
         const int rp = o.k <= 32 ? 256 : (o.k <= 64 ? 128 : 64);
         d.rows_per = std::min(kFlowMaxK, std::max(rp, iceil(iceil(o.m, maxp), 64) * 64));
         d.nwg = std::max(1, iceil(o.m, d.rows_per));
-        solve_bytes_ += sizeof(U) * (2.0 * o.m * o.k - (double)o.k * o.k + 2.0 * o.m);
+        p.bytes += sizeof(U) * (2.0 * o.m * o.k - (double)o.k * o.k + 2.0 * o.m);
         add_op(d, d.nwg);
         int off = d.out;
         for (auto& sg : o.segs) {
@@ -3086,13 +3126,12 @@ bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, Flo
         }
       d.nblk = (int)blks.size() - d.blk0;
       if (it.type == kFlowBack) d.nwg = std::max(1, std::min({maxp, d.nblk, d.nblk * iceil(d.k, 64) / 8}));
-      solve_bytes_ += by + sizeof(U) * (0.5 * d.k * d.k + 2.0 * d.k);
+      p.bytes += by + sizeof(U) * (0.5 * d.k * d.k + 2.0 * d.k);
       const int nb = iceil(d.k, nb_);
-      U* D = (U*)perm_.alloc(sizeof(U) * (size_t)nb * nb_ * (nb_ + 1));
-      diags.push_back(FlowDiag<U>{d.A, D, d.lda, d.k, it.type == kFlowSolveT, 0});
+      diags.push_back(FlowDiag<U>{d.A, nullptr, d.lda, d.k, it.type == kFlowSolveT, 0});
       diag_start.push_back(diag_start.back() + nb);
-      d.B = D;
-      add_op(d, d.nwg);
+      add_op(d, d.nwg, p.diag_elems);
+      p.diag_elems += (int64_t)flow_diag_elems(d.k);
       set_rows(o.c, d.out, d.k);
     }
     // the products x_n - sum A^T x_c after the transposed solves, by target
@@ -3158,23 +3197,35 @@ bool Engine<T>::flow_prog(const std::vector<FlowStage>& stages, FlowRows& R, Flo
     }
     for (auto& f : st.moves) f();
   }
-  if (!fits) return false;
-  const size_t slot_words = slots * sizeof(U) / 4;
-  p.nzero = (int64_t)(slot_words + 64);
-  p.zero = (unsigned int*)perm_.alloc(4 * (size_t)p.nzero);
-  for (size_t i = 0; i < parts.size(); ++i)
-    if (parts[i].nwg > 1) parts[i].slots = (U*)p.zero + slot_at[i];
-  p.grid = cap;
-  p.args.nparts = (int)parts.size();
-  const FlowDiag<U>* dd = stager_.push(diags);
-  const int* ds = stager_.push(diag_start);
-  timed("wy", 0.0, 0.0, [&] { launch_flow_diag<U>(stream_, dd, ds, (int)diags.size(), diag_start.back()); });
-  p.args.parts = stager_.upload(perm_, parts);
-  p.args.segs = stager_.upload(perm_, segs);
-  p.args.blks = stager_.upload(perm_, blks);
-  p.args.ctl = p.zero + slot_words;
-  p.args.err = solve_err_;
-  return true;
+}
+
+// The plan's tables and work space on the device.
+template <typename T>
+template <typename U>
+void Engine<T>::flow_place(FlowPlan<U>& p, FlowProg<U>& g) {
+  const size_t slot_words = p.slots * sizeof(U) / 4;
+  g.nzero = (int64_t)(slot_words + 64);
+  g.zero = (unsigned int*)perm_.alloc(4 * (size_t)g.nzero);
+  U* const D = (U*)perm_.alloc(sizeof(U) * (size_t)p.diag_elems);
+  for (size_t i = 0; i < p.parts.size(); ++i) {
+    if (p.parts[i].nwg > 1) p.parts[i].slots = (U*)g.zero + p.slot_at[i];
+    if (p.diag_at[i] >= 0) p.parts[i].B = D + p.diag_at[i];
+  }
+  int64_t at = 0;
+  for (auto& d : p.diags) {
+    d.D = D + at;
+    at += (int64_t)flow_diag_elems(d.k);
+  }
+  g.grid = p.grid;
+  g.args.nparts = (int)p.parts.size();
+  const FlowDiag<U>* dd = stager_.push(p.diags);
+  const int* ds = stager_.push(p.diag_start);
+  timed("wy", 0.0, 0.0, [&] { launch_flow_diag<U>(stream_, dd, ds, (int)p.diags.size(), p.diag_start.back()); });
+  g.args.parts = stager_.upload(perm_, p.parts);
+  g.args.segs = stager_.upload(perm_, p.segs);
+  g.args.blks = stager_.upload(perm_, p.blks);
+  g.args.ctl = g.zero + slot_words;
+  g.args.err = solve_err_;
 }
 
 // places of the clusters' rows, one after the other
@@ -3187,10 +3238,9 @@ std::vector<int> Engine<T>::flow_places(const FlowRows& R, const std::vector<int
   return at;
 }
 
+// The dataflow programs; false where an op has too many input segments.
 template <typename T>
 bool Engine<T>::build_flow() {
-  solve_err_ = (int*)perm_.alloc(256);
-  launch_zero(stream_, 4, solve_err_, 64);
   scratch_.rewind();
   // W of every op with reflectors
   std::vector<WyJob<T>> wj;
@@ -3198,25 +3248,63 @@ bool Engine<T>::build_flow() {
   for (auto& o : ops_) {
     if (o.kind != OpOrthoD && !(square_ && (o.kind == OpQR || o.kind == OpScaleD))) continue;
     if (o.k <= 0) continue;
-    if (o.V64) {
-      double* W = (double*)perm_.alloc(sizeof(double) * (size_t)o.m * o.k);
-      o.W = W;
-      wj64.push_back(WyJob<double>{o.V64, o.Tb64, W, o.ldv, o.m, o.k});
-    } else {
-      T* W = alloc_perm((size_t)o.m * o.k);
-      o.W = W;
-      wj.push_back(WyJob<T>{o.V, o.Tb, W, o.ldv, o.m, o.k});
-    }
+    o.W = perm_.alloc((o.V64 ? sizeof(double) : sizeof(T)) * (size_t)o.m * o.k);
+    if (o.V64) wj64.push_back(WyJob<double>{o.V64, o.Tb64, (double*)o.W, o.ldv, o.m, o.k});
+    else wj.push_back(WyJob<T>{o.V, o.Tb, (T*)o.W, o.ldv, o.m, o.k});
   }
   build_w(wj);
   build_w(wj64);
-  return square_ ? build_flow_mode(0) : build_flow_ls();
+  // the programs, planned side by side while W is formed
+  const int nm = square_ ? 2 : 1;
+  const int grid = std::min(flow_capacity<T>(), 2 * num_cus_), grid64 = std::min(flow_capacity<double>(), 2 * num_cus_);
+  std::vector<FlowModePlan> plan(nm);
+  parallel_for(nm, 1, [&](int, int b, int e) {
+    for (int t = b; t < e; ++t)
+      if (square_) plan_flow_mode(t, grid, grid64, plan[t]);
+      else plan_flow_ls(grid, plan[t]);
+  });
+  for (auto& P : plan)
+    if (!P.fits()) return false;
+  int nx = 0, nx64 = 0;
+  for (int t = 0; t < nm; ++t) {
+    FlowModePlan& P = plan[t];
+    FlowMode& M = flow_mode_[t];
+    M.run.resize(P.run.size());
+    for (size_t r = 0; r < P.run.size(); ++r) flow_place<T>(P.run[r], M.run[r]);
+    if (P.run.size() > 1) flow_place<double>(P.top, M.top);
+    M.top_in = stager_.upload(perm_, P.top_in);
+    M.top_out = stager_.upload(perm_, P.top_out);
+    M.out = stager_.upload(perm_, P.out);
+    M.top_at = P.top_at;
+    M.xplaces = P.xplaces;
+    M.x64places = P.x64places;
+    flow_top_n_ = P.top_n;
+    nx = std::max(nx, P.xplaces);
+    nx64 = std::max(nx64, P.x64places);
+  }
+  flow_x_ = (T*)perm_.alloc(sizeof(T) * (size_t)std::max(nx, 1));
+  if (nx64 > 0) flow_x64_ = (double*)perm_.alloc(sizeof(double) * (size_t)nx64);
+  for (auto& M : flow_mode_) {
+    for (auto& r : M.run) r.args.x = flow_x_;
+    M.top.args.x = flow_x64_;
+  }
+  // rows and columns in cluster order (least squares: both sides are columns)
+  std::vector<int> rp, cp;
+  for (int c : bottoms_[0]) {
+    for (int i = 0; square_ && i < cl_[c].rsize_org; ++i) rp.push_back(rperm_[cl_[c].rstart + i]);
+    for (int i = 0; i < cl_[c].csize_org; ++i) cp.push_back(cperm_[cl_[c].cstart + i]);
+  }
+  flow_cperm_ = stager_.upload(perm_, cp);
+  flow_rperm_ = square_ ? stager_.upload(perm_, rp) : flow_cperm_;
+  for (auto& r : plan[0].run) solve_bytes_ += r.bytes;
+  solve_bytes_ += plan[0].top.bytes;
+  flow_ = true;
+  return true;
 }
 
-// The program of M^{-1} (t = 0), built with the factors, or of M^{-T} (1), built
-// when it is first asked for.
+// The plan of M^{-1} (t = 0) or of M^{-T} (1).
 template <typename T>
-bool Engine<T>::build_flow_mode(int t) {
+void Engine<T>::plan_flow_mode(int t, int grid, int grid64, FlowModePlan& M) const {
   std::vector<std::vector<const Op*>> by_level(nlevels_);
   for (auto& o : ops_) by_level[o.level].push_back(&o);
   // stages of the forward and the backward tape; the FP64 top apart
@@ -3291,76 +3379,55 @@ bool Engine<T>::build_flow_mode(int t) {
     return a;
   };
   const std::vector<FlowStage> first = t ? transpose(bwd) : std::move(fwd), second = t ? transpose(fwd) : std::move(bwd);
-  FlowMode& M = flow_mode_[t];
-  {
-    FlowRows R;
-    R.of.resize(cl_.size());
-    R.scratch.assign(cl_.size(), 0);
-    for (int c : bottoms_[0]) {
-      if (cl_[c].rsize_org > 0) R.of[c].push_back(FlowSeg{R.next, cl_[c].rsize_org});
-      R.next += cl_[c].rsize_org;
-    }
-    M.run.clear();
-    if (top) {
-      M.run.resize(2);
-      if (!flow_prog<T>(first, R, M.run[0])) return false;
-      const int c = top->c;
-      flow_top_n_ = top->m;
-      M.top_in = stager_.upload(perm_, flow_places(R, {c}));
-      FlowRows R64;
-      R64.of.resize(cl_.size());
-      R64.scratch.assign(cl_.size(), 0);
-      R64.of[c].push_back(FlowSeg{0, top->m});
-      R64.next = top->m;
-      std::vector<FlowStage> tf(1), tb(1);
-      tf[0].items.push_back(FlowItem{top, kFlowWY, false});
-      tb[0].items.push_back(FlowItem{top, kFlowBack, false});
-      if (!flow_prog<double>(t ? join(transpose(tb), transpose(tf)) : join(tf, tb), R64, M.top)) return false;
-      M.top_out = stager_.upload(perm_, flow_places(R64, {c}));
-      M.x64places = R64.next;
-      M.top_at = R.next;
-      R.of[c].assign(1, FlowSeg{R.next, top->m});
-      R.next += top->m;
-      if (!flow_prog<T>(second, R, M.run[1])) return false;
-    } else {
-      M.run.resize(1);
-      if (!flow_prog<T>(join(first, second), R, M.run[0])) return false;
-    }
-    M.xplaces = R.next;
-    M.out = stager_.upload(perm_, flow_places(R, bottoms_[0]));
+  FlowRows R;
+  R.of.resize(cl_.size());
+  R.scratch.assign(cl_.size(), 0);
+  for (int c : bottoms_[0]) {
+    if (cl_[c].rsize_org > 0) R.of[c].push_back(FlowSeg{R.next, cl_[c].rsize_org});
+    R.next += cl_[c].rsize_org;
   }
-  M.x = alloc_perm((size_t)M.xplaces);
-  for (auto& r : M.run) r.args.x = M.x;
-  if (top) M.top.args.x = M.x64 = (double*)perm_.alloc(sizeof(double) * (size_t)M.x64places);
-  if (t) return true;
-  std::vector<int> rp, cp;
-  for (int c : bottoms_[0])
-    for (int i = 0; i < cl_[c].rsize_org; ++i) {
-      rp.push_back(rperm_[cl_[c].rstart + i]);
-      cp.push_back(cperm_[cl_[c].cstart + i]);
-    }
-  flow_rperm_ = stager_.upload(perm_, rp);
-  flow_cperm_ = stager_.upload(perm_, cp);
-  flow_ = true;
-  return true;
+  if (top) {
+    M.run.resize(2);
+    flow_plan<T>(first, R, grid, M.run[0]);
+    const int c = top->c;
+    M.top_in = flow_places(R, {c});
+    M.top_n = top->m;
+    FlowRows R64;
+    R64.of.resize(cl_.size());
+    R64.scratch.assign(cl_.size(), 0);
+    R64.of[c].push_back(FlowSeg{0, top->m});
+    R64.next = top->m;
+    std::vector<FlowStage> tf(1), tb(1);
+    tf[0].items.push_back(FlowItem{top, kFlowWY, false});
+    tb[0].items.push_back(FlowItem{top, kFlowBack, false});
+    flow_plan<double>(t ? join(transpose(tb), transpose(tf)) : join(tf, tb), R64, grid64, M.top);
+    M.top_out = flow_places(R64, {c});
+    M.x64places = R64.next;
+    M.top_at = R.next;
+    R.of[c].assign(1, FlowSeg{R.next, top->m});
+    R.next += top->m;
+    flow_plan<T>(second, R, grid, M.run[1]);
+  } else {
+    M.run.resize(1);
+    flow_plan<T>(join(first, second), R, grid, M.run[0]);
+  }
+  M.xplaces = R.next;
+  M.out = flow_places(R, bottoms_[0]);
 }
 
 // (W^T W)^{-1} of a least-squares tree (tree.cpp:1471-1517): R^{-T} and the
 // interfaces' reflectors up the tree on xt, row permutations down and up again,
 // and the backward tape on x.  Only list entries move in the permutations.
 template <typename T>
-bool Engine<T>::build_flow_ls() {
+void Engine<T>::plan_flow_ls(int grid, FlowModePlan& M) const {
   std::vector<std::vector<const Op*>> by_level(nlevels_);
   for (auto& o : ops_) by_level[o.level].push_back(&o);
-  FlowMode& M = flow_mode_[0];
   FlowRows R;
   R.of.resize(cl_.size());
   R.scratch.assign(cl_.size(), 0);
-  std::vector<int> cp;
   for (int c : bottoms_[0]) {
     if (cl_[c].csize_org > 0) R.of[c].push_back(FlowSeg{R.next, cl_[c].csize_org});
     R.next += cl_[c].csize_org;
-    for (int i = 0; i < cl_[c].csize_org; ++i) cp.push_back(cperm_[cl_[c].cstart + i]);
   }
   R.zero = R.next;
   R.next += kFlowZeros;
@@ -3458,27 +3525,20 @@ bool Engine<T>::build_flow_ls() {
     st.push_back(std::move(qr));
   }
   M.run.resize(1);
-  if (!flow_prog<T>(st, R, M.run[0])) return false;
+  flow_plan<T>(st, R, grid, M.run[0]);
   M.xplaces = R.next;
-  std::vector<int> out;
   for (int c : bottoms_[0])
     for (const FlowSeg& sg : flow_slice(R.of[c], 0, cl_[c].csize_org))
-      for (int i = 0; i < sg.len; ++i) out.push_back(sg.off < 0 ? R.zero : sg.off + i);
-  M.out = stager_.upload(perm_, out);
-  flow_cperm_ = flow_rperm_ = stager_.upload(perm_, cp);
-  M.x = alloc_perm((size_t)M.xplaces);
-  M.run[0].args.x = M.x;
-  flow_ = true;
-  return true;
+      for (int i = 0; i < sg.len; ++i) M.out.push_back(sg.off < 0 ? R.zero : sg.off + i);
 }
 
 // Solve program: per level, forward stages QR (waves) -> ScaleD -> OrthogonalD
 // -> SplitD -> Merge, backward stages in the reverse order (tree.cpp:1440-1466).
 template <typename T>
 void Engine<T>::build_solve_program() {
-  const double bytes0 = solve_bytes_;
+  solve_err_ = (int*)perm_.alloc(256);
+  launch_zero(stream_, 4, solve_err_, 64);
   if (flow_fits() && build_flow()) return;
-  solve_bytes_ = bytes0;
   layout_x();
   // temporary segments for SplitD moves whose ranges overlap (least-squares
   // clusters with extra rows)
@@ -3987,8 +4047,6 @@ void Engine<T>::build_solve_program() {
   finish(hab, abwd_);
   n_solve_sync_ = nsync;
   solve_sync_ = (unsigned int*)perm_.alloc(sizeof(unsigned int) * std::max(nsync, 1));
-  solve_err_ = (int*)perm_.alloc(256);
-  SPQ_HIP(hipMemsetAsync(solve_err_, 0, 256, stream_));
   auto upload_stage = [&](std::vector<HStage>& hs, std::vector<Stage>& st) {
     for (size_t i = 0; i < hs.size(); ++i) {
       auto& h = hs[i];
@@ -4080,23 +4138,23 @@ void Engine<T>::run_flow(const double* b, double* x, bool transposed) {
     c.p[i] = (unsigned int*)p;
     c.n[i++] = words;
   };
-  clear(M.x + ncols_ + nz, (int64_t)(M.xplaces - ncols_ - nz) * (int64_t)(sizeof(T) / 4));
+  clear(flow_x_ + ncols_ + nz, (int64_t)(M.xplaces - ncols_ - nz) * (int64_t)(sizeof(T) / 4));
   for (auto& r : M.run) clear(r.zero, r.nzero);
   const bool top = M.run.size() > 1;
   if (top) {
-    clear(M.x64, 2 * (int64_t)M.x64places);
+    clear(flow_x64_, 2 * (int64_t)M.x64places);
     clear(M.top.zero, M.top.nzero);
   }
   // M^{-T}: b enters through the exit map and leaves through the entry map
-  launch_flow_begin<T>(stream_, transposed ? flow_cperm_ : flow_rperm_, ncols_, b, M.x, nz, c);
+  launch_flow_begin<T>(stream_, transposed ? flow_cperm_ : flow_rperm_, ncols_, b, flow_x_, nz, c);
   launch_flow<T>(stream_, M.run[0].args, M.run[0].grid);
   if (top) {
-    launch_flow_cvt<T, double>(stream_, M.top_in, flow_top_n_, M.x, M.x64, 0);
+    launch_flow_cvt<T, double>(stream_, M.top_in, flow_top_n_, flow_x_, flow_x64_, 0);
     launch_flow<double>(stream_, M.top.args, M.top.grid);
-    launch_flow_cvt<double, T>(stream_, M.top_out, flow_top_n_, M.x64, M.x, M.top_at);
+    launch_flow_cvt<double, T>(stream_, M.top_out, flow_top_n_, flow_x64_, flow_x_, M.top_at);
     launch_flow<T>(stream_, M.run[1].args, M.run[1].grid);
   }
-  launch_flow_out<T>(stream_, M.out, ncols_, M.x, transposed ? flow_rperm_ : flow_cperm_, x);
+  launch_flow_out<T>(stream_, M.out, ncols_, flow_x_, transposed ? flow_rperm_ : flow_cperm_, x);
 }
 
 template <typename T>
@@ -4228,17 +4286,6 @@ template <typename T>
 void Engine<T>::solve_t_dev(const double* b, double* x) {
   if (!factored_) throw Error(kErrState, "solve_transpose before factorize");
   if (!square_) throw Error(kErrState, "solve_transpose: rectangular (least-squares) tree");
-  if (flow_) {
-    if (flow_mode_[1].run.empty()) {
-      const double bytes = solve_bytes_;
-      flow_ = build_flow_mode(1);
-      if (!flow_) {  // an op with too many input segments: this tree's applies are staged from here on
-        flow_off_ = true;
-        build_solve_program();
-      }
-      solve_bytes_ = bytes;
-    }
-  }
   if (flow_) {
     timed("apply", 0.0, solve_bytes_, [&] { run_flow(b, x, true); });
     return;

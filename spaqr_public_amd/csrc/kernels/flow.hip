@@ -568,6 +568,7 @@ __global__ __launch_bounds__(kFNB * 8) void k_flow_diag(const FlowDiag<T>* ds, c
     d.D[(int64_t)nb * kFNB * kFNB + r] = r < d.k ? T(1) / d.R[r + (int64_t)r * d.ld] : T(0);
   }
 }
+size_t flow_diag_elems(int k) { return (size_t)((k + kFNB - 1) / kFNB) * kFNB * (kFNB + 1); }
 template <typename T>
 void launch_flow_diag(hipStream_t s, const FlowDiag<T>* d, const int* start, int nd, int nblocks) {
   if (nblocks > 0) hipLaunchKernelGGL((k_flow_diag<T>), dim3(nblocks), dim3(kFNB * 8), 0, s, d, start, nd);

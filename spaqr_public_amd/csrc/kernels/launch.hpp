@@ -129,8 +129,9 @@ template <typename T>
 int flow_capacity();
 template <typename T>
 void launch_flow(hipStream_t s, const FlowArgs<T>& a, int grid);
-// the diagonal blocks of triangular factors as k_flow reads them (flow_diag_elems
-// entries each); start: exclusive prefix sums of ceil(k / 32)
+// the diagonal blocks of triangular factors (k x k) as k_flow reads them,
+// flow_diag_elems(k) entries each; start: exclusive prefix sums of ceil(k / 32)
+size_t flow_diag_elems(int k);
 template <typename T>
 void launch_flow_diag(hipStream_t s, const FlowDiag<T>* d, const int* start, int nd, int nblocks);
 // the start of an apply: n values of b (through src, or in order) and nz zeros

@@ -339,7 +339,7 @@ int flow_one(int type, int m, int k, int par, int unit, const T* A, int lda, con
   unsigned int* ctl = dup<unsigned int>(nullptr, 64);
   int* err = dup<int>(nullptr, 64);
   if (tri) {
-    T* D = dup<T>(nullptr, (size_t)nb * 32 * 33);
+    T* D = dup<T>(nullptr, flow_diag_elems(k));
     FlowDiag<T> fd{dA, D, lda, k, type == kFlowSolveT, 0};
     const int st[2] = {0, nb};
     launch_flow_diag<T>(0, dup(&fd, 1), dup(st, 2), 1, nb);

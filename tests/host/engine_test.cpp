@@ -1,0 +1,132 @@
+// Host code of the engine against the runtime of fake_hip.hpp, where what the
+// device would read, and memory that has run out, can be looked at.  One case per
+// argument; exit code 0 and "ok" when it holds.
+#define private public
+#include "engine.cpp"
+#undef private
+#include "fake_hip.hpp"
+
+using namespace spq;
+
+// ---- launchers the cases reach
+namespace seen {
+const void* flow_x = nullptr;  // of the last apply
+int flow_begins = 0, flow_parts = 0, panel_calls = 0;
+void (*on_panel)(const RrqrDesc<double>*, int) = nullptr;
+}  // namespace seen
+namespace spq {
+void host_prof_start() {}
+int panel_nb() { return 32; }
+int refl_lds_cap(int) { return 1 << 20; }
+int bwdr_max_k() { return 1 << 20; }
+size_t flow_diag_elems(int k) { return (size_t)((k + 31) / 32) * 32 * 33; }
+template <> int flow_capacity<double>() { return 512; }
+template <> int flow_capacity<float>() { return 512; }
+void launch_zero(hipStream_t, int elem, void* p, int64_t n) { std::memset(p, 0, (size_t)elem * (size_t)n); }
+template <> void launch_flow_diag<double>(hipStream_t, const FlowDiag<double>*, const int*, int, int) {}
+template <> void launch_gemm<double>(hipStream_t, const GemmDesc<double>*, const int*, int, int) {}
+template <> void launch_flow_begin<double>(hipStream_t, const int*, int, const double*, double* x, int, const FlowClear&) {
+  CHECK(x);
+  seen::flow_x = x;
+  ++seen::flow_begins;
+}
+template <> void launch_flow<double>(hipStream_t, const FlowArgs<double>& a, int grid) {
+  CHECK(a.x == seen::flow_x && a.nparts > 0 && a.parts && a.segs && a.ctl && a.err && grid > 0);
+  seen::flow_parts = a.nparts;
+}
+template <> void launch_flow_out<double>(hipStream_t, const int* at, int n, const double* x, const int*, double*) {
+  CHECK(at && x == seen::flow_x && n > 0);
+}
+int rrqr_form(int k, int) { return k <= 704 ? 1 : 0; }
+int rrqr_form_waves(int f) { return f == 1 ? 1 : 0; }
+int rrqr_form_rows(int f) { return f == 1 ? 16 : 0; }
+int rrqr_init_tiles(int) { return 1; }
+int rrqr_update_cols() { return 16; }
+template <> void launch_rrqr_init<double>(hipStream_t, const RrqrDesc<double>* d, const int*, int nd, int) {
+  for (int q = 0; q < nd; ++q) *d[q].st = RrqrState{};
+}
+template <> void launch_rrqr_panel<double>(hipStream_t, const RrqrDesc<double>* d, int nd, int) {
+  ++seen::panel_calls;
+  if (seen::on_panel) seen::on_panel(d, nd);
+}
+template <> void launch_rrqr_update<double>(hipStream_t, const RrqrDesc<double>*, const int*, int, int, int) {}
+}  // namespace spq
+
+namespace {
+CscMat grid(int n) {  // 5-point pattern
+  CscMat A;
+  A.m = A.n = n * n;
+  A.p.push_back(0);
+  for (int j = 0; j < n * n; ++j) {
+    const int x = j % n, y = j / n;
+    for (int d : {-n, -1, 0, 1, n}) {
+      if ((d == -n && y == 0) || (d == n && y == n - 1) || (d == -1 && x == 0) || (d == 1 && x == n - 1)) continue;
+      A.i.push_back(j + d);
+      A.x.push_back(d == 0 ? 4.0 : -1.0);
+    }
+    A.p.push_back((int)A.i.size());
+  }
+  return A;
+}
+
+// a partitioned tree with the ops of an elimination of its leaves
+struct Made {
+  Engine<double> e;
+  std::vector<double> factors;
+  explicit Made(int n = 16, int nlevels = 3) : e(nlevels, 0, 0), factors(1 << 16) {
+    e.set_square(1);
+    e.set_coords(tensor_coordinates(n, 2), 2);
+    e.partition(grid(n));
+    for (int c : e.bottoms_[0]) {
+      const int k = e.cl_[c].rsize;
+      if (k <= 0) continue;
+      Engine<double>::Op o{};
+      o.kind = Engine<double>::OpQR;
+      o.level = 0;
+      o.c = c;
+      o.V = o.Tb = o.R = factors.data();
+      o.ldv = o.m = o.k = o.ldr = o.kr = k;
+      o.segs.push_back({c, k});
+      e.ops_.push_back(o);
+      e.alloc_x(c, k);
+    }
+    CHECK(!e.ops_.empty());
+  }
+  void build() {
+    e.build_solve_program();
+    e.sync();
+    e.factored_ = true;
+  }
+};
+
+// Both applies are whole once the tree is factored: neither allocates, so a
+// full device cannot leave one half built.
+void transposed() {
+  Made t;
+  t.build();
+  CHECK(t.e.flow_);
+  std::vector<double> b(t.e.nrows_, 1.0);
+  fake::dev_limit = 0;
+  t.e.perm_.cur_ = t.e.perm_.chunks_.size();  // nothing left in the arena either
+  const long before = fake::n_malloc;
+  for (int i = 0; i < 2; ++i) {
+    t.e.solve_t_dev(b.data(), b.data());
+    t.e.solve_dev(b.data(), b.data());
+  }
+  CHECK(seen::flow_begins == 4 && seen::flow_parts > 0 && fake::n_malloc == before);
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::string c = argc > 1 ? argv[1] : "";
+  try {
+    if (c == "transposed") transposed();
+    else CHECK(!"a known case");
+  } catch (const std::exception& e) {
+    std::printf("exception: %s\n", e.what());
+    return 1;
+  }
+  std::printf("ok\n");
+  std::fflush(stdout);
+  std::_Exit(0);  // the host pool's threads sleep
+}
