@@ -162,7 +162,7 @@ class Engine final : public EngineBase {
   void counters(unsigned long long* nnz4, double* d8) const override {
     nnz4[0] = nnzA_; nnz4[1] = nnzR_; nnz4[2] = nnzH_; nnz4[3] = nnzQ_;
     d8[0] = flops_; d8[1] = t_partition_; d8[2] = t_assemble_; d8[3] = t_factorize_;
-    d8[4] = top_size_; d8[5] = (double)perm_.reserved(); d8[6] = factor_bytes_; d8[7] = solve_bytes_;
+    d8[4] = top_size_; d8[5] = (double)(perm_.reserved() + flow_mem_.reserved()); d8[6] = factor_bytes_; d8[7] = solve_bytes_;
   }
 
  private:
@@ -901,6 +901,7 @@ class Engine final : public EngineBase {
   }
   bool flow_fits() const;
   bool build_flow();
+  bool make_flow();
   template <typename U>
   void build_w(const std::vector<WyJob<U>>& jobs);
   template <typename U>
@@ -934,6 +935,7 @@ class Engine final : public EngineBase {
   void plan_flow_mode(int t, int grid, int grid64, FlowModePlan& P) const;
   void plan_flow_ls(int grid, FlowModePlan& P) const;
   bool flow_ = false;  // applies run the dataflow programs
+  Arena flow_mem_{size_t(64) << 20};  // W and the programs; given back where the staged program takes over
   FlowMode flow_mode_[2];
   T* flow_x_ = nullptr;
   double* flow_x64_ = nullptr;
@@ -3205,8 +3207,8 @@ template <typename U>
 void Engine<T>::flow_place(FlowPlan<U>& p, FlowProg<U>& g) {
   const size_t slot_words = p.slots * sizeof(U) / 4;
   g.nzero = (int64_t)(slot_words + 64);
-  g.zero = (unsigned int*)perm_.alloc(4 * (size_t)g.nzero);
-  U* const D = (U*)perm_.alloc(sizeof(U) * (size_t)p.diag_elems);
+  g.zero = (unsigned int*)flow_mem_.alloc(4 * (size_t)g.nzero);
+  U* const D = (U*)flow_mem_.alloc(sizeof(U) * (size_t)p.diag_elems);
   for (size_t i = 0; i < p.parts.size(); ++i) {
     if (p.parts[i].nwg > 1) p.parts[i].slots = (U*)g.zero + p.slot_at[i];
     if (p.diag_at[i] >= 0) p.parts[i].B = D + p.diag_at[i];
@@ -3221,9 +3223,9 @@ void Engine<T>::flow_place(FlowPlan<U>& p, FlowProg<U>& g) {
   const FlowDiag<U>* dd = stager_.push(p.diags);
   const int* ds = stager_.push(p.diag_start);
   timed("wy", 0.0, 0.0, [&] { launch_flow_diag<U>(stream_, dd, ds, (int)p.diags.size(), p.diag_start.back()); });
-  g.args.parts = stager_.upload(perm_, p.parts);
-  g.args.segs = stager_.upload(perm_, p.segs);
-  g.args.blks = stager_.upload(perm_, p.blks);
+  g.args.parts = stager_.upload(flow_mem_, p.parts);
+  g.args.segs = stager_.upload(flow_mem_, p.segs);
+  g.args.blks = stager_.upload(flow_mem_, p.blks);
   g.args.ctl = g.zero + slot_words;
   g.args.err = solve_err_;
 }
@@ -3238,9 +3240,27 @@ std::vector<int> Engine<T>::flow_places(const FlowRows& R, const std::vector<int
   return at;
 }
 
-// The dataflow programs; false where an op has too many input segments.
+// The dataflow programs, or false where the staged one has to take over: an op
+// with too many input segments, or no memory for a second copy of the
+// reflectors.  Then nothing of them stays.
 template <typename T>
 bool Engine<T>::build_flow() {
+  try {
+    flow_ = make_flow();
+  } catch (const Error& e) {
+    if (e.code != kErrOom) throw;
+    (void)hipGetLastError();
+  }
+  if (flow_) return true;
+  sync();  // the memory goes to the pool
+  for (auto& o : ops_) o.W = nullptr;
+  for (auto& M : flow_mode_) M = FlowMode{};
+  flow_mem_.release();
+  return false;
+}
+
+template <typename T>
+bool Engine<T>::make_flow() {
   scratch_.rewind();
   // W of every op with reflectors
   std::vector<WyJob<T>> wj;
@@ -3248,7 +3268,7 @@ bool Engine<T>::build_flow() {
   for (auto& o : ops_) {
     if (o.kind != OpOrthoD && !(square_ && (o.kind == OpQR || o.kind == OpScaleD))) continue;
     if (o.k <= 0) continue;
-    o.W = perm_.alloc((o.V64 ? sizeof(double) : sizeof(T)) * (size_t)o.m * o.k);
+    o.W = flow_mem_.alloc((o.V64 ? sizeof(double) : sizeof(T)) * (size_t)o.m * o.k);
     if (o.V64) wj64.push_back(WyJob<double>{o.V64, o.Tb64, (double*)o.W, o.ldv, o.m, o.k});
     else wj.push_back(WyJob<T>{o.V, o.Tb, (T*)o.W, o.ldv, o.m, o.k});
   }
@@ -3272,9 +3292,9 @@ bool Engine<T>::build_flow() {
     M.run.resize(P.run.size());
     for (size_t r = 0; r < P.run.size(); ++r) flow_place<T>(P.run[r], M.run[r]);
     if (P.run.size() > 1) flow_place<double>(P.top, M.top);
-    M.top_in = stager_.upload(perm_, P.top_in);
-    M.top_out = stager_.upload(perm_, P.top_out);
-    M.out = stager_.upload(perm_, P.out);
+    M.top_in = stager_.upload(flow_mem_, P.top_in);
+    M.top_out = stager_.upload(flow_mem_, P.top_out);
+    M.out = stager_.upload(flow_mem_, P.out);
     M.top_at = P.top_at;
     M.xplaces = P.xplaces;
     M.x64places = P.x64places;
@@ -3282,8 +3302,8 @@ bool Engine<T>::build_flow() {
     nx = std::max(nx, P.xplaces);
     nx64 = std::max(nx64, P.x64places);
   }
-  flow_x_ = (T*)perm_.alloc(sizeof(T) * (size_t)std::max(nx, 1));
-  if (nx64 > 0) flow_x64_ = (double*)perm_.alloc(sizeof(double) * (size_t)nx64);
+  flow_x_ = (T*)flow_mem_.alloc(sizeof(T) * (size_t)std::max(nx, 1));
+  if (nx64 > 0) flow_x64_ = (double*)flow_mem_.alloc(sizeof(double) * (size_t)nx64);
   for (auto& M : flow_mode_) {
     for (auto& r : M.run) r.args.x = flow_x_;
     M.top.args.x = flow_x64_;
@@ -3294,11 +3314,10 @@ bool Engine<T>::build_flow() {
     for (int i = 0; square_ && i < cl_[c].rsize_org; ++i) rp.push_back(rperm_[cl_[c].rstart + i]);
     for (int i = 0; i < cl_[c].csize_org; ++i) cp.push_back(cperm_[cl_[c].cstart + i]);
   }
-  flow_cperm_ = stager_.upload(perm_, cp);
-  flow_rperm_ = square_ ? stager_.upload(perm_, rp) : flow_cperm_;
+  flow_cperm_ = stager_.upload(flow_mem_, cp);
+  flow_rperm_ = square_ ? stager_.upload(flow_mem_, rp) : flow_cperm_;
   for (auto& r : plan[0].run) solve_bytes_ += r.bytes;
   solve_bytes_ += plan[0].top.bytes;
-  flow_ = true;
   return true;
 }
 

@@ -19,6 +19,10 @@ void host_prof_start() {}
 int panel_nb() { return 32; }
 int refl_lds_cap(int) { return 1 << 20; }
 int bwdr_max_k() { return 1 << 20; }
+int reflr_rows() { return 448; }
+int r12_chunk_cols() { return 64; }
+int reflr_row_waves(int) { return 7; }
+size_t reflr_lds(int) { return 0; }
 size_t flow_diag_elems(int k) { return (size_t)((k + 31) / 32) * 32 * 33; }
 template <> int flow_capacity<double>() { return 512; }
 template <> int flow_capacity<float>() { return 512; }
@@ -107,7 +111,8 @@ void transposed() {
   CHECK(t.e.flow_);
   std::vector<double> b(t.e.nrows_, 1.0);
   fake::dev_limit = 0;
-  t.e.perm_.cur_ = t.e.perm_.chunks_.size();  // nothing left in the arena either
+  t.e.perm_.cur_ = t.e.perm_.chunks_.size();  // nothing left in the arenas either
+  t.e.flow_mem_.cur_ = t.e.flow_mem_.chunks_.size();
   const long before = fake::n_malloc;
   for (int i = 0; i < 2; ++i) {
     t.e.solve_t_dev(b.data(), b.data());
@@ -115,12 +120,45 @@ void transposed() {
   }
   CHECK(seen::flow_begins == 4 && seen::flow_parts > 0 && fake::n_malloc == before);
 }
+
+// Where the staged program takes over, nothing of the dataflow programs stays.
+void staged(Made& t) {
+  t.build();
+  CHECK(!t.e.flow_ && t.e.flow_mem_.reserved() == 0 && t.e.xbuf_ && t.e.bin_ && !t.e.fwd_.empty());
+  for (auto& o : t.e.ops_) CHECK(!o.W);
+  for (auto& m : t.e.flow_mode_) CHECK(m.run.empty());
+  CHECK(hipGetLastError() == hipSuccess);  // no launch check finds a handled failure
+}
+void segments() {
+  Made t;
+  auto& o = t.e.ops_.back();  // one input segment more than the kernel takes
+  o.segs.assign(kFlowMaxSegs + 1, {o.c, 1});
+  o.m = o.ldv = kFlowMaxSegs + 1;
+  o.k = o.kr = 1;
+  staged(t);
+}
+// no memory for the first, or for a later part of a second copy of the reflectors
+void no_memory() {
+  for (size_t room : {size_t(32) << 20, size_t(96) << 20}) {
+    Made t;
+    auto o = t.e.ops_[0];
+    o.m = o.ldv = 3000;
+    o.k = o.kr = o.ldr = 1000;
+    for (int i = 0; i < 3; ++i) t.e.ops_.push_back(o);  // 24 MB each
+    t.e.scratch_.alloc(1);
+    fake::dev_limit = fake::dev_used + room;
+    staged(t);
+    fake::dev_limit = ~size_t(0);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::string c = argc > 1 ? argv[1] : "";
   try {
     if (c == "transposed") transposed();
+    else if (c == "segments") segments();
+    else if (c == "no_memory") no_memory();
     else CHECK(!"a known case");
   } catch (const std::exception& e) {
     std::printf("exception: %s\n", e.what());

@@ -34,7 +34,7 @@ def engine_test(tmp_path_factory):
     return exe
 
 
-CASES = ["transposed"]
+CASES = ["transposed", "segments", "no_memory"]
 
 
 @pytest.mark.parametrize("case", CASES)
