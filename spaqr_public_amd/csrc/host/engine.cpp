@@ -307,10 +307,14 @@ class Engine final : public EngineBase {
   }
   void sync() {
     stager_.flush_uploads();
+    wait();
+    stager_.reset();
+  }
+  // the stream alone: tables pushed so far stay valid
+  void wait() {
     const double a = wall();
     SPQ_HIP(hipStreamSynchronize(stream_));
     t_wait_ += wall() - a;
-    stager_.reset();
   }
   double t_wait_ = 0;  // host time blocked in stream synchronisations (diagnostics)
   double t_flush_ = 0, t_launch_ = 0;  // host time in descriptor uploads / launch calls (verbose > 1)
@@ -1729,7 +1733,9 @@ void Engine<T>::rrqr_blocked(std::vector<RrqrJob>& jobs) {
       timed("rrqr_upd", 0.0, 2 * by, [&] { launch_rrqr_update<T>(stream_, dd, dus, nd, nut, kmax); });
     }
     SPQ_HIP(hipMemcpyAsync(hs, st, sizeof(RrqrState) * nj, hipMemcpyDeviceToHost, stream_));
-    sync();
+    // not sync(): further rounds read the tables, which may lie in a ring that
+    // the stager has outgrown since and would give away
+    wait();
     bool all = true;
     for (size_t q = 0; q < nj && all; ++q) all = hs[q].done != 0;
     if (all) break;
@@ -1737,6 +1743,7 @@ void Engine<T>::rrqr_blocked(std::vector<RrqrJob>& jobs) {
     if (queued > kmax) throw Error(kErrNumeric, "rrqr: a round made no progress");
     rounds = 2;
   }
+  stager_.reset();
   for (size_t q = 0; q < nj; ++q) jobs[q].rank = hs[q].next;
   if (kprof_)
     for (size_t q = 0; q < nj; ++q) {

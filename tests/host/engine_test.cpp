@@ -151,6 +151,38 @@ void no_memory() {
     fake::dev_limit = ~size_t(0);
   }
 }
+
+// RRQR rounds after a read-back read the tables of the first ones, also when the
+// staging ring was outgrown between two of them and another tree takes what the
+// pool has to give.
+void rrqr_ring() {
+  Engine<double> e(3, 0, 0);
+  e.set_tol(1e-2);
+  const int k = 20, N = 300, nj = 3;
+  std::vector<double> C((size_t)k * N);
+  std::vector<Engine<double>::RrqrJob> jobs(nj);
+  for (auto& j : jobs) { j.Ct = C.data(); j.k = k; j.N = N; }
+  // room for the descriptors, not for the next table
+  const size_t room = (sizeof(RrqrDesc<double>) * nj + 255) / 256 * 256;
+  std::vector<char> fill(e.stager_.cap_ - e.stager_.off_ - room);
+  e.stager_.push_raw(fill.data(), fill.size());
+  seen::on_panel = [](const RrqrDesc<double>* d, int nd) {
+    for (const long have = fake::n_malloc; fake::n_malloc == have;) {  // all that is pooled
+      size_t bytes = 1;
+      char* p = pool_take(false, bytes, true);
+      std::memset(p, 0xee, bytes);
+    }
+    CHECK(nd == 3);
+    for (int q = 0; q < nd; ++q) {
+      CHECK(d[q].k == 20 && d[q].N == 300 && d[q].ldc == 300);
+      // the fourth round of two times two ends it
+      if (seen::panel_calls == 4) *d[q].st = RrqrState{6, 1, 7, 1, 1.0};
+    }
+  };
+  e.rrqr_blocked(jobs);
+  CHECK(seen::panel_calls == 4 && e.stager_.n_grow == 1 && e.stager_.retired_.empty());
+  for (auto& j : jobs) CHECK(j.rank == 7);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -159,6 +191,7 @@ int main(int argc, char** argv) {
     if (c == "transposed") transposed();
     else if (c == "segments") segments();
     else if (c == "no_memory") no_memory();
+    else if (c == "rrqr_ring") rrqr_ring();
     else CHECK(!"a known case");
   } catch (const std::exception& e) {
     std::printf("exception: %s\n", e.what());
