@@ -116,7 +116,11 @@ class Engine final : public EngineBase {
     int e = 0;
     SPQ_HIP(hipMemcpyAsync(&e, solve_err_, sizeof(int), hipMemcpyDeviceToHost, stream_));
     SPQ_HIP(hipStreamSynchronize(stream_));
-    if (e) throw Error(kErrNumeric, "solve: an inter-workgroup barrier wait timed out");
+    if (!e) return;
+    // the flag is of this call: the next one's waits would give up under it
+    launch_zero(stream_, 4, solve_err_, 64);
+    SPQ_HIP(hipStreamSynchronize(stream_));
+    throw Error(kErrNumeric, "solve: an inter-workgroup barrier wait timed out");
   }
   void reset_kernel_stats() override {
     SPQ_HIP(hipStreamSynchronize(stream_));

@@ -183,6 +183,23 @@ void rrqr_ring() {
   CHECK(seen::panel_calls == 4 && e.stager_.n_grow == 1 && e.stager_.retired_.empty());
   for (auto& j : jobs) CHECK(j.rank == 7);
 }
+
+// A wait that timed out is reported once; later applies start without it.
+void timeout() {
+  Made t;
+  t.build();
+  std::vector<double> b(t.e.nrows_, 1.0);
+  *t.e.solve_err_ = 1;
+  bool thrown = false;
+  try {
+    t.e.check_solve();
+  } catch (const Error& e) {
+    thrown = e.code == kErrNumeric;
+  }
+  CHECK(thrown && *t.e.solve_err_ == 0);
+  t.e.solve_dev(b.data(), b.data());
+  t.e.check_solve();
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -192,6 +209,7 @@ int main(int argc, char** argv) {
     else if (c == "segments") segments();
     else if (c == "no_memory") no_memory();
     else if (c == "rrqr_ring") rrqr_ring();
+    else if (c == "timeout") timeout();
     else CHECK(!"a known case");
   } catch (const std::exception& e) {
     std::printf("exception: %s\n", e.what());
