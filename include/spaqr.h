@@ -44,6 +44,12 @@ const char* spaqr_last_error(void);
 spaqr_tree* spaqr_tree_create(int nlevels, int skip, int precision, int device);
 /* ~Tree()                                                  tree.h:150     */
 void spaqr_tree_destroy(spaqr_tree* t);
+/* No counterpart in the reference.  Destroyed trees leave their memory in a
+ * process-wide pool for the next ones: at most 8 GiB of device and 2 GiB of
+ * pinned memory per device, emptied by itself only when an allocation of this
+ * library finds no device memory left.  This gives back all that no tree is
+ * using, for other libraries of the process.  Any thread, any time.        */
+int spaqr_pool_trim(void);
 
 /* Tree::set_tol / set_skip / set_scale / set_square / set_order / set_hsl
  *                                                          tree.cpp:14-19 */

@@ -41,7 +41,7 @@ SYMBOLS = [
     "spaqr_kernel_stats_reset", "spaqr_solve_nrml_device", "spaqr_cgls", "spaqr_cgls_device",
     "spaqr_solve_transpose", "spaqr_solve_transpose_device", "spaqr_gmres_transpose_device",
     "spaqr_csc_outer_device", "spaqr_num_extra_sparsified", "spaqr_extra_sparsified", "spaqr_profile_json",
-    "spaqr_gmres_device_noalloc", "spaqr_set_row_parts", "spaqr_row_parts",
+    "spaqr_gmres_device_noalloc", "spaqr_set_row_parts", "spaqr_row_parts", "spaqr_pool_trim",
 ]
 
 
@@ -146,6 +146,13 @@ def random_vec(n, seed=2021):
 def default_levels(ncols):
     """spaQR.cpp:111 (integer division inside the log)."""
     return int(math.ceil(math.log2(ncols // 64)))
+
+
+def pool_trim():
+    """Gives back the memory that closed trees left for the next ones (at most
+    8 GiB of device and 2 GiB of pinned memory), for other libraries of the
+    process; the pool fills again as trees are closed."""
+    _check(load_library().spaqr_pool_trim(), "pool_trim")
 
 
 class Tree:

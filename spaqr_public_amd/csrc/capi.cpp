@@ -58,6 +58,7 @@ spaqr_tree* spaqr_tree_create(int nlevels, int skip, int precision, int device) 
   return t;
 }
 void spaqr_tree_destroy(spaqr_tree* t) { delete t; }
+int spaqr_pool_trim(void) { return guard([] { pool_trim(); }); }
 
 int spaqr_set_tol(spaqr_tree* t, double v) { return guard([&] { eng(t).set_tol(v); }); }
 int spaqr_set_skip(spaqr_tree* t, int v) { return guard([&] { eng(t).set_skip(v); }); }

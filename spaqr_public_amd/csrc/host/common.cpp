@@ -63,8 +63,8 @@ void Arena::release() {
 
 namespace {
 struct PoolEntry { int dev; bool host; size_t bytes; char* p; };
-// kept per device: pinned host memory, and device memory (the arenas of a
-// tree of a million unknowns; 3% of the device's)
+// kept per device: device memory (the arenas of a tree of a million unknowns; 3%
+// of the device's), and pinned host memory
 constexpr size_t kPoolBytes[2] = {size_t(8) << 30, size_t(2) << 30};
 constexpr size_t kPoolStreams = 16;
 std::mutex& pool_mu() {
@@ -128,6 +128,18 @@ hipError_t dev_malloc(void** p, size_t bytes) {
   (void)hipGetLastError();
   for (auto& d : drop) (void)hipFree(d.p);
   return hipMalloc(p, bytes);
+}
+
+void pool_trim() {
+  std::vector<PoolEntry> drop;
+  {
+    std::lock_guard<std::mutex> lk(pool_mu());
+    drop.swap(pool());
+  }
+  for (auto& e : drop) {
+    if (e.host) host_free(e.p);
+    else dev_free(e.p);
+  }
 }
 
 namespace {

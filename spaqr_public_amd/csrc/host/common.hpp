@@ -121,12 +121,14 @@ class Arena {
 // else a new one) and sets `bytes` to its size; pool_give returns it to the pool of device `dev` (the device
 // current when it was taken; the caller's stream work on it must be
 // complete).  At most 8 GiB of device and 2 GiB of pinned memory per device stay
-// pooled, and none of it once an allocation finds no memory left.  A tree of a
+// pooled, no device memory once an allocation here finds none left, and nothing
+// after pool_trim (other libraries of the process cannot make it leave).  A tree of a
 // small problem spent a fifth of its life in hipMalloc and hipFree (2-D 40^2:
 // 1.0 of 4.7 ms), and after some hundred trees in a process the driver made
 // single allocations wait for 20 ms to seconds.
 char* pool_take(bool host, size_t& bytes, bool largest = false);
 void pool_give(bool host, char* p, size_t bytes, int dev);
+void pool_trim();
 // The same for streams (default priority, non-blocking, idle when given back;
 // at most 16 per device are kept).
 hipStream_t stream_take();

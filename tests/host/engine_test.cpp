@@ -200,6 +200,26 @@ void timeout() {
   t.e.solve_dev(b.data(), b.data());
   t.e.check_solve();
 }
+
+// Memory of closed trees stays for the next ones, and leaves when asked to.
+void trim() {
+  { Made t; t.build(); }
+  const size_t kept = fake::dev_used;
+  CHECK(kept > 0 && !fake::pinned.empty());
+  const long n = fake::n_malloc;
+  { Made t; t.build(); }
+  CHECK(fake::n_malloc == n && fake::dev_used == kept);
+  Made alive;
+  alive.build();
+  pool_trim();
+  std::vector<double> b(alive.e.nrows_, 1.0);
+  alive.e.solve_dev(b.data(), b.data());  // what a tree uses is not pooled
+  CHECK(fake::dev_used == kept);
+  { Made other; other.build(); }
+  CHECK(fake::dev_used > kept);
+  pool_trim();
+  CHECK(fake::dev_used == kept);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -210,6 +230,7 @@ int main(int argc, char** argv) {
     else if (c == "no_memory") no_memory();
     else if (c == "rrqr_ring") rrqr_ring();
     else if (c == "timeout") timeout();
+    else if (c == "trim") trim();
     else CHECK(!"a known case");
   } catch (const std::exception& e) {
     std::printf("exception: %s\n", e.what());
