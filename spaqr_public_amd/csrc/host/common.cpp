@@ -169,7 +169,12 @@ hipStream_t stream_take() {
 
 void stream_give(hipStream_t s, int dev) {
   if (!s) return;
-  {
+  // a capture that an error left open, or an error on the stream, must not
+  // reach the next tree
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  const bool idle = hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone &&
+                    hipStreamSynchronize(s) == hipSuccess;
+  if (idle) {
     std::lock_guard<std::mutex> lk(pool_mu());
     auto& v = stream_pool();
     size_t n = 0;

@@ -129,8 +129,8 @@ class Arena {
 char* pool_take(bool host, size_t& bytes, bool largest = false);
 void pool_give(bool host, char* p, size_t bytes, int dev);
 void pool_trim();
-// The same for streams (default priority, non-blocking, idle when given back;
-// at most 16 per device are kept).
+// The same for streams (default priority, non-blocking; at most 16 idle ones per
+// device are kept).
 hipStream_t stream_take();
 void stream_give(hipStream_t s, int dev);
 

@@ -220,6 +220,16 @@ void trim() {
   pool_trim();
   CHECK(fake::dev_used == kept);
 }
+
+// A stream that an error left in a capture does not go to the next tree.
+void stream() {
+  hipStream_t s;
+  { Made t; s = t.e.stream_; }
+  { Made t; CHECK(t.e.stream_ == s); fake::capturing.insert(s); }
+  CHECK(!fake::streams.count(s));
+  Made t;
+  CHECK(!fake::capturing.count(t.e.stream_));
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -231,6 +241,7 @@ int main(int argc, char** argv) {
     else if (c == "rrqr_ring") rrqr_ring();
     else if (c == "timeout") timeout();
     else if (c == "trim") trim();
+    else if (c == "stream") stream();
     else CHECK(!"a known case");
   } catch (const std::exception& e) {
     std::printf("exception: %s\n", e.what());

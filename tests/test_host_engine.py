@@ -34,7 +34,7 @@ def engine_test(tmp_path_factory):
     return exe
 
 
-CASES = ["transposed", "segments", "no_memory", "rrqr_ring", "timeout", "trim"]
+CASES = ["transposed", "segments", "no_memory", "rrqr_ring", "timeout", "trim", "stream"]
 
 
 @pytest.mark.parametrize("case", CASES)
