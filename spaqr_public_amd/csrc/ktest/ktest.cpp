@@ -22,17 +22,23 @@ thread_local std::string g_err;
     if (e_ != hipSuccess) { g_err = hipGetErrorString(e_); return -1; } \
   } while (0)
 
+// n elements on the device: the `given` of them that the caller's array has, then
+// zeros
 template <typename X>
-X* dup(const X* h, size_t n) {
+X* dup(const X* h, size_t n, size_t given) {
   X* d = nullptr;
   if (hipMalloc((void**)&d, sizeof(X) * (n ? n : 1)) != hipSuccess) return nullptr;
-  if (h && n) (void)hipMemcpy(d, h, sizeof(X) * n, hipMemcpyHostToDevice);
-  else (void)hipMemset(d, 0, sizeof(X) * (n ? n : 1));
+  if (!h || given < std::max(n, size_t(1))) (void)hipMemset(d, 0, sizeof(X) * (n ? n : 1));
+  if (h && given) (void)hipMemcpy(d, h, sizeof(X) * given, hipMemcpyHostToDevice);
   return d;
 }
 template <typename X>
+X* dup(const X* h, size_t n) {
+  return dup(h, n, n);
+}
+template <typename X>
 void back(X* h, const X* d, size_t n) {
-  (void)hipMemcpy(h, d, sizeof(X) * n, hipMemcpyDeviceToHost);
+  if (n) (void)hipMemcpy(h, d, sizeof(X) * n, hipMemcpyDeviceToHost);
 }
 }  // namespace
 
@@ -109,7 +115,7 @@ int ktest_smin(int k, const double* R, int ld, double* out) {
 int ktest_qr(int m, int k, double* A, double* tau, double* Tb, int nc, double* Cm) {
   const int nb = panel_nb(), kk = m < k ? m : k, nblk = (k + nb - 1) / nb;
   double *dA = dup(A, (size_t)m * k), *dt = dup<double>(nullptr, k), *dT = dup<double>(nullptr, (size_t)nb * nb * nblk);
-  double* dC = dup(Cm, (size_t)m * (nc > 0 ? nc : 1));
+  double* dC = dup(Cm, (size_t)m * (nc > 0 ? nc : 1), (size_t)m * nc);
   int zero = 0;
   int* ds = dup(&zero, 1);
   int* err = dup<int>(nullptr, 1);
@@ -242,7 +248,7 @@ int rrqr_one(int k, int N, X* Ct, X* V, X* tau, double tol, int nd, int* perm, i
   if (!form || k < 1 || N < 0) { g_err = "k beyond the blocked form"; return -1; }
   const size_t n1 = std::max(N, 1);
   const int ldv = k + kRrqrPivots - 1, kr = k + 15;  // V by rows, padded
-  X *dC = dup(Ct, n1 * k), *dV = dup<X>(nullptr, (size_t)kr * ldv), *dt = dup<X>(nullptr, k);
+  X *dC = dup(Ct, n1 * k, (size_t)N * k), *dV = dup<X>(nullptr, (size_t)kr * ldv), *dt = dup<X>(nullptr, k);
   double* tm = dup<double>(nullptr, kRrqrPivots * kRrqrPivots);
   double* vn = dup<double>(nullptr, n1);
   int *ip = dup<int>(nullptr, n1), *pm = dup<int>(nullptr, n1);
@@ -262,7 +268,7 @@ int rrqr_one(int k, int N, X* Ct, X* V, X* tau, double tol, int nd, int* perm, i
     if (h.done) break;
   }
   std::vector<X> hv((size_t)kr * ldv);
-  back(Ct, dC, n1 * k);
+  back(Ct, dC, (size_t)N * k);
   back(hv.data(), dV, hv.size());
   for (int c = 0; c < k; ++c)
     for (int i = 0; i < k; ++i) V[i + (size_t)c * k] = hv[(size_t)i * ldv + c];
@@ -499,7 +505,7 @@ int ktest_refl(int m, int k, const double* V, const double* Tb, double* x, int t
 // xs <- R^{-1}(xs - A1 x1) (trans=0) ; or xs <- R^{-T} xs, x1 -= A1^T xs (trans=1)
 // form 1: the latency form (one workgroup, no R12 products: s must be 0)
 int ktest_bwd(int k, const double* R, int s, const double* A1, double* xs, double* x1, int trans, int form) {
-  double *dR = dup(R, (size_t)k * k), *dA = dup(A1, (size_t)k * (s > 0 ? s : 1));
+  double *dR = dup(R, (size_t)k * k), *dA = dup(A1, (size_t)k * (s > 0 ? s : 1), (size_t)k * s);
   std::vector<double> xb((size_t)k + s);
   std::memcpy(xb.data(), xs, sizeof(double) * k);
   if (s > 0) std::memcpy(xb.data() + k, x1, sizeof(double) * s);
