@@ -813,9 +813,12 @@ class Engine final : public EngineBase {
     bool byrows = false;
     T* tau = nullptr;
   };
+  void rrqr_batch(std::vector<RrqrJob>& jobs);
   // rc_force > 0: rows per lane of the register form (the autotuner's trial
   // runs); else the tuned or closed-form choice
-  void rrqr_batch(std::vector<RrqrJob>& jobs, int rc_force = 0);
+  void rrqr_columns(std::vector<RrqrJob>& jobs, int rc_force = 0);
+  static std::string rrqr_key(const std::vector<RrqrJob>& jobs);
+  void rrqr_tune(const std::vector<RrqrJob>& jobs, const std::string& key, bool blocked);
   void rrqr_blocked(std::vector<RrqrJob>& jobs);
   // the first `rank` reflectors of a job as columns (ld k)
   static CopyDesc rrqr_v_copy(const RrqrJob& j, T* V, int rank) {
@@ -1708,7 +1711,7 @@ void Engine<T>::rrqr_blocked(std::vector<RrqrJob>& jobs) {
     ucnt[q] = iceil(std::max(jb.N, 1), utile);
     by += (double)sizeof(T) * jb.k * jb.N;
     const int kk = std::min(jb.k, jb.N);
-    flops_ += 4.0 * jb.k * jb.N * kk - 2.0 * (jb.k + jb.N) * kk * kk + 4.0 / 3.0 * kk * kk * kk;
+    if (!trial_) flops_ += 4.0 * jb.k * jb.N * kk - 2.0 * (jb.k + jb.N) * kk * kk + 4.0 / 3.0 * kk * kk * kk;
   }
   const int nit = prefix_tiles(icnt, ist), nut = prefix_tiles(ucnt, ust);
   const RrqrDesc<T>* dd = stager_.push(qd);
@@ -1758,28 +1761,89 @@ void Engine<T>::rrqr_blocked(std::vector<RrqrJob>& jobs) {
 
 // Truncated column-pivoted QR (the geqp3 + choose_rank of util.cpp:466-477,
 // 795-816) of a batch of independent problems whose transposed inputs Ct
-// (N x k, ld N) are already gathered.  Per problem: the register form when its
-// columns fit the resident workgroups, else the streaming form; single-
-// workgroup problems in plain launches, multi-workgroup ones cooperatively
-// within the resident capacity.  Fills rank, V (k x k, ld k) and tau; on
-// exit Ct(0:rank, j) = triu(R(0:rank,:)) P^T for every column j.
+// (N x k, ld N) are already gathered.  Fills rank, V (reflectors as columns of
+// k x k, or by rows) and tau; on exit Ct(0:rank, j) = triu(R(0:rank,:)) P^T for
+// every column j.  The blocked form takes every problem whose rows one panel
+// workgroup holds, unless the tuner's file has timed the two forms on such a
+// batch and found a column-by-column one faster; those take the larger
+// problems and what is asked for by name.
 template <typename T>
-void Engine<T>::rrqr_batch(std::vector<RrqrJob>& jobs, int rc_force) {
-  if (jobs.empty()) return;
-  // the blocked form takes every problem whose rows one panel workgroup
-  // holds; the column-by-column forms below keep the larger ones, the
-  // autotuner's trials and the forms asked for by name
-  if (rc_force == 0 && qp3_rc_ == 0 && qp3_reg_ && tol_ < 1.0 && !global_tuner().tuning()) {
-    std::vector<RrqrJob> blk, rest;
-    for (auto& j : jobs) (rrqr_form(j.k, 1) ? blk : rest).push_back(j);
-    if (!blk.empty()) {
-      rrqr_blocked(blk);
-      if (!rest.empty()) rrqr_batch(rest);
-      size_t b = 0, r = 0;
-      for (auto& j : jobs) j = rrqr_form(j.k, 1) ? blk[b++] : rest[r++];
-      return;
-    }
+void Engine<T>::rrqr_batch(std::vector<RrqrJob>& jobs) {
+  if (qp3_rc_ > 0 || !qp3_reg_ || !(tol_ < 1.0)) {
+    rrqr_columns(jobs);
+    return;
   }
+  std::vector<RrqrJob> blk, rest;
+  for (auto& j : jobs) (rrqr_form(j.k, 1) ? blk : rest).push_back(j);
+  if (!blk.empty()) {
+    Tuner& tu = global_tuner();
+    const std::string key = rrqr_key(blk);
+    if (tu.tuning() && tu.prefers_register(key) < 0) rrqr_tune(blk, key, true);
+    if (tu.prefers_register(key) == 1) rrqr_columns(blk);
+    else rrqr_blocked(blk);
+  }
+  rrqr_columns(rest);
+  size_t b = 0, r = 0;
+  for (auto& j : jobs) j = rrqr_form(j.k, 1) ? blk[b++] : rest[r++];
+}
+
+template <typename T>
+std::string Engine<T>::rrqr_key(const std::vector<RrqrJob>& jobs) {
+  int kmax = 0, nmax = 0;
+  for (auto& j : jobs) { kmax = std::max(kmax, j.k); nmax = std::max(nmax, j.N); }
+  char key[96];
+  snprintf(key, sizeof key, "qp3r/%s/k%d/n%d/p%d", sizeof(T) == 8 ? "f64" : "f32", log2_bucket(kmax), log2_bucket(nmax),
+           log2_bucket((long)jobs.size()));
+  return key;
+}
+
+// Times every register form, and the blocked one, on copies of the batch's
+// inputs (the RRQR works in place) and records them.
+template <typename T>
+void Engine<T>::rrqr_tune(const std::vector<RrqrJob>& jobs, const std::string& key, bool blocked) {
+  std::vector<std::pair<int, double>> ms;
+  double best_ms = -1, blocked_ms = -1;
+  int rc = 0;
+  std::vector<int> forms;  // 0: blocked
+  for (int r : qp3r_rcs())
+    if (qp3r_cap(256, r) > 0) forms.push_back(r);
+  if (blocked) forms.push_back(0);
+  for (int r : forms) {
+    std::vector<RrqrJob> trial;
+    std::vector<CopyDesc> cp;
+    for (auto& j : jobs) {
+      RrqrJob t{alloc_scr((size_t)std::max(j.N, 1) * j.k), j.k, j.N};
+      cp.push_back(CopyDesc{j.Ct, t.Ct, std::max(j.N, 1), std::max(j.N, 1), j.N, j.k, 0, 0});
+      trial.push_back(t);
+    }
+    const bool kp = kprof_;
+    kprof_ = false;
+    copy_blocks(cp);
+    sync();
+    const double t0 = wall();
+    trial_ = true;
+    if (r) rrqr_columns(trial, r);
+    else rrqr_blocked(trial);
+    trial_ = false;
+    const double t1 = 1e3 * (wall() - t0);
+    kprof_ = kp;
+    if (r == 0) {
+      blocked_ms = t1;
+      continue;
+    }
+    ms.push_back({r, t1});
+    if (best_ms < 0 || t1 < best_ms) { best_ms = t1; rc = r; }
+  }
+  if (rc > 0) global_tuner().record(key, rc, ms, blocked_ms);
+}
+
+// The column-by-column forms.  Per problem: the register form when its columns
+// fit the resident workgroups, else the streaming form; single-workgroup
+// problems in plain launches, multi-workgroup ones cooperatively within the
+// resident capacity.
+template <typename T>
+void Engine<T>::rrqr_columns(std::vector<RrqrJob>& jobs, int rc_force) {
+  if (jobs.empty()) return;
   int kmax = 0, nmax = 0;
   for (auto& j : jobs) { kmax = std::max(kmax, j.k); nmax = std::max(nmax, j.N); }
   // rows per lane of the register form, one for the whole batch (one launch
@@ -1805,42 +1869,11 @@ void Engine<T>::rrqr_batch(std::vector<RrqrJob>& jobs, int rc_force) {
       if (best < 0 || cost < best) { best = cost; rc = r; }
     }
     if (qp3_reg_ && tol_ < 1.0) {
-      char key[96];
-      snprintf(key, sizeof key, "qp3r/%s/k%d/n%d/p%d", sizeof(T) == 8 ? "f64" : "f32", log2_bucket(kmax),
-               log2_bucket(nmax), log2_bucket((long)jobs.size()));
+      const std::string key = rrqr_key(jobs);
       Tuner& tu = global_tuner();
-      const int cached = tu.lookup(key);
-      if (cached > 0 && qp3r_cap(256, cached) > 0) {
-        rc = cached;
-      } else if (tu.tuning()) {
-        // time every form on copies of the batch's inputs (the RRQR works
-        // in place), keep the fastest
-        std::vector<std::pair<int, double>> ms;
-        double best_ms = -1;
-        for (int r : qp3r_rcs()) {
-          if (qp3r_cap(256, r) <= 0) continue;
-          std::vector<RrqrJob> trial;
-          std::vector<CopyDesc> cp;
-          for (auto& j : jobs) {
-            RrqrJob t{alloc_scr((size_t)std::max(j.N, 1) * j.k), j.k, j.N};
-            cp.push_back(CopyDesc{j.Ct, t.Ct, std::max(j.N, 1), std::max(j.N, 1), j.N, j.k, 0, 0});
-            trial.push_back(t);
-          }
-          const bool kp = kprof_;
-          kprof_ = false;
-          copy_blocks(cp);
-          sync();
-          const double t0 = wall();
-          trial_ = true;
-          rrqr_batch(trial, r);
-          trial_ = false;
-          const double t1 = 1e3 * (wall() - t0);
-          kprof_ = kp;
-          ms.push_back({r, t1});
-          if (best_ms < 0 || t1 < best_ms) { best_ms = t1; rc = r; }
-        }
-        tu.record(key, rc, ms);
-      }
+      if (tu.tuning() && tu.lookup(key) <= 0) rrqr_tune(jobs, key, false);
+      const int tuned = tu.lookup(key);
+      if (tuned > 0 && qp3r_cap(256, tuned) > 0) rc = tuned;
     }
   }
   const bool lds_ok = sizeof(T) * (size_t)std::max(kmax, 1) <= (size_t)48 * 1024;

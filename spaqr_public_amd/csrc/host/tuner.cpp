@@ -46,7 +46,7 @@ void Tuner::init(const std::string& arch) {
   ss << f.rdbuf();
   const std::string s = ss.str();
   // the file this class writes: one entry per line,
-  //   {"key": "<key>", "choice": <int>, "ms": {"<cand>": <ms>, ...}}
+  //   {"key": "<key>", "choice": <int>, "ms": {"<cand>": <ms>, ...}[, "blocked": <ms>]}
   size_t pos = 0;
   while ((pos = s.find("{\"key\": \"", pos)) != std::string::npos) {
     pos += 9;
@@ -71,6 +71,8 @@ void Tuner::init(const std::string& arch) {
         m = colon + 1;
       }
     }
+    const size_t next = s.find("{\"key\": \"", q), bl = s.find("\"blocked\": ", q);
+    if (bl < next) e.blocked = std::atof(s.c_str() + bl + 11);
     entries_[key] = e;
     pos = q;
   }
@@ -82,11 +84,21 @@ int Tuner::lookup(const std::string& key) {
   return it == entries_.end() ? -1 : it->second.choice;
 }
 
-void Tuner::record(const std::string& key, int choice, const std::vector<std::pair<int, double>>& ms) {
+int Tuner::prefers_register(const std::string& key) {
+  std::lock_guard<std::mutex> lk(mu_);
+  auto it = entries_.find(key);
+  if (it == entries_.end() || it->second.blocked < 0) return -1;
+  for (auto& m : it->second.ms)
+    if (m.first == it->second.choice) return m.second < it->second.blocked;
+  return -1;
+}
+
+void Tuner::record(const std::string& key, int choice, const std::vector<std::pair<int, double>>& ms, double blocked) {
   std::lock_guard<std::mutex> lk(mu_);
   Entry& e = entries_[key];
   e.choice = choice;
   e.ms = ms;
+  e.blocked = blocked;
   save();
 }
 
@@ -112,7 +124,13 @@ void Tuner::save() {
       snprintf(buf, sizeof buf, "%s\"%d\": %.4f", c ? ", " : "", kv.second.ms[c].first, kv.second.ms[c].second);
       f << buf;
     }
-    f << "}}" << (++i < entries_.size() ? "," : "") << "\n";
+    f << "}";
+    if (kv.second.blocked >= 0) {
+      char buf[64];
+      snprintf(buf, sizeof buf, ", \"blocked\": %.4f", kv.second.blocked);
+      f << buf;
+    }
+    f << "}" << (++i < entries_.size() ? "," : "") << "\n";
   }
   f << "]}\n";
 }

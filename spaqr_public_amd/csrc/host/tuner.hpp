@@ -8,7 +8,9 @@
 // the measured times of all candidates are kept in a JSON file, which later
 // runs read (SPAQR_TUNE_FILE, default tune/<gfx arch>.json beside the
 // library's package).  Keys missing from the file fall back to the engine's
-// closed-form rule.
+// closed-form rule.  For the RRQR the choice is among the register forms; where
+// the blocked form takes the batch too, its time is kept beside theirs and the
+// faster of the two runs (an entry without that time leaves the blocked form).
 #pragma once
 #include <map>
 #include <mutex>
@@ -24,14 +26,18 @@ class Tuner {
   bool tuning() const { return tuning_; }
   // Cached choice for key, or -1.
   int lookup(const std::string& key);
-  // Records a tuned choice with the candidates' measured times (ms) and
-  // rewrites the file.
-  void record(const std::string& key, int choice, const std::vector<std::pair<int, double>>& ms);
+  // 1 if the choice was measured to be faster than the blocked form, 0 if it
+  // was not, -1 if that was not measured.
+  int prefers_register(const std::string& key);
+  // Records a tuned choice with the candidates' measured times (ms; the blocked
+  // form's, or -1) and rewrites the file.
+  void record(const std::string& key, int choice, const std::vector<std::pair<int, double>>& ms, double blocked);
   const std::string& path() const { return path_; }
 
  private:
   struct Entry {
     int choice = -1;
+    double blocked = -1;
     std::vector<std::pair<int, double>> ms;
   };
   void save();

@@ -230,6 +230,23 @@ void stream() {
   Made t;
   CHECK(!fake::capturing.count(t.e.stream_));
 }
+
+// The tuner's file, written and read again.
+void tuner(const char* path) {
+  setenv("SPAQR_TUNE_FILE", path, 1);
+  {
+    Tuner t;
+    t.init("gfx950");
+    t.record("slower", 28, {{16, 3.5}, {28, 2.5}}, 1.5);
+    t.record("faster", 16, {{16, 0.5}, {28, 2.5}}, 1.5);
+    t.record("alone", 40, {{40, 2.0}}, -1);
+  }
+  Tuner t;
+  t.init("gfx950");
+  CHECK(t.lookup("slower") == 28 && t.lookup("faster") == 16 && t.lookup("alone") == 40 && t.lookup("none") == -1);
+  CHECK(t.prefers_register("slower") == 0 && t.prefers_register("faster") == 1);
+  CHECK(t.prefers_register("alone") == -1 && t.prefers_register("none") == -1);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -242,6 +259,7 @@ int main(int argc, char** argv) {
     else if (c == "timeout") timeout();
     else if (c == "trim") trim();
     else if (c == "stream") stream();
+    else if (c == "tuner" && argc > 2) tuner(argv[2]);
     else CHECK(!"a known case");
   } catch (const std::exception& e) {
     std::printf("exception: %s\n", e.what());

@@ -34,11 +34,11 @@ def engine_test(tmp_path_factory):
     return exe
 
 
-CASES = ["transposed", "segments", "no_memory", "rrqr_ring", "timeout", "trim", "stream"]
+CASES = ["transposed", "segments", "no_memory", "rrqr_ring", "timeout", "trim", "stream", "tuner"]
 
 
 @pytest.mark.parametrize("case", CASES)
-def test_host(engine_test, case):
+def test_host(engine_test, case, tmp_path):
     env = dict(os.environ, SPAQR_TUNE_FILE="/dev/null")
-    r = subprocess.run([engine_test, case], env=env, capture_output=True, text=True, timeout=120)
+    r = subprocess.run([engine_test, case, str(tmp_path / "tune.json")], env=env, capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
