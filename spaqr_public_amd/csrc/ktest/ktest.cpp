@@ -110,50 +110,53 @@ int ktest_smin(int k, const double* R, int ld, double* out) {
   return 0;
 }
 
+}  // extern "C"
+namespace {
 // Blocked Householder QR of one m x k panel (col-major, ld m): A <- V\R,
 // tau (min(m,k)), Tb (nb x roundup(k,nb)), and C (m x nc) <- Q^T C.
-int ktest_qr(int m, int k, double* A, double* tau, double* Tb, int nc, double* Cm) {
+template <typename X>
+int qr_one(int m, int k, X* A, X* tau, X* Tb, int nc, X* Cm) {
   const int nb = panel_nb(), kk = m < k ? m : k, nblk = (k + nb - 1) / nb;
-  double *dA = dup(A, (size_t)m * k), *dt = dup<double>(nullptr, k), *dT = dup<double>(nullptr, (size_t)nb * nb * nblk);
-  double* dC = dup(Cm, (size_t)m * (nc > 0 ? nc : 1), (size_t)m * nc);
+  X *dA = dup(A, (size_t)m * k), *dt = dup<X>(nullptr, k), *dT = dup<X>(nullptr, (size_t)nb * nb * nblk);
+  X* dC = dup(Cm, (size_t)m * (nc > 0 ? nc : 1), (size_t)m * nc);
   int zero = 0;
   int* ds = dup(&zero, 1);
   int* err = dup<int>(nullptr, 1);
   for (int jb = 0; jb < kk; jb += nb) {
-    const int nwg = panel_wgs<double>(m - jb);
-    if (nwg > panel_r_capacity<double>()) { g_err = "nwg exceeds resident capacity"; return -1; }
-    double* part = dup<double>(nullptr, panel_slots(nwg));
-    PanelDesc<double> pd{dA, dt, dT, m, m, k, nwg, part, err};
-    PanelDesc<double>* dpd = dup(&pd, 1);
-    const int rc = launch_panel_r<double>(0, dpd, ds, 1, nwg, jb, m - jb, nwg > 1 ? 1 : 0);
+    const int nwg = panel_wgs<X>(m - jb);
+    if (nwg > panel_r_capacity<X>()) { g_err = "nwg exceeds resident capacity"; return -1; }
+    X* part = dup<X>(nullptr, panel_slots(nwg));
+    PanelDesc<X> pd{dA, dt, dT, m, m, k, nwg, part, err};
+    PanelDesc<X>* dpd = dup(&pd, 1);
+    const int rc = launch_panel_r<X>(0, dpd, ds, 1, nwg, jb, m - jb, nwg > 1 ? 1 : 0);
     if (rc != 0) { g_err = hipGetErrorString((hipError_t)rc); return -1; }
     KT(hipDeviceSynchronize());
     for (void* q : {(void*)part, (void*)dpd}) (void)hipFree(q);
     const int w = (nb < kk - jb) ? nb : kk - jb, rows = m - jb;
-    const double* Vb = dA + jb + (size_t)jb * m;
-    const double* Tbb = dT + (size_t)jb * nb;
+    const X* Vb = dA + jb + (size_t)jb * m;
+    const X* Tbb = dT + (size_t)jb * nb;
     // the engine's descriptors for this step (W = V_b T_b^T, Y = V_b^T C,
     // C -= W Y), each list run as one batched launch as the engine does
-    std::vector<LarfbTarget<double>> tg;
+    std::vector<LarfbTarget<X>> tg;
     const int c0 = jb + ((nb < k - jb) ? nb : k - jb);
     if (k > c0) tg.push_back({dA + jb + (size_t)c0 * m, m, k - c0});
     if (nc > 0) tg.push_back({dC + jb, m, nc});
     std::vector<void*> scratch;
     auto alloc = [&](int64_t elems) {
-      double* p = dup<double>(nullptr, (size_t)(elems > 0 ? elems : 1));
+      X* p = dup<X>(nullptr, (size_t)(elems > 0 ? elems : 1));
       scratch.push_back(p);
       return p;
     };
-    std::vector<GemmDesc<double>> g1, g3;
-    larfb_step_descs<double>(Vb, m, Tbb, nb, rows, w, tg.data(), (int)tg.size(), alloc, g1, g3);
+    std::vector<GemmDesc<X>> g1, g3;
+    larfb_step_descs<X>(Vb, m, Tbb, nb, rows, w, tg.data(), (int)tg.size(), alloc, g1, g3);
     for (auto* gl : {&g1, &g3}) {
       if (gl->empty()) continue;
       std::vector<int> st(gl->size());
       int nt = 0;
       for (size_t i = 0; i < gl->size(); ++i) { st[i] = nt; nt += gemm_tiles((*gl)[i].m, (*gl)[i].n); }
-      GemmDesc<double>* dg = dup(gl->data(), gl->size());
+      GemmDesc<X>* dg = dup(gl->data(), gl->size());
       int* dst = dup(st.data(), st.size());
-      launch_gemm<double>(0, dg, dst, (int)gl->size(), nt);
+      launch_gemm<X>(0, dg, dst, (int)gl->size(), nt);
       KT(hipDeviceSynchronize());
       (void)hipFree(dg);
       (void)hipFree(dst);
@@ -173,18 +176,33 @@ int ktest_qr(int m, int k, double* A, double* tau, double* Tb, int nc, double* C
 }
 
 // Block T factors of V (m x r) and tau.
-int ktest_larft(int m, int r, const double* V, const double* tau, double* Tb) {
+template <typename X>
+int larft_one(int m, int r, const X* V, const X* tau, X* Tb) {
   const int nb = panel_nb(), nblk = (r + nb - 1) / nb;
-  double *dV = dup(V, (size_t)m * r), *dt = dup(tau, r), *dT = dup<double>(nullptr, (size_t)nb * nb * nblk);
-  LarftDesc<double> d{dV, dt, dT, m, m, r, 0};
-  LarftDesc<double>* dd = dup(&d, 1);
+  X *dV = dup(V, (size_t)m * r), *dt = dup(tau, r), *dT = dup<X>(nullptr, (size_t)nb * nb * nblk);
+  LarftDesc<X> d{dV, dt, dT, m, m, r, 0};
+  LarftDesc<X>* dd = dup(&d, 1);
   int zero = 0;
   int* ds = dup(&zero, 1);
-  launch_larft<double>(0, dd, ds, 1, nblk);
+  launch_larft<X>(0, dd, ds, 1, nblk);
   KT(hipDeviceSynchronize());
   back(Tb, dT, (size_t)nb * nb * nblk);
   for (void* p : {(void*)dV, (void*)dt, (void*)dT, (void*)dd, (void*)ds}) (void)hipFree(p);
   return 0;
+}
+}  // namespace
+extern "C" {
+int ktest_qr(int m, int k, double* A, double* tau, double* Tb, int nc, double* Cm) {
+  return qr_one<double>(m, k, A, tau, Tb, nc, Cm);
+}
+int ktest_qr_f32(int m, int k, float* A, float* tau, float* Tb, int nc, float* Cm) {
+  return qr_one<float>(m, k, A, tau, Tb, nc, Cm);
+}
+int ktest_larft(int m, int r, const double* V, const double* tau, double* Tb) {
+  return larft_one<double>(m, r, V, tau, Tb);
+}
+int ktest_larft_f32(int m, int r, const float* V, const float* tau, float* Tb) {
+  return larft_one<float>(m, r, V, tau, Tb);
 }
 
 // Truncated QP3 of C (k x N): Ct is N x k (ld N) in/out; V k x k, tau k.
@@ -302,19 +320,28 @@ int larfb_one(int form, int rows, int cols, int nt, int w, const T* V, int ldv, 
 namespace {
 // One dataflow op (kernels/flow.hip) on x (m values) and, for the triangular
 // and the pull form, xn (n values) with the block Bn: the inputs lie in two
-// segments in reverse order, the blocks' tiles start with a short one.
+// segments (or `pieces`) in reverse order, the blocks' tiles start with a short
+// one.
 //   WY: A, B m x k (lda, ldb), parts of rows_per rows; unit: A is V, B is W
 //   Back: R = A (k x k, m = k), Bn k x n (ldb), nwg parts; SolveT: R alone
 //   Pull: Bn = B n x m (ldb)
 template <typename T>
 int flow_one(int type, int m, int k, int par, int unit, const T* A, int lda, const T* B, int ldb, int n,
-             const double* x, const double* xn, double* out) {
-  const int h = m / 3, total = 2 * m + n + 7;
+             const double* x, const double* xn, double* out, int pieces = 0) {
+  const int total = 2 * m + n + 7;
+  std::vector<int> cut{0};
+  if (pieces)
+    for (int p = 1; p <= pieces; ++p) cut.push_back((int)((int64_t)m * p / pieces));
+  else
+    for (int e : {m - m / 3, m}) cut.push_back(e);
   std::vector<FlowSeg> segs;
-  if (m - h > 0) segs.push_back(FlowSeg{h, m - h});  // rows 0 .. m-h-1 of x lie after the others
-  if (h > 0) segs.push_back(FlowSeg{0, h});
   std::vector<double> xin(m + n);
-  for (int i = 0; i < m; ++i) xin[i < m - h ? h + i : i - (m - h)] = x[i];
+  for (size_t p = 0; p + 1 < cut.size(); ++p) {
+    const int len = cut[p + 1] - cut[p], off = m - cut[p + 1];  // the last rows lie first
+    if (len > 0) segs.push_back(FlowSeg{off, len});
+    for (int i = 0; i < len; ++i) xin[off + i] = x[cut[p] + i];
+  }
+  if ((int)segs.size() > kFlowMaxSegs) { g_err = "too many segments"; return -1; }
   for (int i = 0; i < n; ++i) xin[m + i] = xn[i];
   const bool tri = type == kFlowBack || type == kFlowSolveT, wy = type == kFlowWY;
   T* dA = A ? dup(A, (size_t)lda * k) : nullptr;
@@ -374,6 +401,10 @@ extern "C" {
 int ktest_flow(int type, int m, int k, int par, int unit, const double* A, int lda, const double* B, int ldb, int n,
                const double* x, const double* xn, double* out) {
   return flow_one<double>(type, m, k, par, unit, A, lda, B, ldb, n, x, xn, out);
+}
+int ktest_flow_pieces(int pieces, int type, int m, int k, int par, int unit, const double* A, int lda, const double* B,
+                      int ldb, int n, const double* x, const double* xn, double* out) {
+  return flow_one<double>(type, m, k, par, unit, A, lda, B, ldb, n, x, xn, out, pieces);
 }
 // One k_larfb step of `form` on nt targets of cols columns each (C: ldc x nt
 // cols, target t at its column t cols)
