@@ -2985,6 +2985,8 @@ bool Engine<T>::flow_fits() const {
     if (o.k > kFlowMaxK || o.kr > kFlowMaxK) return false;
     if (o.m > kFlowMaxParts * kFlowMaxK || too_long(std::max(o.ldv, o.m), o.k) || too_long(o.ldr, std::max(o.kr, o.k)))
       return false;
+    for (auto& q : o.r12)  // read whole by the transposed products
+      if (too_long(q.first.ld, q.second.second)) return false;
   }
   for (int c : bottoms_[0])
     if (square_ && cl_[c].rsize_org != cl_[c].csize_org) return false;

@@ -247,6 +247,42 @@ void tuner(const char* path) {
   CHECK(t.prefers_register("slower") == 0 && t.prefers_register("faster") == 1);
   CHECK(t.prefers_register("alone") == -1 && t.prefers_register("none") == -1);
 }
+
+// Blocks beyond the kernel's 32-bit byte offsets go to the staged apply: factors,
+// and the off-diagonal blocks that the transposed products read.
+void offsets() {
+  Made t;
+  CHECK(t.e.flow_fits());
+  auto& o = t.e.ops_.back();
+  Engine<double>::Block b{};
+  b.ld = 1 << 18;
+  o.r12.push_back({b, {o.c, 1 << 10}});
+  CHECK(t.e.flow_fits());
+  o.r12.back().second.second = 1 << 12;
+  CHECK(!t.e.flow_fits());
+  o.r12.clear();
+  o.ldr = 1 << 30;
+  CHECK(!t.e.flow_fits());
+}
+// What a caller sees when device memory ends: the arenas' code and that of the
+// Krylov work space.
+void codes() {
+  Made t;
+  t.build();
+  fake::dev_limit = 0;
+  auto code = [](auto&& f) {
+    try {
+      f();
+    } catch (const Error& e) {
+      return e.code;
+    }
+    return (int)kOk;
+  };
+  CHECK(code([&] { t.e.perm_.alloc(size_t(1) << 40); }) == kErrOom);
+  CHECK(code([&] { t.e.work_dev(0, size_t(1) << 37); }) == kErrHip);
+  fake::dev_limit = ~size_t(0);
+  CHECK(code([&] { t.e.work_dev(0, 1000); }) == kOk);  // and the slot is usable again
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -260,6 +296,8 @@ int main(int argc, char** argv) {
     else if (c == "trim") trim();
     else if (c == "stream") stream();
     else if (c == "tuner" && argc > 2) tuner(argv[2]);
+    else if (c == "offsets") offsets();
+    else if (c == "codes") codes();
     else CHECK(!"a known case");
   } catch (const std::exception& e) {
     std::printf("exception: %s\n", e.what());

@@ -34,7 +34,8 @@ def engine_test(tmp_path_factory):
     return exe
 
 
-CASES = ["transposed", "segments", "no_memory", "rrqr_ring", "timeout", "trim", "stream", "tuner"]
+CASES = ["transposed", "segments", "no_memory", "rrqr_ring", "timeout", "trim", "stream", "tuner", "offsets",
+         "codes"]
 
 
 @pytest.mark.parametrize("case", CASES)
