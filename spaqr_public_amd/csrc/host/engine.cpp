@@ -753,8 +753,9 @@ class Engine final : public EngineBase {
   }
 
   // tables of the larfb block steps, kept per host thread across block steps
-  // and trees: a level-0 step plans more than 100k descriptors, and fresh memory costs more host time (page faults) than
-  // filling it.  The memory is held until the thread ends.
+  // and trees: a level-0 step plans more than 100k descriptors, and fresh memory
+  // costs more host time (page faults) than filling it.  The memory is held until
+  // the thread ends.
   template <typename U>
   struct LarfbBufs {
     std::vector<LarfbDesc<U>> ds;
@@ -2743,6 +2744,7 @@ void Engine<T>::reassign_level(const std::vector<int>& cs) {
   // few rows, took 14 of the 16 ms of the first level of a 100^2 problem)
   std::vector<RowGatherDesc<T>> rg;
   std::vector<int> rgcnt, ridx;
+  std::vector<size_t> rgat;  // where a run's list begins
   for (auto& kv : grow) {
     Grow& g = kv.second;
     if (g.rows == g.base.rows && g.app.empty()) continue;
@@ -2751,8 +2753,8 @@ void Engine<T>::reassign_level(const std::vector<int>& cs) {
     if (g.base.rows > 0 && g.base.cols > 0)
       copies.push_back(CopyDesc{g.base.p, nb.p, g.base.ld, nb.ld, g.base.rows, g.base.cols, 0, 0});
     for (auto& a : g.app) {
-      rg.push_back(RowGatherDesc<T>{a.src, nb.p, (const int*)ridx.size(), a.lds, nb.ld, a.row0, (int)a.idx.size(),
-                                    nb.cols, 0});  // offset for now
+      rg.push_back(RowGatherDesc<T>{a.src, nb.p, nullptr, a.lds, nb.ld, a.row0, (int)a.idx.size(), nb.cols, 0});
+      rgat.push_back(ridx.size());
       ridx.insert(ridx.end(), a.idx.begin(), a.idx.end());
       rgcnt.push_back(rowgather_tiles((int)a.idx.size(), nb.cols));
     }
@@ -2762,7 +2764,7 @@ void Engine<T>::reassign_level(const std::vector<int>& cs) {
   copy_blocks(copies);
   if (!rg.empty()) {
     const int* didx = stager_.upload(perm_, ridx);
-    for (auto& d : rg) d.idx = didx + (size_t)d.idx;
+    for (size_t q = 0; q < rg.size(); ++q) rg[q].idx = didx + rgat[q];
     std::vector<int> st;
     const int nt = prefix_tiles(rgcnt, st);
     const RowGatherDesc<T>* dd = stager_.push(rg);

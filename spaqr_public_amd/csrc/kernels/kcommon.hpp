@@ -162,14 +162,6 @@ __device__ __forceinline__ void store_at(T* base, unsigned byte_off, T v) {
   *(gmut<T>)((__attribute__((address_space(1))) char*)to_global_mut(base) + byte_off) = v;
 }
 
-// a pointer every lane of the wave holds alike, as a scalar
-template <typename T>
-__device__ __forceinline__ const T* uniform_ptr(const T* p) {
-  const unsigned long long b = (unsigned long long)p;
-  const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32));
-  return (const T*)(((unsigned long long)hi << 32) | lo);
-}
 // Value of v in lane l (l uniform) for every lane of the wave.
 __device__ __forceinline__ double lane_bcast(double v, int l) {
   const unsigned long long b = __double_as_longlong(v);

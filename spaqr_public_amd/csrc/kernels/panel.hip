@@ -48,7 +48,9 @@ __device__ __forceinline__ void t_factor(const T (&Gs)[kNB][kNB], const T (&taus
 //   v_j^T A(:, c) = A(j, c) + scal * d_c
 // gives both the update of the later columns and the products with the
 // earlier reflectors for T.  Row j is final after step j in every column: it
-// is stored and its registers are zeroed, so no pass masks rows.
+// is stored and its registers are zeroed, so no pass masks rows.  (A column that is
+// not finite meets the earlier ones as x times zero, so that their V entries are
+// not kept; the block's T is not finite then, nor anything it is applied to.)
 // What bounds it: the latency of one step, and a launch has few panels (1-24
 // per elimination wave above level 2), so a panel stays in one workgroup as
 // long as its registers hold it (1280 rows in FP64).  One row per thread, 256
