@@ -99,6 +99,7 @@ class Arena {
   Arena& operator=(const Arena&) = delete;
   void* alloc(size_t bytes, size_t align = 256);
   void rewind();  // keep chunks, reset offsets
+  void set_chunk(size_t bytes) { chunk_ = bytes; }  // of the chunks taken from here on
   void release();  // chunks go back to the pool: the stream work on them is complete
   size_t used() const { return used_; }
   // chunk allocations of all arenas: count and host seconds (diagnostics)

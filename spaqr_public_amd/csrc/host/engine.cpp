@@ -857,7 +857,6 @@ class Engine final : public EngineBase {
     std::vector<FlowSeg> segs;
     std::vector<FlowBlk<U>> blks;
     std::vector<FlowDiag<U>> diags;
-    std::vector<int> diag_start{0};
     // by part: its exchange slots; where its diagonal blocks begin (-1: none)
     std::vector<size_t> slot_at;
     std::vector<int64_t> diag_at;
@@ -919,7 +918,9 @@ class Engine final : public EngineBase {
   template <typename U>
   void flow_plan(const std::vector<FlowStage>& stages, FlowRows& rows, int grid, FlowPlan<U>& plan) const;
   template <typename U>
-  void flow_place(FlowPlan<U>& plan, FlowProg<U>& prog);
+  void flow_space(const std::vector<std::pair<FlowPlan<U>*, FlowProg<U>*>>& progs);
+  template <typename U>
+  void flow_tables(const FlowPlan<U>& plan, FlowProg<U>& prog);
   std::vector<int> flow_places(const FlowRows& rows, const std::vector<int>& clusters) const;
   void run_flow(const double* b, double* x, bool transposed);
   // M^{-1} and M^{-T} (flow_mode_[0], [1]): one program, or around the FP64 top
@@ -3046,7 +3047,6 @@ void Engine<T>::flow_plan(const std::vector<FlowStage>& stages, FlowRows& R, int
   auto &segs = p.segs;
   auto &blks = p.blks;
   auto &diags = p.diags;
-  auto &diag_start = p.diag_start;
   constexpr bool top = sizeof(U) > sizeof(T);  // the FP64 factors of an FP32 tree's top
   std::vector<int>& wave = R.scratch;  // of a chain: waves so far on a cluster
   p.grid = cap;
@@ -3177,9 +3177,7 @@ void Engine<T>::flow_plan(const std::vector<FlowStage>& stages, FlowRows& R, int
       d.nblk = (int)blks.size() - d.blk0;
       if (it.type == kFlowBack) d.nwg = std::max(1, std::min({maxp, d.nblk, d.nblk * iceil(d.k, 64) / 8}));
       p.bytes += by + sizeof(U) * (0.5 * d.k * d.k + 2.0 * d.k);
-      const int nb = iceil(d.k, nb_);
       diags.push_back(FlowDiag<U>{d.A, nullptr, d.lda, d.k, it.type == kFlowSolveT, 0});
-      diag_start.push_back(diag_start.back() + nb);
       add_op(d, d.nwg, p.diag_elems);
       p.diag_elems += (int64_t)flow_diag_elems(d.k);
       set_rows(o.c, d.out, d.k);
@@ -3249,33 +3247,47 @@ void Engine<T>::flow_plan(const std::vector<FlowStage>& stages, FlowRows& R, int
   }
 }
 
-// The plan's tables and work space on the device.
+// The plans' work space on the device, and the diagonal blocks of their
+// triangular factors, in one launch for all.
 template <typename T>
 template <typename U>
-void Engine<T>::flow_place(FlowPlan<U>& p, FlowProg<U>& g) {
-  const size_t slot_words = p.slots * sizeof(U) / 4;
-  g.nzero = (int64_t)(slot_words + 64);
-  g.zero = (unsigned int*)flow_mem_.alloc(4 * (size_t)g.nzero);
-  U* const D = (U*)flow_mem_.alloc(sizeof(U) * (size_t)p.diag_elems);
-  for (size_t i = 0; i < p.parts.size(); ++i) {
-    if (p.parts[i].nwg > 1) p.parts[i].slots = (U*)g.zero + p.slot_at[i];
-    if (p.diag_at[i] >= 0) p.parts[i].B = D + p.diag_at[i];
+void Engine<T>::flow_space(const std::vector<std::pair<FlowPlan<U>*, FlowProg<U>*>>& progs) {
+  std::vector<FlowDiag<U>> diags;
+  std::vector<int> start{0};
+  for (auto& pg : progs) {
+    FlowPlan<U>& p = *pg.first;
+    FlowProg<U>& g = *pg.second;
+    const size_t slot_words = p.slots * sizeof(U) / 4;
+    g.nzero = (int64_t)(slot_words + 64);
+    g.zero = (unsigned int*)flow_mem_.alloc(4 * (size_t)g.nzero);
+    U* D = (U*)flow_mem_.alloc(sizeof(U) * (size_t)p.diag_elems);
+    for (size_t i = 0; i < p.parts.size(); ++i) {
+      if (p.parts[i].nwg > 1) p.parts[i].slots = (U*)g.zero + p.slot_at[i];
+      if (p.diag_at[i] >= 0) p.parts[i].B = D + p.diag_at[i];
+    }
+    for (auto& d : p.diags) {
+      d.D = D;
+      D += flow_diag_elems(d.k);
+      diags.push_back(d);
+      start.push_back(start.back() + iceil(d.k, nb_));
+    }
+    g.grid = p.grid;
+    g.args.nparts = (int)p.parts.size();
+    g.args.ctl = g.zero + slot_words;
+    g.args.err = solve_err_;
   }
-  int64_t at = 0;
-  for (auto& d : p.diags) {
-    d.D = D + at;
-    at += (int64_t)flow_diag_elems(d.k);
-  }
-  g.grid = p.grid;
-  g.args.nparts = (int)p.parts.size();
-  const FlowDiag<U>* dd = stager_.push(p.diags);
-  const int* ds = stager_.push(p.diag_start);
-  timed("wy", 0.0, 0.0, [&] { launch_flow_diag<U>(stream_, dd, ds, (int)p.diags.size(), p.diag_start.back()); });
+  const FlowDiag<U>* dd = stager_.push(diags);
+  const int* ds = stager_.push(start);
+  timed("wy", 0.0, 0.0, [&] { launch_flow_diag<U>(stream_, dd, ds, (int)diags.size(), start.back()); });
+}
+
+// A plan's tables (one after the other in the arena: they travel in one copy).
+template <typename T>
+template <typename U>
+void Engine<T>::flow_tables(const FlowPlan<U>& p, FlowProg<U>& g) {
   g.args.parts = stager_.upload(flow_mem_, p.parts);
   g.args.segs = stager_.upload(flow_mem_, p.segs);
   g.args.blks = stager_.upload(flow_mem_, p.blks);
-  g.args.ctl = g.zero + slot_words;
-  g.args.err = solve_err_;
 }
 
 // places of the clusters' rows, one after the other
@@ -3310,13 +3322,21 @@ bool Engine<T>::build_flow() {
 template <typename T>
 bool Engine<T>::make_flow() {
   scratch_.rewind();
-  // W of every op with reflectors
+  // W of every op with reflectors.  Large trees take the factors' chunk size: the
+  // pool frees its smallest buffers first when it is over its limit, and 64^3's 30
+  // chunks of 64 MB each were freed and allocated again by every tree (6 ms).
+  auto w_bytes = [&](const Op& o) -> size_t {
+    const bool has = o.kind == OpOrthoD || (square_ && (o.kind == OpQR || o.kind == OpScaleD));
+    return has && o.k > 0 ? (o.V64 ? sizeof(double) : sizeof(T)) * (size_t)o.m * o.k : 0;
+  };
+  size_t wbytes = 0;
+  for (auto& o : ops_) wbytes += w_bytes(o);
+  flow_mem_.set_chunk(wbytes > size_t(192) << 20 ? size_t(512) << 20 : size_t(64) << 20);
   std::vector<WyJob<T>> wj;
   std::vector<WyJob<double>> wj64;
   for (auto& o : ops_) {
-    if (o.kind != OpOrthoD && !(square_ && (o.kind == OpQR || o.kind == OpScaleD))) continue;
-    if (o.k <= 0) continue;
-    o.W = flow_mem_.alloc((o.V64 ? sizeof(double) : sizeof(T)) * (size_t)o.m * o.k);
+    if (!w_bytes(o)) continue;
+    o.W = flow_mem_.alloc(w_bytes(o));
     if (o.V64) wj64.push_back(WyJob<double>{o.V64, o.Tb64, (double*)o.W, o.ldv, o.m, o.k});
     else wj.push_back(WyJob<T>{o.V, o.Tb, (T*)o.W, o.ldv, o.m, o.k});
   }
@@ -3334,12 +3354,26 @@ bool Engine<T>::make_flow() {
   for (auto& P : plan)
     if (!P.fits()) return false;
   int nx = 0, nx64 = 0;
+  std::vector<std::pair<FlowPlan<T>*, FlowProg<T>*>> progs;
+  std::vector<std::pair<FlowPlan<double>*, FlowProg<double>*>> tops;
   for (int t = 0; t < nm; ++t) {
     FlowModePlan& P = plan[t];
     FlowMode& M = flow_mode_[t];
     M.run.resize(P.run.size());
-    for (size_t r = 0; r < P.run.size(); ++r) flow_place<T>(P.run[r], M.run[r]);
-    if (P.run.size() > 1) flow_place<double>(P.top, M.top);
+    for (size_t r = 0; r < P.run.size(); ++r) progs.push_back({&P.run[r], &M.run[r]});
+    if (P.run.size() > 1) tops.push_back({&P.top, &M.top});
+    nx = std::max(nx, P.xplaces);
+    nx64 = std::max(nx64, P.x64places);
+  }
+  flow_space<T>(progs);
+  if (!tops.empty()) flow_space<double>(tops);
+  flow_x_ = (T*)flow_mem_.alloc(sizeof(T) * (size_t)std::max(nx, 1));
+  if (nx64 > 0) flow_x64_ = (double*)flow_mem_.alloc(sizeof(double) * (size_t)nx64);
+  for (auto& pg : progs) flow_tables<T>(*pg.first, *pg.second);
+  for (auto& pg : tops) flow_tables<double>(*pg.first, *pg.second);
+  for (int t = 0; t < nm; ++t) {
+    FlowModePlan& P = plan[t];
+    FlowMode& M = flow_mode_[t];
     M.top_in = stager_.upload(flow_mem_, P.top_in);
     M.top_out = stager_.upload(flow_mem_, P.top_out);
     M.out = stager_.upload(flow_mem_, P.out);
@@ -3347,12 +3381,6 @@ bool Engine<T>::make_flow() {
     M.xplaces = P.xplaces;
     M.x64places = P.x64places;
     flow_top_n_ = P.top_n;
-    nx = std::max(nx, P.xplaces);
-    nx64 = std::max(nx64, P.x64places);
-  }
-  flow_x_ = (T*)flow_mem_.alloc(sizeof(T) * (size_t)std::max(nx, 1));
-  if (nx64 > 0) flow_x64_ = (double*)flow_mem_.alloc(sizeof(double) * (size_t)nx64);
-  for (auto& M : flow_mode_) {
     for (auto& r : M.run) r.args.x = flow_x_;
     M.top.args.x = flow_x64_;
   }
