@@ -865,6 +865,11 @@ class Engine final : public EngineBase {
     int grid = 0;
     double bytes = 0;  // the factors and vectors an apply streams
     bool fits = true;  // no op has more input segments than the kernel takes
+    // emptied, its memory kept
+    void clear() {
+      parts.clear(); segs.clear(); blks.clear(); diags.clear(); slot_at.clear(); diag_at.clear();
+      slots = 0; diag_elems = 0; grid = 0; bytes = 0; fits = true;
+    }
   };
   // places of x holding the rows of each cluster, as segments (least squares:
   // zeros, off -1, where nothing was written)
@@ -943,6 +948,13 @@ class Engine final : public EngineBase {
       bool f = top.fits;
       for (auto& r : run) f = f && r.fits;
       return f;
+    }
+    void clear(size_t runs) {
+      run.resize(runs);
+      for (auto& r : run) r.clear();
+      top.clear();
+      top_in.clear(); top_out.clear(); out.clear();
+      top_n = top_at = xplaces = x64places = 0;
     }
   };
   void plan_flow_mode(int t, int grid, int grid64, FlowModePlan& P) const;
@@ -3345,14 +3357,17 @@ bool Engine<T>::make_flow() {
   // the programs, planned side by side while W is formed
   const int nm = square_ ? 2 : 1;
   const int grid = std::min(flow_capacity<T>(), 2 * num_cus_), grid64 = std::min(flow_capacity<double>(), 2 * num_cus_);
-  std::vector<FlowModePlan> plan(nm);
+  // (kept per host thread, as the larfb tables are: two planners that fault fresh
+  // pages in at the same time take turns in the kernel)
+  static thread_local std::vector<FlowModePlan> kept(2);
+  std::vector<FlowModePlan>& plan = kept;
   parallel_for(nm, 1, [&](int, int b, int e) {
     for (int t = b; t < e; ++t)
       if (square_) plan_flow_mode(t, grid, grid64, plan[t]);
       else plan_flow_ls(grid, plan[t]);
   });
-  for (auto& P : plan)
-    if (!P.fits()) return false;
+  for (int t = 0; t < nm; ++t)
+    if (!plan[t].fits()) return false;
   int nx = 0, nx64 = 0;
   std::vector<std::pair<FlowPlan<T>*, FlowProg<T>*>> progs;
   std::vector<std::pair<FlowPlan<double>*, FlowProg<double>*>> tops;
@@ -3482,7 +3497,7 @@ void Engine<T>::plan_flow_mode(int t, int grid, int grid64, FlowModePlan& M) con
     R.next += cl_[c].rsize_org;
   }
   if (top) {
-    M.run.resize(2);
+    M.clear(2);
     flow_plan<T>(first, R, grid, M.run[0]);
     const int c = top->c;
     M.top_in = flow_places(R, {c});
@@ -3503,7 +3518,7 @@ void Engine<T>::plan_flow_mode(int t, int grid, int grid64, FlowModePlan& M) con
     R.next += top->m;
     flow_plan<T>(second, R, grid, M.run[1]);
   } else {
-    M.run.resize(1);
+    M.clear(1);
     flow_plan<T>(join(first, second), R, grid, M.run[0]);
   }
   M.xplaces = R.next;
@@ -3619,7 +3634,7 @@ void Engine<T>::plan_flow_ls(int grid, FlowModePlan& M) const {
     st.push_back(std::move(sc));
     st.push_back(std::move(qr));
   }
-  M.run.resize(1);
+  M.clear(1);
   flow_plan<T>(st, R, grid, M.run[0]);
   M.xplaces = R.next;
   for (int c : bottoms_[0])
